@@ -66,7 +66,9 @@ typedef enum { SHK_PREC_IDENTITY = 0, SHK_PREC_JACOBI = 1 } shk_precond;
  *             rows with sorted columns near the diagonal (banded, stencil
  *             and FEM matrices in natural order; RowSymSparse upper parts
  *             and their transposes are walked one after the other);
- *   AUTO   -- PANELS where it applies, else ROWS. */
+ *   AUTO   -- PANELS where it applies, else ROWS; for matrices whose rows
+ *             repeat a few column offsets (stencils, bands) the SpMV reads a
+ *             copy of the entries grouped by offset beside it. */
 /* Device layouts of a matrix: ROWS (row blocks, the caller's order), PANELS
  * (column-window chunks of 2048-row panels), SLICED (RowSparse only: the row
  * layout plus a copy of the entries in 8192-row panels whose lanes own rows,

@@ -132,6 +132,13 @@ struct shk_csr_s {
     unsigned short *sl_col = nullptr;  // [sl_ns] window-local columns
     void *sl_val = nullptr;            // [sl_ns] values
     int *sl_src = nullptr;             // [sl_ns] caller's entry index of each stream position
+    // Diagonal-slice copy of the entries (shk_dia.hpp), AUTO layouts of
+    // stencil and banded matrices: the SpMV reads it when it is there, every
+    // other use the layout above
+    int dia_steps = 0, dia_groups = 0;
+    void *dia_step = nullptr;          // [slices * dia_steps] DiaStep
+    void *dia_val = nullptr;           // [slices * dia_steps * 64] values
+    int *dia_src = nullptr;            // caller's entry index of each value slot (-1: none)
     // A^T for the transposed products (RowSparse, ArrayRowSparse), built on
     // first use as an ArrayRowSparse matrix whose rows list, for each column
     // c of A, the entries (i, c) in increasing i
@@ -283,6 +290,16 @@ int noalloc_scratch_init(int device);
 // free it
 int sliced_build(shk_csr A, const int *ptr, const int *ind, bool *applies);
 int sliced_set_values(shk_csr A);
+// diagonal-slice copy (shk_dia.hip): build it from device row arrays (mid,
+// src_of: RowSymSparse's expanded rows, else null; flags on ind are ignored);
+// *applies = false when the matrix is not regular enough.  Its values from
+// the caller's stored order; free it.
+int dia_build(shk_csr A, const int *ptr, const int *mid, const uint32_t *ind, const int64_t *src_of, bool *applies);
+int dia_set_values(shk_csr A, const void *dval);
+void dia_free(shk_csr A);
+// work-groups of its SpMV: at most kDiaWgPerCu per CU
+int dia_grid(shk_csr A);
+constexpr int kDiaWgPerCu = 8;
 // the matrix behind A's transposed products (built on first use)
 int transpose_of(shk_csr A, shk_csr *out);
 void sliced_free(shk_csr A);

@@ -719,11 +719,15 @@ __global__ __launch_bounds__(NT, MINW) void k_panel(SpmvArgs<T> a, const int4 *_
 
 }  // namespace shk
 
+#include "shk_dia.hpp"
 #include "shk_sliced.hpp"
 
 namespace shk {
 
 // ------------------------------------------------------------ launch ----
+// work-groups an SpMV of A may launch (partials per fused dot)
+inline int spmv_partials(shk_csr A) { return A->dia_val ? dia_grid(A) : A->nblk_launch; }
+
 template <typename T, typename Fin>
 inline int launch_spmv(shk_csr A, SpmvArgs<T> &a, Fin fin)
 {
@@ -743,11 +747,17 @@ inline int launch_spmv(shk_csr A, SpmvArgs<T> &a, Fin fin)
     a.slot_row = A->slot_row;
     const bool dots = a.dot0 != kDotNone || a.dot1 != kDotNone;
     if (dots && !a.partials) {
-        SHK_TRY(ensure_red(ctx, sizeof(T) * 2 * (size_t)A->nblk_launch));
+        SHK_TRY(ensure_red(ctx, sizeof(T) * 2 * (size_t)spmv_partials(A)));
         a.partials = (T *)ctx->red.partials;
     }
     constexpr bool defer = std::is_same<Fin, FinDefer>::value;
     if (A->m == 0) return SHK_OK;
+    if (A->dia_val) {
+        a.grid_used = launch_dia<T>(A, a);
+        if (dots && !defer) grid_finish<T>(ctx->stream, a.partials, a.grid_used, a.skip, fin);
+        SHK_HIP(hipGetLastError());
+        return SHK_OK;
+    }
     if (A->layout == SHK_LAYOUT_SLICED) {
         SHK_CHECK(A->sl_pchunk && A->sl_desc && A->sl_wstart && A->sl_bits && A->sl_rowmap && A->sl_col &&
                       A->sl_val,

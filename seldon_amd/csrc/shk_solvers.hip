@@ -2324,7 +2324,7 @@ struct Solve {
         size_t vb = (((size_t)n * sizeof(T) + 255) & ~(size_t)255);
         size_t hist_cap = it->hist && it->hist_cap > 0 ? (size_t)it->hist_cap : 0;
         size_t need = vec_count * vb + extra_bytes + 256 + hist_cap * (sizeof(double) + sizeof(int)) + 512;
-        const size_t maxb = (size_t)std::max(nb, a->nblk_launch);
+        const size_t maxb = (size_t)std::max(nb, spmv_partials(a));
         const size_t red = sizeof(T) * 10 * maxb;  // two buffers of [2][maxb], one of [6][maxb]
         if (ext) {
             need = (need + 255) & ~(size_t)255;
@@ -3596,7 +3596,7 @@ static int ir_impl(shk_ctx ctx, shk_csr A64, shk_csr A32, double *x, const doubl
     const int64_t n = A64->m;
     const size_t vb8 = ((size_t)n * 8 + 255) & ~(size_t)255, vb4 = ((size_t)n * 4 + 255) & ~(size_t)255;
     SHK_TRY(ensure_ws2(ctx, vb8 + 2 * vb4));
-    SHK_TRY(ensure_red(ctx, sizeof(double) * 2 * (size_t)std::max(red_blocks(n), A64->nblk_launch)));
+    SHK_TRY(ensure_red(ctx, sizeof(double) * 2 * (size_t)std::max(red_blocks(n), spmv_partials(A64))));
     char *w = (char *)ctx->ws2;
     double *r = (double *)w;
     float *r32 = (float *)(w + vb8), *d32 = (float *)(w + vb8 + vb4);

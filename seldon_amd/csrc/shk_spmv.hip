@@ -466,6 +466,60 @@ static int upload(shk_csr A, const HostPlan &P, const T *val_host)
     return SHK_OK;
 }
 
+// Whether a diagonal-slice copy is worth trying (dia_build decides): no row
+// longer than its step limit, and the middle slice's distinct offsets within
+// it and the fill bound.
+static bool dia_plausible(int m, const HostPlan &P)
+{
+    if (m == 0 || P.ind.empty() || P.max_row > 2 * kDiaMaxSteps) return false;
+    const int r0 = (m / 2) & ~(kWave - 1), r1 = std::min(m, r0 + kWave);
+    std::vector<int64_t> off;
+    for (int r = r0; r < r1; r++)
+        for (int j = P.ptr[r]; j < P.ptr[r + 1]; j++) {
+            const int64_t direct = !P.mid.empty() && j >= P.mid[r] ? (int64_t)1 << 40 : 0;
+            off.push_back((int64_t)(P.ind[j] & ~kLowerFlag) - r + direct);
+        }
+    const size_t entries = off.size();
+    std::sort(off.begin(), off.end());
+    const size_t steps = (size_t)(std::unique(off.begin(), off.end()) - off.begin());
+    return steps <= (size_t)kDiaMaxSteps &&
+           (double)(steps * kWave) <= 2 * kDiaFill * (double)entries + (double)kDiaSlack;
+}
+
+// The diagonal-slice copy of a matrix just uploaded, where it applies:
+// columns, expanded positions and the caller's values go up once more for
+// the build, what the layout above already holds is read in place.
+template <typename T>
+static int dia_upload(shk_csr A, const HostPlan &P, const T *val_host)
+{
+    hipStream_t s = A->ctx->stream;
+    const bool sym = !P.mid.empty(), own_ind = A->layout == SHK_LAYOUT_PANELS, own_val = own_ind || sym;
+    uint32_t *ind = nullptr;
+    int64_t *src_of = nullptr;
+    T *val = nullptr;
+    hipError_t e = hipSuccess;
+    auto put = [&](auto **dst, const auto *src, size_t n) {
+        if (e == hipSuccess) e = hipMalloc((void **)dst, sizeof(*src) * std::max<size_t>(n, 1));
+        if (e == hipSuccess) e = hipMemcpyAsync(*dst, src, sizeof(*src) * n, hipMemcpyHostToDevice, s);
+    };
+    if (own_ind) put(&ind, P.ind.data(), P.ind.size());
+    if (sym) put(&src_of, P.src_of.data(), P.src_of.size());
+    bool applies = false;
+    int st = SHK_OK;
+    if (e == hipSuccess)
+        st = dia_build(A, A->ptr, sym ? (const int *)A->mid : nullptr, own_ind ? ind : A->ind, src_of, &applies);
+    if (st == SHK_OK && applies) {
+        if (own_val) put(&val, val_host, (size_t)A->nnz_stored);
+        if (e == hipSuccess) st = dia_set_values(A, own_val ? (const void *)val : A->val);
+    }
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    hipFree(ind);
+    hipFree(src_of);
+    hipFree(val);
+    if (st == SHK_OK) SHK_HIP(e);
+    return st;
+}
+
 template <typename T>
 static int set_values_dev(shk_csr A, const T *dval)
 {
@@ -488,7 +542,7 @@ static int set_values_dev(shk_csr A, const T *dval)
                            (const int64_t *)A->map_diag, (const T *)A->val, (T *)A->diag);
     SHK_HIP(hipGetLastError());
     if (A->layout == SHK_LAYOUT_SLICED) SHK_TRY(sliced_set_values(A));
-    return SHK_OK;
+    return dia_set_values(A, dval);
 }
 
 template <typename T>
@@ -918,6 +972,14 @@ int shk_csr_create_layout(shk_ctx ctx, shk_storage storage, shk_dtype dtype, int
         st = dtype == SHK_F64 ? upload<double>(A, P, (const double *)hval.data())
                               : upload<float>(A, P, (const float *)hval.data());
     }
+    if (st == SHK_OK && want == SHK_LAYOUT_AUTO && dia_plausible(m, P)) {
+        if (layout == SHK_LAYOUT_SLICED) A->layout = SHK_LAYOUT_ROWS;  // what is uploaded so far
+        st = dtype == SHK_F64 ? dia_upload<double>(A, P, (const double *)hval.data())
+                              : dia_upload<float>(A, P, (const float *)hval.data());
+        // with it no second copy is planned: the row layout serves the rest
+        if (A->dia_val) layout = A->layout;
+        else A->layout = layout;
+    }
     if (st == SHK_OK && layout == SHK_LAYOUT_SLICED) {
         bool applies = false;
         st = sliced_build(A, hptr.data(), hind.data(), &applies);
@@ -961,6 +1023,7 @@ int shk_csr_destroy(shk_csr A)
     hipFree(A->chunk);
     hipFree(A->slot_row);
     sliced_free(A);
+    dia_free(A);
     delete A;
     return SHK_OK;
 }

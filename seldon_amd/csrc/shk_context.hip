@@ -57,6 +57,14 @@ int ensure_ws2(shk_ctx ctx, size_t bytes)
     return SHK_OK;
 }
 
+int wall_clock_ticks(shk_ctx ctx, long long seconds, long long *ticks)
+{
+    int khz = 0;
+    SHK_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ctx->device));
+    *ticks = (long long)(khz > 0 ? khz : 100000) * 1000LL * seconds;  // 100 MHz where none is reported
+    return SHK_OK;
+}
+
 int check_device_ptr(const void *p, const char *what)
 {
     if (!p) return fail(SHK_ERR_ARG, std::string("null device pointer: ") + what);

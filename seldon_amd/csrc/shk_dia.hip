@@ -12,13 +12,12 @@ namespace {
 // The steps of one slice, by one wavefront: each lane walks its row's entries
 // and every step takes the smallest offset any lane is at.  The stored part
 // [ptr, mid) comes first, then the transposed part [mid, ptr end) (mid null:
-// one part).  fill = false counts the steps into *most (a row whose columns
-// do not increase, or more than kDiaMaxSteps, sets *bad); fill = true writes
-// the steps and, per slot, the entry's position (src; -1 where the row has
+// one part).  fill = false fills flag[] = {most steps of a slice; a row's
+// columns do not increase or there are more than kDiaMaxSteps; largest row -
+// col; largest col - row}; fill = true writes the steps and, per slot, the entry's position (src; -1 where the row has
 // none).
 __global__ __launch_bounds__(kBlock) void k_dia_build(int m, const int *ptr, const int *mid, const uint32_t *ind,
-                                                      int steps, DiaStep *step, int *src, int *most, int *bad,
-                                                      bool fill)
+                                                      int steps, DiaStep *step, int *src, int *flag, bool fill)
 {
     const int slice = blockIdx.x * kDiaWaves + (int)(threadIdx.x >> 6);
     const int lane = threadIdx.x & (kWave - 1);
@@ -29,7 +28,7 @@ __global__ __launch_bounds__(kBlock) void k_dia_build(int m, const int *ptr, con
     const int end = in ? ptr[row + 1] : 0;
     const int split = in && mid ? mid[row] : end;
     const size_t s0 = (size_t)slice * steps;
-    int k = 0;
+    int k = 0, left = 0, right = 0;
     bool ok = true;
     for (int part = 0; part < (mid ? 2 : 1); part++) {
         const int e = part == 0 ? split : end;
@@ -44,6 +43,8 @@ __global__ __launch_bounds__(kBlock) void k_dia_build(int m, const int *ptr, con
                 if (lo != INT32_MAX) ok = false;
                 break;
             }
+            left = max(left, -lo);
+            right = max(right, lo);
             const bool act = j < e && off == lo;
             const uint64_t mask = __builtin_amdgcn_ballot_w64(act);
             if (fill) {
@@ -58,8 +59,12 @@ __global__ __launch_bounds__(kBlock) void k_dia_build(int m, const int *ptr, con
         }
     }
     if (!fill) {
-        if (!ok) atomicOr(bad, 1);
-        if (lane == 0) atomicMax(most, k);
+        if (!ok) atomicOr(flag + 1, 1);
+        if (lane == 0) {
+            atomicMax(flag, k);
+            atomicMax(flag + 2, left);
+            atomicMax(flag + 3, right);
+        }
     } else {
         for (; k < steps; k++) {
             if (lane == 0) step[s0 + k] = DiaStep{0ull, 0, mid ? 1 : 0};
@@ -97,12 +102,12 @@ int dia_build(shk_csr A, const int *ptr, const int *mid, const uint32_t *ind, co
     hipStream_t s = A->ctx->stream;
     const int slices = (A->m + kWave - 1) / kWave;
     const dim3 grid((slices + kDiaWaves - 1) / kDiaWaves), blk(kBlock);
-    int *flag = nullptr, h[2] = {0, 0};
+    int *flag = nullptr, h[4] = {0, 0, 0, 0};
     SHK_HIP(hipMalloc(&flag, sizeof(h)));
     hipError_t e = hipMemcpyAsync(flag, h, sizeof(h), hipMemcpyHostToDevice, s);
     if (e == hipSuccess) {
         hipLaunchKernelGGL(k_dia_build, grid, blk, 0, s, A->m, ptr, mid, ind, 0, (DiaStep *)nullptr, (int *)nullptr,
-                           flag, flag + 1, false);
+                           flag, false);
         e = hipMemcpyAsync(h, flag, sizeof(h), hipMemcpyDeviceToHost, s);
     }
     if (e == hipSuccess) e = hipStreamSynchronize(s);
@@ -111,12 +116,14 @@ int dia_build(shk_csr A, const int *ptr, const int *mid, const uint32_t *ind, co
     const int64_t slots = (int64_t)slices * h[0] * kWave;
     if (h[1] || h[0] == 0 || slots > (int64_t)(kDiaFill * (double)A->nnz_dev) + kDiaSlack) return SHK_OK;
     A->dia_steps = h[0];
+    A->dia_left = h[2];
+    A->dia_right = h[3];
     A->dia_groups = (slices + kDiaWaves - 1) / kDiaWaves;
     SHK_HIP(hipMalloc(&A->dia_step, sizeof(DiaStep) * (size_t)slices * h[0]));
     SHK_HIP(hipMalloc((void **)&A->dia_src, sizeof(int) * (size_t)slots));
     SHK_HIP(hipMalloc(&A->dia_val, dsize(A->dtype) * (size_t)slots));
     hipLaunchKernelGGL(k_dia_build, grid, blk, 0, s, A->m, ptr, mid, ind, h[0], (DiaStep *)A->dia_step, A->dia_src,
-                       (int *)nullptr, (int *)nullptr, true);
+                       (int *)nullptr, true);
     if (src_of)
         hipLaunchKernelGGL(k_dia_map, dim3(red_blocks(slots)), blk, 0, s, slots, src_of, A->dia_src);
     SHK_HIP(hipGetLastError());

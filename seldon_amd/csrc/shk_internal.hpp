@@ -9,6 +9,7 @@
 
 #include <cstdint>
 #include <cstdio>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -136,6 +137,7 @@ struct shk_csr_s {
     // stencil and banded matrices: the SpMV reads it when it is there, every
     // other use the layout above
     int dia_steps = 0, dia_groups = 0;
+    int dia_left = 0, dia_right = 0;   // largest row - col and col - row
     void *dia_step = nullptr;          // [slices * dia_steps] DiaStep
     void *dia_val = nullptr;           // [slices * dia_steps * 64] values
     int *dia_src = nullptr;            // caller's entry index of each value slot (-1: none)
@@ -307,5 +309,12 @@ void sliced_free(shk_csr A);
 // many rows (256 panels of 8192 rows)
 constexpr int kSlAutoMinRows = 1 << 21;
 int check_device_ptr(const void *p, const char *what);
+// wall_clock64 ticks of the given seconds
+int wall_clock_ticks(shk_ctx ctx, long long seconds, long long *ticks);
+// Kernels whose work-groups wait for each other need all of them on the GPU
+// at once: two such launches from two threads could each hold half of it.
+// Whoever launches one holds the device's mutex until it has ended.
+std::mutex &resident_mutex(int device);
+constexpr size_t kResLds = 158 * 1024;  // LDS of a resident work-group's window
 
 }  // namespace shk

@@ -20,6 +20,8 @@ struct KState {
     int done, init_failed, hist_len, hist_cap;
     int skip;          // done, or (GMRES) the current cycle is over
     int stop_slot;     // BiCgStab / TfQmr: loop slot (TfQmr: half step) that ended the solve
+    // resident Cg: a member's wait ran out / the solve ran to its end
+    unsigned res_stall, res_ran;
     double *hist;
     int *hist_it;
     // Cg / BiCgStab scalars, typed like Seldon's `Complexe` (= value type)

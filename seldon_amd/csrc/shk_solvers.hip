@@ -2435,9 +2435,15 @@ struct Solve {
 
 constexpr int kChunk = 16;
 
+// one solve on chip (shk_resident.hip): whether the matrix fits, and the
+// launches after the first Finished(r); zw holds 2 n values, slot the partials
+bool cg_resident_fits(shk_csr A);
+template <typename T>
+int cg_resident(shk_ctx ctx, shk_csr A, const T *diag, T *x, T *r, void *zw, void *slot, KState<T> *st);
+
 template <typename T>
 int cg_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration *it, int *code,
-            char *ext = nullptr, size_t ext_cap = 0)
+            char *ext = nullptr, size_t ext_cap = 0, bool resident = true)
 {
     Solve<T> S;
     S.ext = ext;
@@ -2466,6 +2472,14 @@ int cg_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration *i
     }
     SHK_HIP(hipGetLastError());
     const T *dg = (const T *)A->diag;
+    if (resident && cg_resident_fits(A)) {
+        std::lock_guard<std::mutex> lk(resident_mutex(ctx->device));
+        SHK_TRY(cg_resident<T>(ctx, A, jac ? dg : nullptr, x, r, p, S.partials, S.dst));
+        SHK_TRY(S.read_state());
+        if (!S.hst->res_stall) return S.finish(it, code);
+    }
+    if (S.hst->res_stall)  // a member waited too long for the others (a shared GPU): x is as it was, start over
+        return cg_impl<T>(ctx, A, x, b, prec, it, code, ext, ext_cap, false);
     const int64_t limit = (int64_t)std::max(it->max_iter, 0) + 2;
     // the loop head of iterations 1 .. kChunk - 1 of a chunk is folded into
     // the next kernel (identity: k_cg_p_top; Jacobi: k_cg_z_top, and rho =

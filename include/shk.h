@@ -408,9 +408,10 @@ int shk_sddmm(shk_ctx ctx, shk_csr A, const void *dlam, const void *dx, void *dg
  * [row_off[s], row_off[s+1]).  One persistent kernel runs every CG (identity
  * preconditioner, Seldon's Cg recurrences per system) to tol relative to
  * ||b_s||; per-system iterations and codes come back in its[], codes[].
- * group = threads per system work-group (64..1024, power of two; 0 = 512);
- * rows_per_pass = rows a thread keeps in flight per pass (1, 2, 4 or 8;
- * 0 = 4). */
+ * Systems whose rows repeat a few column offsets (stencils) are held on chip
+ * while they are solved; for the others, group = threads per system work-group
+ * (64..1024, power of two; 0 = 512) and rows_per_pass = rows a thread keeps in
+ * flight per pass (1, 2, 4 or 8; 0 = 4). */
 int shk_cg_batched(shk_ctx ctx, shk_csr A, int count, const int *row_off_host,
                    void *dx, const void *db, double tol, int max_iter, int group,
                    int rows_per_pass, int use_graph, int *its, int *codes);

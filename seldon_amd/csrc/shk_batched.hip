@@ -24,6 +24,13 @@
 // breakdown codes 1 and 2, ErrorCode -2 at max_iter.  Row sums of the SpMV are
 // sequential in stored order, as in Functions_MatVect.cxx:424-430.
 //
+// Stencil systems (up to seven column offsets per 64-row slice) are held on
+// chip while they are solved (shk_resident.hpp); the streaming kernel here
+// serves the others and the mixed variant.  Bounded by the latency of an
+// iteration's two sums (3 to 5 us at up to 4096 rows per member) where the
+// streaming kernel was bounded by memory: 512 anisotropic Laplacians of 1K to
+// 65K rows (12.8M in all) to 1e-8, 411 -> 36.4 ms.
+//
 // The mixed variant runs, per system, FP32 Cg inner solves on the scaled
 // correction equation A d = r / |r| and FP64 refinement x += |r| d with the
 // true residual r = b - A x in FP64.
@@ -32,6 +39,7 @@
 #include <numeric>
 
 #include "shk_kernels.hpp"
+#include "shk_resident.hpp"
 
 namespace shk {
 
@@ -506,6 +514,355 @@ __global__ __launch_bounds__(kMaxGroup, kBatchWaves<U>) void k_cg_batched_ir(Bat
     }
 }
 
+// ------------------------------------------- systems held on chip ----
+constexpr int kBrThreads = 512;
+// rows per thread, at most: what fits 256 VGPRs (seven steps spill at eight)
+constexpr int br_rows(int steps) { return steps <= 5 ? 8 : 4; }
+constexpr int kBrMinRows = 2;                         // rows per thread a plan goes down to
+constexpr int kBrSteps = 7;                           // steps stored per slice
+
+// The diagonal slices of every system (64 rows from the system's first row
+// on), values in place; flag[] = {most steps; a column outside its system;
+// columns that do not increase or too many steps}, band[s] = {largest row -
+// col, largest col - row} of system s.
+__global__ __launch_bounds__(kBlock) void k_batch_dia(int count, const int *row_off, const int *slice_off, int nslice,
+                                                      const int *ptr, const uint32_t *ind, const double *val,
+                                                      DiaStep *step, double *sval, int *flag, int2 *band)
+{
+    const int slice = blockIdx.x * kDiaWaves + (int)(threadIdx.x >> 6);
+    const int lane = threadIdx.x & (kWave - 1);
+    if (slice >= nslice) return;
+    int lo = 0, hi = count - 1;  // the system: the last s with slice_off[s] <= slice
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (slice_off[mid] <= slice) lo = mid;
+        else hi = mid - 1;
+    }
+    const int s = lo, c0 = row_off[s], c1 = row_off[s + 1];
+    const int row = c0 + (slice - slice_off[s]) * kWave + lane;
+    const bool in = row < c1;
+    int j = in ? ptr[row] : 0;
+    const int end = in ? ptr[row + 1] : 0;
+    const size_t s0 = (size_t)slice * kBrSteps;
+    int k = 0, left = 0, right = 0, last = -1;
+    bool outside = false, irregular = false;
+    for (;; k++) {
+        const bool have = j < end;
+        const int col = have ? (int)(ind[j] & ~kLowerFlag) : 0;
+        if (have) {
+            irregular |= col <= last;
+            outside |= col < c0 || col >= c1;
+        }
+        const int off = have ? col - row : INT32_MAX;
+        int least = off;
+        for (int o = 32; o > 0; o >>= 1) least = min(least, __shfl_xor(least, o, kWave));
+        if (least == INT32_MAX) break;
+        if (k == kBrSteps) {
+            irregular = true;
+            break;
+        }
+        const bool act = have && off == least;
+        const uint64_t mask = __builtin_amdgcn_ballot_w64(act);
+        if (lane == 0) step[s0 + k] = DiaStep{mask, least, 0};
+        sval[(s0 + k) * kWave + lane] = act ? val[j] : 0.0;
+        left = max(left, -least);
+        right = max(right, least);
+        if (act) {
+            last = col;
+            j++;
+        }
+    }
+    if (outside) atomicOr(flag + 1, 1);
+    if (irregular) atomicOr(flag + 2, 1);
+    if (lane == 0) {
+        atomicMax(flag, k);
+        atomicMax(&band[s].x, left);
+        atomicMax(&band[s].y, right);
+        for (; k < kBrSteps; k++) step[s0 + k] = DiaStep{0ull, 0, 0};
+    }
+}
+
+struct ResBatch {
+    int nslot;
+    const int2 *slots;     // queue position -> {system, member}
+    const int *row_off, *slice_off, *team, *share, *slot_off;
+    const int2 *band;
+    const DiaStep *step;
+    const double *val;
+    const double *b;
+    double *x;
+    ll_word *zw, *words;   // z of every row; sum words, system s from slot_off[s] on
+    int n, nwords, steps;
+    unsigned *queue, *stall;
+    long long limit;
+    double tol;
+    int max_iter;
+    int *its, *codes;
+};
+
+// A persistent grid draws (system, member) slots; res_cg solves.
+template <int KS>
+__global__ __launch_bounds__(kBrThreads, 2) void k_cg_batched_res(ResBatch a)
+{
+    constexpr int RPT = br_rows(KS);
+    extern __shared__ char res_lds[];
+    __shared__ ResShared<double> sh;
+    __shared__ int s_q;
+    const int tid = threadIdx.x;
+    if (tid == 0) sh.bad = 0;
+    const LlBuf zw(a.zw, (int64_t)a.n * ll_words<double>());
+    for (;;) {
+        __syncthreads();  // the last system's scratch is free
+        if (tid == 0) s_q = (int)atomicAdd(a.queue, 1u);
+        __syncthreads();
+        const int qi = s_q;
+        if (qi >= a.nslot) return;
+        const int2 sl = a.slots[qi];
+        const int s = sl.x;
+        ResRows R;
+        R.r0 = a.row_off[s];
+        R.r1 = a.row_off[s + 1];
+        R.m0 = min(R.r1, R.r0 + sl.y * a.share[s]);
+        R.m1 = min(R.r1, R.m0 + a.share[s]);
+        R.left = a.band[s].x;
+        R.right = a.band[s].y;
+        R.slice0 = a.slice_off[s] + (R.m0 - R.r0) / kWave;
+        R.steps = a.steps;
+        R.stride = kBrSteps;
+        R.step = a.step;
+        res_window(R);
+        const int k = a.team[s];
+        ResTeam t{k, sl.y, LlBuf(a.words + a.slot_off[s], 2 * k * res_slot_words<double>()), 0u, a.stall, a.limit};
+        // Init(b); x = 0, r = b (Cg.cxx:58-67)
+        double x[RPT], r[RPT], c[1] = {0.0};
+#pragma unroll
+        for (int u = 0; u < RPT; u++) {
+            const int row = R.m0 + u * kBrThreads + tid;
+            x[u] = 0.0;
+            r[u] = row < R.m1 ? a.b[row] : 0.0;
+            c[0] += r[u] * r[u];
+        }
+        res_post<double, 1, kBrThreads>(c, t, sh);
+        if (!res_wait<double, 1, kBrThreads>(c, t, sh)) return;
+        const double bn = sqrt(c[0]);
+        ResIter<double> it{0.0, a.tol, a.max_iter, 0, 0, c[0]};
+        if (bn != 0.0) {
+            it.facteur = 1.0 / bn;
+            auto head = [&](int nb, double rr) { return it.facteur * sqrt(rr) < it.tol || nb >= it.max_iter; };
+            unsigned zepoch = 0u;
+            if (!head(0, c[0]) &&
+                !res_cg<double, kBrThreads, RPT, KS, false>(R, a.val, nullptr, x, r, zw, (double *)res_lds, it, t,
+                                                                sh, zepoch, head))
+                return;
+#pragma unroll
+            for (int u = 0; u < RPT; u++) {
+                const int row = R.m0 + u * kBrThreads + tid;
+                if (row < R.m1) a.x[row] = x[u];
+            }
+        }
+        if (tid == 0 && sl.y == 0) {
+            a.its[s] = it.nb;
+            a.codes[s] = bn != 0.0 && it.nb >= it.max_iter ? -2 : it.code;
+        }
+    }
+}
+
+// queue head, stall flag and the exchanged words to their start
+__global__ __launch_bounds__(kBlock) void k_batch_res_reset(unsigned *queue, unsigned *stall, int64_t n, ll_word *words)
+{
+    const int64_t i0 = blockIdx.x * (int64_t)kBlock + threadIdx.x;
+    if (i0 == 0) {
+        *queue = 0u;
+        *stall = 0u;
+    }
+    for (int64_t i = i0; i < n; i += (int64_t)gridDim.x * kBlock) words[i] = 0;
+}
+
+// Members of each system and the queue.  A system gets the members its rows
+// need at `most_rows` rows per thread; while all of a batch fits the GPU at
+// once, shares are cut smaller (more CUs per system, down to kBrMinRows).
+// Systems are queued by size, the longest solve first.
+static bool plan_resident(const std::vector<int> &sizes, int most_rows, int cus, std::vector<int> &team,
+                          std::vector<int> &share, std::vector<int2> &slots)
+{
+    const int count = (int)sizes.size(), most = std::min(cus, kResMaxTeam);
+    int rows = most_rows * kBrThreads;
+    for (int r = kBrMinRows * kBrThreads; r < rows; r *= 2) {
+        int64_t members = 0;
+        for (int n : sizes) members += (n + r - 1) / r;
+        if (members <= cus) {
+            rows = r;
+            break;
+        }
+    }
+    team.assign(count, 1);
+    share.assign(count, kWave);
+    for (int s = 0; s < count; s++) {
+        team[s] = std::max(1, (sizes[s] + rows - 1) / rows);
+        if (team[s] > most) return false;
+        const int per = (sizes[s] + team[s] - 1) / team[s];
+        share[s] = std::max(kWave, (per + kWave - 1) / kWave * kWave);
+    }
+    std::vector<int> order(count);
+    std::iota(order.begin(), order.end(), 0);
+    std::stable_sort(order.begin(), order.end(), [&](int i, int j) { return sizes[i] > sizes[j]; });
+    slots.clear();
+    for (int s : order)
+        for (int j = 0; j < team[s]; j++) slots.push_back(make_int2(s, j));
+    return true;
+}
+
+// Record `enqueue(stream)` once on the context's own non-blocking stream (the
+// legacy default stream cannot be captured) and launch it on `st`, so it
+// stays ordered after the copies there; or enqueue it directly.
+template <class Enqueue>
+static int launch_batch(shk_ctx ctx, hipStream_t st, int use_graph, Enqueue enqueue)
+{
+    if (!use_graph) return enqueue(st);
+    hipGraph_t graph;
+    hipGraphExec_t exec;
+    SHK_HIP(hipStreamBeginCapture(ctx->own, hipStreamCaptureModeThreadLocal));
+    const int e = enqueue(ctx->own);
+    const hipError_t ce = hipStreamEndCapture(ctx->own, &graph);
+    SHK_TRY(e);
+    SHK_HIP(ce);
+    SHK_HIP(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
+    SHK_HIP(hipGraphLaunch(exec, st));
+    SHK_HIP(hipStreamSynchronize(st));
+    SHK_HIP(hipGraphExecDestroy(exec));
+    SHK_HIP(hipGraphDestroy(graph));
+    return SHK_OK;
+}
+
+// The batch on chip; *solved = false when a system does not fit (irregular,
+// too wide a band, too many rows): nothing has been written then.
+static int batched_resident(shk_ctx ctx, shk_csr A, int count, const int *row_off_host, const std::vector<int> &sizes,
+                            double *x, const double *b, double tol, int max_iter, int use_graph, int *its, int *codes,
+                            bool *solved)
+{
+    *solved = false;
+    const int n = A->m;
+    if (n == 0 || A->max_row > kBrSteps || (int64_t)n * 16 >= INT32_MAX) return SHK_OK;
+    std::vector<int> slice_off(count + 1, 0);
+    int most_slots = 0;  // of the finest plan
+    for (int s = 0; s < count; s++) {
+        slice_off[s + 1] = slice_off[s] + (sizes[s] + kWave - 1) / kWave;
+        most_slots += std::max(1, (sizes[s] + kBrMinRows * kBrThreads - 1) / (kBrMinRows * kBrThreads));
+    }
+    const int nslice = slice_off[count];
+    const int64_t zwords = (int64_t)n * ll_words<double>();
+    hipStream_t st = ctx->stream;
+    char *base = nullptr;
+    size_t used = 0;
+    auto take = [&](size_t bytes) {
+        char *p = base + used;
+        used += (bytes + 255) & ~(size_t)255;
+        return p;
+    };
+    int *d_off, *d_slice, *d_team, *d_share, *d_slot, *d_its, *d_codes;
+    int2 *d_slots, *d_band;
+    DiaStep *d_step;
+    double *d_val;
+    ll_word *d_words;
+    unsigned *d_flag;  // {most steps, outside, irregular, stall}
+    auto lay = [&]() {
+        used = 0;
+        d_flag = (unsigned *)take(4 * sizeof(unsigned));
+        d_band = (int2 *)take(sizeof(int2) * (size_t)count);  // with d_flag: read back together
+        d_off = (int *)take(sizeof(int) * (size_t)(count + 1));
+        d_slice = (int *)take(sizeof(int) * (size_t)(count + 1));
+        d_slot = (int *)take(sizeof(int) * (size_t)(count + 1));
+        d_team = (int *)take(sizeof(int) * (size_t)count);
+        d_share = (int *)take(sizeof(int) * (size_t)count);
+        d_slots = (int2 *)take(sizeof(int2) * (size_t)most_slots);
+        d_its = (int *)take(sizeof(int) * (size_t)count);
+        d_codes = (int *)take(sizeof(int) * (size_t)count);
+        d_words = (ll_word *)take(sizeof(ll_word) * ((size_t)zwords + 2 * res_slot_words<double>() * (size_t)most_slots));
+        d_step = (DiaStep *)take(sizeof(DiaStep) * kBrSteps * (size_t)nslice);
+        d_val = (double *)take(sizeof(double) * kBrSteps * kWave * (size_t)nslice);
+    };
+    lay();
+    SHK_TRY(ensure_ws2(ctx, used));
+    base = (char *)ctx->ws2;
+    lay();
+    const size_t head_bytes = (size_t)((char *)d_band - (char *)d_flag) + sizeof(int2) * (size_t)count;
+    std::vector<char> head(head_bytes, 0);
+    SHK_HIP(hipMemcpyAsync(d_flag, head.data(), head_bytes, hipMemcpyHostToDevice, st));
+    SHK_HIP(hipMemcpyAsync(d_off, row_off_host, sizeof(int) * (size_t)(count + 1), hipMemcpyHostToDevice, st));
+    SHK_HIP(hipMemcpyAsync(d_slice, slice_off.data(), sizeof(int) * (size_t)(count + 1), hipMemcpyHostToDevice, st));
+    hipLaunchKernelGGL(k_batch_dia, dim3((nslice + kDiaWaves - 1) / kDiaWaves), dim3(kBlock), 0, st, count,
+                       (const int *)d_off, (const int *)d_slice, nslice, (const int *)A->ptr,
+                       (const uint32_t *)A->ind, (const double *)A->val, d_step, d_val, (int *)d_flag, d_band);
+    SHK_HIP(hipGetLastError());
+    SHK_HIP(hipMemcpyAsync(head.data(), d_flag, head_bytes, hipMemcpyDeviceToHost, st));
+    SHK_HIP(hipStreamSynchronize(st));
+    const int *flag = (const int *)head.data();
+    const int2 *band = (const int2 *)(head.data() + ((char *)d_band - (char *)d_flag));
+    // an irregular slice stops before its last entries: the streaming path
+    // checks every column itself
+    if (flag[2]) return SHK_OK;
+    SHK_CHECK(flag[1] == 0, SHK_ERR_ARG, "cg_batched: a system has a column outside its own rows");
+    std::vector<int> team, share, slot_off(count + 1, 0);
+    std::vector<int2> slots;
+    if (!plan_resident(sizes, br_rows(flag[0]), ctx->num_cus, team, share, slots)) return SHK_OK;
+    const int nslot = (int)slots.size();
+    int window = 0;
+    for (int s = 0; s < count; s++) slot_off[s + 1] = slot_off[s] + 2 * team[s] * res_slot_words<double>();
+    const int nwords = slot_off[count];
+    for (int s = 0; s < count; s++)
+        window = std::max(window, (int)std::min<int64_t>(sizes[s], (int64_t)share[s] + band[s].x + band[s].y) + 1);
+    const size_t lds = sizeof(double) * (size_t)window;
+    if (lds > kResLds || window > 0xffff) return SHK_OK;
+    SHK_HIP(hipMemcpyAsync(d_slot, slot_off.data(), sizeof(int) * (size_t)(count + 1), hipMemcpyHostToDevice, st));
+    SHK_HIP(hipMemcpyAsync(d_team, team.data(), sizeof(int) * (size_t)count, hipMemcpyHostToDevice, st));
+    SHK_HIP(hipMemcpyAsync(d_share, share.data(), sizeof(int) * (size_t)count, hipMemcpyHostToDevice, st));
+    SHK_HIP(hipMemcpyAsync(d_slots, slots.data(), sizeof(int2) * (size_t)nslot, hipMemcpyHostToDevice, st));
+    ResBatch a{};
+    a.nslot = nslot;
+    a.slots = d_slots;
+    a.row_off = d_off;
+    a.slice_off = d_slice;
+    a.team = d_team;
+    a.share = d_share;
+    a.slot_off = d_slot;
+    a.band = d_band;
+    a.step = d_step;
+    a.val = d_val;
+    a.b = b;
+    a.x = x;
+    a.zw = d_words;
+    a.words = d_words + zwords;
+    a.n = n;
+    a.nwords = nwords;
+    a.steps = flag[0];
+    a.queue = ctx->red.ticket + 32;  // a ticket slot of its own
+    a.stall = d_flag + 3;
+    SHK_TRY(wall_clock_ticks(ctx, kTeamWaitSeconds, &a.limit));
+    a.tol = tol;
+    a.max_iter = max_iter;
+    a.its = d_its;
+    a.codes = d_codes;
+    const dim3 grid(std::min(nslot, ctx->num_cus));
+    std::lock_guard<std::mutex> lk(resident_mutex(ctx->device));
+    SHK_TRY(launch_batch(ctx, st, use_graph, [&](hipStream_t s) -> int {
+        hipLaunchKernelGGL(k_batch_res_reset, dim3(red_blocks(zwords + nwords)), dim3(kBlock), 0, s, a.queue, a.stall,
+                           zwords + nwords, d_words);
+        if (a.steps <= 5) hipLaunchKernelGGL(k_cg_batched_res<5>, grid, dim3(kBrThreads), lds, s, a);
+        else hipLaunchKernelGGL(k_cg_batched_res<7>, grid, dim3(kBrThreads), lds, s, a);
+        SHK_HIP(hipGetLastError());
+        return SHK_OK;
+    }));
+    unsigned stall = 0;
+    SHK_HIP(hipMemcpyAsync(its, d_its, sizeof(int) * (size_t)count, hipMemcpyDeviceToHost, st));
+    SHK_HIP(hipMemcpyAsync(codes, d_codes, sizeof(int) * (size_t)count, hipMemcpyDeviceToHost, st));
+    SHK_HIP(hipMemcpyAsync(&stall, a.stall, sizeof(unsigned), hipMemcpyDeviceToHost, st));
+    SHK_HIP(hipStreamSynchronize(st));
+    SHK_CHECK(stall == 0u, SHK_ERR_STATE,
+              "cg_batched: a team of work-groups waited too long for its members (is the GPU shared?)");
+    *solved = true;
+    return SHK_OK;
+}
+
 // Team sizes and the queue.  A system's estimated work is rows^1.5; it gets
 // k = ceil(work / (the batch's work per resident work-group)) members,
 // 1 <= k <= kMaxTeam (and at most its rows).  Slots are queued by their share
@@ -567,6 +924,12 @@ static int batched_common(shk_ctx ctx, shk_csr A64, shk_csr A32, int count, cons
     }
     SHK_TRY(check_device_ptr(dx, "x"));
     SHK_TRY(check_device_ptr(db, "b"));
+    if (!mixed) {
+        bool solved = false;
+        SHK_TRY(batched_resident(ctx, A64, count, row_off_host, sizes, (double *)dx, (const double *)db, tol, max_iter,
+                                 use_graph, its, codes, &solved));
+        if (solved) return SHK_OK;
+    }
     // work-groups drawing on the queue at a time
     const void *fn = mixed ? (rpp == 1   ? (const void *)k_cg_batched_ir<1>
                               : rpp == 2 ? (const void *)k_cg_batched_ir<2>
@@ -663,8 +1026,6 @@ static int batched_common(shk_ctx ctx, shk_csr A64, shk_csr A32, int count, cons
     SHK_CHECK(bad == 0, SHK_ERR_ARG, "cg_batched: a system has a column outside its own rows");
     SHK_HIP(hipMemcpyAsync(d_slots, slots.data(), slot_bytes, hipMemcpyHostToDevice, st));
     SHK_HIP(hipMemcpyAsync(d_team, team.data(), ord_bytes, hipMemcpyHostToDevice, st));
-    int clock_khz = 0;
-    SHK_HIP(hipDeviceGetAttribute(&clock_khz, hipDeviceAttributeWallClockRate, ctx->device));
     BatchArgs a{};
     a.count = count;
     a.nslot = nslot;
@@ -673,9 +1034,7 @@ static int batched_common(shk_ctx ctx, shk_csr A64, shk_csr A32, int count, cons
     a.team_cnt = d_tcnt;
     a.team_slot = d_tslot;
     a.stall = d_stall;
-    // wall_clock64 ticks per second (the device reports kHz; 100 MHz when it
-    // reports none)
-    a.limit = (long long)(clock_khz > 0 ? clock_khz : 100000) * 1000LL * kTeamWaitSeconds;
+    SHK_TRY(wall_clock_ticks(ctx, kTeamWaitSeconds, &a.limit));
     a.row_off = d_off;
     a.A64 = SellView{(const int *)A64->ptr, d_boff, d_scol, d_sval};
     if (mixed) a.A32 = SellView{(const int *)A64->ptr, d_boff, d_scol, d_sval32};
@@ -691,37 +1050,15 @@ static int batched_common(shk_ctx ctx, shk_csr A64, shk_csr A32, int count, cons
     a.its = d_its;
     a.codes = d_codes;
     a.queue = ctx->red.ticket + 32;  // a ticket slot of its own
-    auto enqueue = [&]() -> int {
-        hipLaunchKernelGGL(k_batch_reset, dim3((count + 255) / 256), dim3(256), 0, st, a.queue, a.stall,
+    std::lock_guard<std::mutex> lk(resident_mutex(ctx->device));
+    // the queue reset is a kernel node, not a memset node
+    SHK_TRY(launch_batch(ctx, st, use_graph, [&](hipStream_t cs) -> int {
+        hipLaunchKernelGGL(k_batch_reset, dim3((count + 255) / 256), dim3(256), 0, cs, a.queue, a.stall,
                            a.team_cnt, count);
         void *args[] = {&a};
-        SHK_HIP(hipLaunchKernel(fn, dim3(grid), dim3(group), args, 0, st));
+        SHK_HIP(hipLaunchKernel(fn, dim3(grid), dim3(group), args, 0, cs));
         return SHK_OK;
-    };
-    if (use_graph) {
-        // Recorded on the context's own non-blocking stream (the legacy
-        // default stream cannot be captured), launched on the caller's stream
-        // so it stays ordered after the copies above.  The queue reset is a
-        // kernel node, not a memset node.
-        hipGraph_t graph;
-        hipGraphExec_t exec;
-        hipStream_t cs = ctx->own;
-        hipStream_t keep = st;
-        st = cs;
-        SHK_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
-        int e = enqueue();
-        hipError_t ce = hipStreamEndCapture(cs, &graph);
-        st = keep;
-        SHK_TRY(e);
-        SHK_HIP(ce);
-        SHK_HIP(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
-        SHK_HIP(hipGraphLaunch(exec, st));
-        SHK_HIP(hipStreamSynchronize(st));
-        SHK_HIP(hipGraphExecDestroy(exec));
-        SHK_HIP(hipGraphDestroy(graph));
-    } else {
-        SHK_TRY(enqueue());
-    }
+    }));
     unsigned stall = 0;
     SHK_HIP(hipMemcpyAsync(its, d_its, ord_bytes, hipMemcpyDeviceToHost, st));
     SHK_HIP(hipMemcpyAsync(codes, d_codes, ord_bytes, hipMemcpyDeviceToHost, st));

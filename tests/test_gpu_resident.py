@@ -121,3 +121,50 @@ def test_resident_cg_exits(gpu):
     b = wl.apply(A, xt)
     runs = [_solve(A, b, "row", torch.float64, "jacobi") for _ in range(2)]
     assert np.array_equal(runs[0][2], runs[1][2]) and np.array_equal(runs[0][1].history, runs[1][1].history)
+
+
+def _systems(kind):
+    if kind == "one_member_each":
+        return [wl.aniso2d(n, n + 3, 4.0) for n in (1, 5, 31, 32, 45)]
+    if kind == "uneven_teams":
+        return [wl.aniso2d(n, n, e) for n, e in ((130, 3.0), (12, 1.0), (64, 50.0), (181, 1.0), (65, 9.0))]
+    if kind == "more_than_the_gpu_holds":
+        return [wl.aniso2d(30 + k % 101, 40 + k % 83, 1.0 + k % 7) for k in range(330)]
+    return [wl.diffusion3d(g, wl.normal(g ** 3, g, 0.0, 0.5)) for g in (5, 16, 27)]
+
+
+@pytest.mark.parametrize("kind", ["one_member_each", "uneven_teams", "more_than_the_gpu_holds", "three_d"])
+def test_resident_batch_matches_oracle(gpu, kind):
+    """Stacked stencil systems, one work-group or a team each: the oracle's
+    iteration counts within one and its solutions to the solve's accuracy; an
+    empty system and a zero right-hand side among them; twice the same bits."""
+    from oracle import oracle as orc
+    from seldon_amd import krylov as K
+    from seldon_amd.batched import cg_batched, stack
+    systems = _systems(kind)
+    empty = wl.CSR(0, 0, np.zeros(1, np.int32), np.zeros(0, np.int32), np.zeros(0))
+    systems.insert(2, empty)
+    A, row_off = stack(systems)
+    b = wl.apply(A, wl.uniform(A.m, 9))
+    b[row_off[1]:row_off[2]] = 0.0
+    Ag = K.Matrix(A, layout="rows")
+    bg = torch.tensor(b, device="cuda")
+    runs = []
+    for _ in range(2):
+        x = torch.full_like(bg, 7.0)
+        its, codes = cg_batched(Ag, row_off, x, bg, tol=1e-8, max_iter=5000)
+        runs.append((its, codes, x.cpu().numpy()))
+    for a, c in zip(*runs):
+        assert np.array_equal(a, c)
+    its, codes, x = runs[0]
+    for s in list(range(min(len(systems), 12))) + [len(systems) - 1]:
+        sl = slice(row_off[s], row_off[s + 1])
+        if s == 1:
+            assert its[s] == codes[s] == 0 and np.all(x[sl] == 7.0)
+            continue
+        if systems[s].m == 0:
+            assert its[s] == codes[s] == 0
+            continue
+        r = orc.solve("cg", systems[s], b[sl], tol=1e-8, max_iter=5000)
+        assert codes[s] == r.code == 0 and abs(int(its[s]) - r.nb_iter) <= 1
+        assert np.linalg.norm(x[sl] - r.x) <= 1e-6 * np.linalg.norm(r.x)

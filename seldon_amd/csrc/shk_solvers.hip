@@ -2055,13 +2055,14 @@ __global__ __launch_bounds__(kBlock) void k_gm_init0(int64_t n, const T *__restr
     block_partial<T, 2>(c, partials, gridDim.x, blockIdx.x);
 }
 
-// V_0 = r * (1/beta)  (:105-106)
+// V_0 = r * (1/beta)  (:105-106); 0 from n to the columns' stride
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_gm_v0(int64_t n, const T *__restrict__ r, T *__restrict__ v0, const KState<T> *st)
+__global__ __launch_bounds__(kBlock) void k_gm_v0(int64_t n, int64_t ldv, const T *__restrict__ r, T *__restrict__ v0,
+                                                  const KState<T> *st)
 {
     if (st->cyc_skip) return;
     const T sc = st->gm_scale;
-    GRID_STRIDE(i, n) v0[i] = r[i] * sc;
+    GRID_STRIDE(i, ldv) v0[i] = i < n ? r[i] * sc : (T)0;
 }
 
 // H(k, i) from the previous kernel's partials of (V_k, w) (the finish folded
@@ -2263,7 +2264,7 @@ __global__ void k_gm_solve(KState<T> *st)
 
 // x += sum_k s(k) V_k, Adds in k order per element (:169-170)
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_gm_xupd(int64_t n, const T *__restrict__ V, T *__restrict__ x, const KState<T> *st)
+__global__ __launch_bounds__(kBlock) void k_gm_xupd(int64_t n, int64_t ldv, const T *__restrict__ V, T *__restrict__ x, const KState<T> *st)
 {
     if (st->cyc_skip) return;
     __shared__ T coef[1024];
@@ -2274,7 +2275,7 @@ __global__ __launch_bounds__(kBlock) void k_gm_xupd(int64_t n, const T *__restri
         T xv = x[j];
         for (int k = 0; k < i; k++) {
             const T a = coef[k];
-            if (a != (T)0) xv += a * V[(size_t)k * n + j];
+            if (a != (T)0) xv += a * V[(size_t)k * ldv + j];
         }
         x[j] = xv;
     }
@@ -2582,19 +2583,36 @@ int bicgstab_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iterat
     return S.finish(it, code);
 }
 
+// the orthogonalisation of a step in one kernel (shk_gmres.hip)
 template <typename T>
-int gmres_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration *it, int *code)
+bool gm_ortho_fits(shk_ctx ctx, int64_t ldv, int m);
+size_t gm_ortho_words();
+template <typename T>
+int gm_ortho_start(shk_ctx ctx, void *slot);
+template <typename T>
+int gm_ortho(shk_ctx ctx, const T *V, int64_t ldv, T *w, int i, unsigned *epoch, void *slot, KState<T> *st);
+
+template <typename T>
+int gmres_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration *it, int *code,
+               bool resident = true)
 {
     const int m = it->parameter_restart;
     SHK_CHECK(m >= 1 && m <= 1000, SHK_ERR_ARG, "gmres: restart must be in [1, 1000]");
     Solve<T> S;
     const bool jac = prec == SHK_PREC_JACOBI;
     const size_t small = sizeof(double) * ((size_t)(m + 1) * (m + 1) + 3 * (size_t)(m + 1)) + 1024;
-    SHK_TRY(S.setup(ctx, A, (size_t)m + 3, small, it));
+    // columns of V at a stride of whole 256-byte lines (16-byte accesses for
+    // every n)
+    const int64_t ldv = ((int64_t)A->m + 31) & ~(int64_t)31;
+    resident = resident && gm_ortho_fits<T>(ctx, ldv, m);
+    const bool keep_x = resident && !it->init_guess_null;  // to start over from
+    SHK_TRY(S.setup(ctx, A, (size_t)m + 4 + (keep_x ? 1 : 0), small + 8 * gm_ortho_words() + 256 * (size_t)(m + 2), it));
     const int64_t n = S.n;
-    T *V = S.take(n * (int64_t)(m + 1));
-    T *w = S.take(n), *r = S.take(n);
+    T *V = S.take(ldv * (int64_t)(m + 1));
+    T *w = S.take(ldv), *r = S.take(n);
     double *H = (double *)S.take((int64_t)((small + sizeof(T) - 1) / sizeof(T)));
+    T *slot = S.take((int64_t)(8 * gm_ortho_words() / sizeof(T)));
+    T *x0 = keep_x ? S.take(n) : nullptr;
     double *gs = H + (size_t)(m + 1) * (m + 1), *gc = gs + (m + 1), *gsn = gc + (m + 1);
     SHK_HIP(hipMemsetAsync(H, 0, small, ctx->stream));
     {
@@ -2609,7 +2627,16 @@ int gmres_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration
     const T *dg = jac ? (const T *)A->diag : nullptr;
     hipStream_t st = ctx->stream;
     dim3 g(S.nb), blk(kBlock);
-    auto Vk = [&](int k) { return V + (size_t)k * n; };
+    auto Vk = [&](int k) { return V + (size_t)k * ldv; };
+    std::unique_lock<std::mutex> lk(resident_mutex(ctx->device), std::defer_lock);
+    unsigned epoch = 0;
+    if (resident) {
+        lk.lock();
+        SHK_TRY(gm_ortho_start<T>(ctx, slot));
+        if (ldv > n)
+            hipLaunchKernelGGL(k_fill<T>, dim3(1), blk, 0, st, ldv - n, (T)0, w + n, (const int *)nullptr);
+        if (keep_x) hipLaunchKernelGGL(k_copy<T>, g, blk, 0, st, n, (const T *)x, x0, (const int *)nullptr);
+    }
     // residual, preconditioning, beta, outer.Init (Gmres.cxx:82-95)
     if (it->init_guess_null) {
         hipLaunchKernelGGL(k_gm_init0<T>, g, blk, 0, st, n, b, dg, x, r, S.dst, S.partials);
@@ -2620,7 +2647,7 @@ int gmres_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration
         a.dot0 = kDotSelf; a.skip = &S.dst->skip;
         SHK_TRY(S.spmv(a, FinGmInit<T>{S.dst}));
     }
-    hipLaunchKernelGGL(k_gm_v0<T>, g, blk, 0, st, n, r, Vk(0), S.dst);
+    hipLaunchKernelGGL(k_gm_v0<T>, g, blk, 0, st, n, ldv, r, Vk(0), S.dst);
     SHK_HIP(hipGetLastError());
     SHK_TRY(S.read_state());
     const int step_chunk = 4;
@@ -2631,8 +2658,13 @@ int gmres_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration
         for (int i0 = 0; i0 < m; i0 += step_chunk) {
             for (int i = i0; i < std::min(m, i0 + step_chunk); i++) {
                 SpmvArgs<T> a{};
-                a.x = Vk(i); a.y_out = w; a.alpha = (T)1; a.mlt = 1; a.diag = dg;
-                a.dot0 = kDotVec; a.u0 = Vk(0); a.skip = &S.dst->skip;
+                a.x = Vk(i); a.y_out = w; a.alpha = (T)1; a.mlt = 1; a.diag = dg; a.skip = &S.dst->skip;
+                if (resident) {
+                    SHK_TRY(S.spmv(a, FinNone{}));
+                    SHK_TRY(gm_ortho<T>(ctx, V, ldv, w, i, &epoch, slot, S.dst));
+                    continue;
+                }
+                a.dot0 = kDotVec; a.u0 = Vk(0);
                 // each dot's finish is folded into the next kernel; the two
                 // partial buffers alternate so a kernel never overwrites the
                 // partials it is still reading
@@ -2661,16 +2693,23 @@ int gmres_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration
             }
             SHK_HIP(hipGetLastError());
             SHK_TRY(S.read_state());
+            if (S.hst->res_stall) {
+                // a work-group waited too long for the others (a shared GPU):
+                // start over with a kernel per pass
+                lk.unlock();
+                if (keep_x) SHK_HIP(hipMemcpyAsync(x, x0, sizeof(T) * n, hipMemcpyDeviceToDevice, st));
+                return gmres_impl<T>(ctx, A, x, b, prec, it, code, false);
+            }
             if (S.hst->gm_cycle_done || S.hst->done) break;
         }
         // cycle end: least squares, update, true residual (Gmres.cxx:165-178)
         hipLaunchKernelGGL(k_gm_solve<T>, dim3(1), dim3(64), 0, st, S.dst);
-        hipLaunchKernelGGL(k_gm_xupd<T>, g, blk, 0, st, n, (const T *)V, x, S.dst);
+        hipLaunchKernelGGL(k_gm_xupd<T>, g, blk, 0, st, n, ldv, (const T *)V, x, S.dst);
         SpmvArgs<T> a{};
         a.x = x; a.y_in = b; a.y_out = r; a.alpha = (T)-1; a.beta = (T)1; a.diag = dg;
         a.dot0 = kDotSelf; a.skip = &S.dst->cyc_skip;
         SHK_TRY(S.spmv(a, FinGmOuter<T>{S.dst}));
-        hipLaunchKernelGGL(k_gm_v0<T>, g, blk, 0, st, n, r, Vk(0), S.dst);
+        hipLaunchKernelGGL(k_gm_v0<T>, g, blk, 0, st, n, ldv, r, Vk(0), S.dst);
         SHK_HIP(hipGetLastError());
         SHK_TRY(S.read_state());
     }

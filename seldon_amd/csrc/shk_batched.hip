@@ -575,9 +575,9 @@ __global__ __launch_bounds__(kBlock) void k_batch_dia(int count, const int *row_
     if (outside) atomicOr(flag + 1, 1);
     if (irregular) atomicOr(flag + 2, 1);
     if (lane == 0) {
-        atomicMax(flag, k);
-        atomicMax(&band[s].x, left);
-        atomicMax(&band[s].y, right);
+        dia_max(flag, k);
+        dia_max(&band[s].x, left);
+        dia_max(&band[s].y, right);
         for (; k < kBrSteps; k++) step[s0 + k] = DiaStep{0ull, 0, 0};
     }
 }

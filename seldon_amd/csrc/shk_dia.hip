@@ -61,9 +61,9 @@ __global__ __launch_bounds__(kBlock) void k_dia_build(int m, const int *ptr, con
     if (!fill) {
         if (!ok) atomicOr(flag + 1, 1);
         if (lane == 0) {
-            atomicMax(flag, k);
-            atomicMax(flag + 2, left);
-            atomicMax(flag + 3, right);
+            dia_max(flag, k);
+            dia_max(flag + 2, left);
+            dia_max(flag + 3, right);
         }
     } else {
         for (; k < steps; k++) {
@@ -118,7 +118,8 @@ int dia_build(shk_csr A, const int *ptr, const int *mid, const uint32_t *ind, co
     A->dia_steps = h[0];
     A->dia_left = h[2];
     A->dia_right = h[3];
-    A->dia_groups = (slices + kDiaWaves - 1) / kDiaWaves;
+    A->dia_block = slices <= 4096 ? kBlock : 1024;
+    A->dia_groups = (int)(((int64_t)slices * kWave + A->dia_block - 1) / A->dia_block);
     SHK_HIP(hipMalloc(&A->dia_step, sizeof(DiaStep) * (size_t)slices * h[0]));
     SHK_HIP(hipMalloc((void **)&A->dia_src, sizeof(int) * (size_t)slots));
     SHK_HIP(hipMalloc(&A->dia_val, dsize(A->dtype) * (size_t)slots));
@@ -155,17 +156,18 @@ void dia_free(shk_csr A)
     A->dia_steps = A->dia_groups = 0;
 }
 
+// Work-groups of a product with fused dots: persistent, two 1024-thread ones
+// per CU at most (see k_dia).
 int dia_grid(shk_csr A)
 {
     const int q = (A->dia_groups + kNumXcd - 1) / kNumXcd;
-    return kNumXcd * std::min(q, std::max(1, A->ctx->num_cus * kDiaWgPerCu / kNumXcd));
+    return kNumXcd * std::min(q, std::max(1, A->ctx->num_cus * (2048 / A->dia_block) / kNumXcd));
 }
 
 template <typename T, int MODE>
-static void launch_dia_mode(shk_csr A, const SpmvArgs<T> &a, const DiaView &v, dim3 grid)
+static void launch_dia_mode(shk_csr A, const SpmvArgs<T> &a, const DiaView &v, dim3 grid, dim3 blk)
 {
     hipStream_t s = A->ctx->stream;
-    const dim3 blk(kBlock);
     switch (v.steps) {
 #define SHK_DIA_CASE(k) \
     case k: hipLaunchKernelGGL((k_dia<T, MODE, k>), grid, blk, 0, s, a, v); break;
@@ -186,12 +188,18 @@ static void launch_dia_mode(shk_csr A, const SpmvArgs<T> &a, const DiaView &v, d
 template <typename T>
 int launch_dia(shk_csr A, SpmvArgs<T> &a)
 {
-    const DiaView v{A->dia_steps, A->dia_groups, (A->dia_groups + kNumXcd - 1) / kNumXcd, (const DiaStep *)A->dia_step};
-    const dim3 grid(dia_grid(A));
+    const bool dots = a.dot0 != kDotNone || a.dot1 != kDotNone;
+    // without dots nothing counts the work-groups: small ones, each a single
+    // step, dealt out as CUs come free
+    const int block = dots ? A->dia_block : kBlock;
+    const int groups = dots ? A->dia_groups : (int)(((int64_t)A->m + kBlock - 1) / kBlock);
+    const int q = (groups + kNumXcd - 1) / kNumXcd;
+    const DiaView v{A->dia_steps, groups, q, (const DiaStep *)A->dia_step};
+    const dim3 grid(dots ? dia_grid(A) : kNumXcd * q), blk(block);
     a.val = (const T *)A->dia_val;
-    if (A->storage == SHK_ARRAYROWSPARSE) launch_dia_mode<T, kArray>(A, a, v, grid);
-    else if (A->storage == SHK_ROWSYMSPARSE) launch_dia_mode<T, kSym>(A, a, v, grid);
-    else launch_dia_mode<T, kCsr>(A, a, v, grid);
+    if (A->storage == SHK_ARRAYROWSPARSE) launch_dia_mode<T, kArray>(A, a, v, grid, blk);
+    else if (A->storage == SHK_ROWSYMSPARSE) launch_dia_mode<T, kSym>(A, a, v, grid, blk);
+    else launch_dia_mode<T, kCsr>(A, a, v, grid, blk);
     return (int)grid.x;
 }
 template int launch_dia<double>(shk_csr, SpmvArgs<double> &);

@@ -32,7 +32,7 @@ constexpr int kDiaMaxSteps = 32;
 // the other layouts' own overheads)
 constexpr double kDiaFill = 1.25;
 constexpr int64_t kDiaSlack = 4096;  // slots a small matrix may add to that
-constexpr int kDiaWaves = kBlock / kWave;  // slices per work-group step
+constexpr int kDiaWaves = kBlock / kWave;  // slices per work-group of the build
 
 struct alignas(16) DiaStep {
     uint64_t mask;  // rows (lanes) of the slice with an entry at this offset
@@ -40,9 +40,16 @@ struct alignas(16) DiaStep {
     int direct;     // RowSymSparse: a transposed-part step
 };
 
+// raise *p to v; almost every wavefront finds it there already, and the read
+// spares an atomic on one address (100K of them were 0.5 ms)
+__device__ __forceinline__ void dia_max(int *p, int v)
+{
+    if (__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < v) atomicMax(p, v);
+}
+
 struct DiaView {
     int steps;              // per slice
-    int groups;             // work-group steps: kDiaWaves slices each
+    int groups;             // work-group steps: a slice per wavefront each
     int q;                  // groups per XCD
     const DiaStep *step;    // [slices * steps]
 };
@@ -89,8 +96,13 @@ __device__ __forceinline__ T dia_row(const SpmvArgs<T> &a, const DiaView &v, int
 
 // Work-groups of one XCD take consecutive groups of that XCD's contiguous
 // range together, so the x lines neighbouring slices share stay in its L2.
+// Work-groups of 256 threads up to 4096 slices, so small matrices reach every
+// CU, of 1024 above, at most two per CU: each leaves one partial per fused
+// dot, and every work-group of the next kernel sums them all (2048 partials
+// instead of 512 made the vector kernels of a 2M-row BiCgStab iteration 22 to
+// 33% slower).
 template <typename T, int MODE, int KS>
-__global__ __launch_bounds__(kBlock, 8) void k_dia(SpmvArgs<T> a, DiaView v)
+__global__ __launch_bounds__(1024, 8) void k_dia(SpmvArgs<T> a, DiaView v)
 {
     if (a.skip && *a.skip) return;
     const int lane = threadIdx.x & (kWave - 1);
@@ -99,7 +111,7 @@ __global__ __launch_bounds__(kBlock, 8) void k_dia(SpmvArgs<T> a, DiaView v)
     const int end = min(v.groups, (xcd + 1) * v.q);
     T c[2] = {(T)0, (T)0};
     for (int g = xcd * v.q + (int)(blockIdx.x / kNumXcd); g < end; g += stride) {
-        const int slice = g * kDiaWaves + w;
+        const int slice = g * (int)(blockDim.x / kWave) + w;
         const int row = slice * kWave + lane;
         if (slice * kWave >= a.m) break;  // wave-uniform: the last group's empty slices
         const bool in = row < a.m;

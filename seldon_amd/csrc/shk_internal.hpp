@@ -136,7 +136,7 @@ struct shk_csr_s {
     // Diagonal-slice copy of the entries (shk_dia.hpp), AUTO layouts of
     // stencil and banded matrices: the SpMV reads it when it is there, every
     // other use the layout above
-    int dia_steps = 0, dia_groups = 0;
+    int dia_steps = 0, dia_groups = 0, dia_block = 0;
     int dia_left = 0, dia_right = 0;   // largest row - col and col - row
     void *dia_step = nullptr;          // [slices * dia_steps] DiaStep
     void *dia_val = nullptr;           // [slices * dia_steps * 64] values
@@ -299,9 +299,8 @@ int sliced_set_values(shk_csr A);
 int dia_build(shk_csr A, const int *ptr, const int *mid, const uint32_t *ind, const int64_t *src_of, bool *applies);
 int dia_set_values(shk_csr A, const void *dval);
 void dia_free(shk_csr A);
-// work-groups of its SpMV: at most kDiaWgPerCu per CU
+// work-groups of its SpMV
 int dia_grid(shk_csr A);
-constexpr int kDiaWgPerCu = 8;
 // the matrix behind A's transposed products (built on first use)
 int transpose_of(shk_csr A, shk_csr *out);
 void sliced_free(shk_csr A);

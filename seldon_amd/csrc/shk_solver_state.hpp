@@ -19,7 +19,8 @@ struct KState {
     int max_iter, nb_iter, error_code, fail;
     int done, init_failed, hist_len, hist_cap;
     int skip;          // done, or (GMRES) the current cycle is over
-    int stop_slot;     // BiCgStab / TfQmr: loop slot (TfQmr: half step) that ended the solve
+    int stop_slot;     // TfQmr: half step that ended the solve
+    int bi_nb, bi_stop;  // BiCgStab: iterations at Finished(s), which ended the solve
     // resident Cg: a member's wait ran out / the solve ran to its end
     unsigned res_stall, res_ran;
     double *hist;
@@ -181,6 +182,10 @@ struct FinBiTop {
     int inc, slot;  // rho_1 also kept in rho_pp[slot] (the head folded into the p update)
     __device__ void operator()(const T (&s)[2]) const
     {
+        if (st->bi_stop) {
+            it_stop(st);
+            return;
+        }
         if (inc) {
             st->rho_2 = st->rho_1;
             st->nb_iter++;
@@ -216,19 +221,23 @@ struct FinBiSigma {  // sigma = (rtilde, v); breakdown #3; alpha (:104-110)
             return;
         }
         st->alpha = st->rho_1 / s[0];
+        st->bi_nb = st->nb_iter + 1;
     }
 };
 
+// ++iter; Finished(s) (:115-121), recorded by the first work-group of
+// k_bi_xr.  Every work-group of that kernel decides alike, from the same total
+// and bi_nb, and still has the x update to do when the solve ends here, so
+// the end is left in bi_stop; the loop head after it sets skip.
 template <typename T>
-struct FinBiS {  // ++iter; Finished(s) (:115-121)
+struct FinBiS {
     KState<T> *st;
-    int slot;
-    __device__ void operator()(const T (&s)[2]) const
+    __device__ void operator()(T ss) const
     {
-        st->nb_iter++;
-        if (it_finished(st, (double)sqrt_t(s[0]), st->nb_iter, st->max_iter)) {
-            st->stop_slot = slot;
-            it_stop(st);
+        st->nb_iter = st->bi_nb;
+        if (it_finished(st, (double)sqrt_t(ss), st->bi_nb, st->max_iter)) {
+            st->done = 1;
+            st->bi_stop = 1;
         }
     }
 };

@@ -379,6 +379,10 @@ __global__ __launch_bounds__(kBlock) void k_bi_p_top(int64_t n, const T *__restr
                                                      KState<T> *st, const T *prev, int prev_nb, int slot)
 {
     if (st->skip) return;
+    if (st->bi_stop) {  // Finished(s) ended the solve in the slot before
+        if (blockIdx.x == 0 && threadIdx.x == 0) it_stop(st);
+        return;
+    }
     const int64_t i0 = blockIdx.x * (int64_t)kBlock + threadIdx.x, stride = (int64_t)gridDim.x * kBlock;
     T pv0[kPre], vv[kPre], rv[kPre];
 #pragma unroll
@@ -481,23 +485,14 @@ __global__ __launch_bounds__(kBlock) void k_bi_s(int64_t n, const T *__restrict_
     block_partial<T, 2>(c, partials, gridDim.x, blockIdx.x);
 }
 
-// Finished(s) ended the solve in this slot: x += alpha phat (:116-120)
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_bi_fix(int64_t n, const T *__restrict__ phat, T *__restrict__ x, const KState<T> *st,
-                                                   int slot)
-{
-    if (st->stop_slot != slot) return;
-    const T alpha = st->alpha;
-    if (alpha == (T)0) return;
-    GRID_STRIDE(i, n) x[i] += alpha * phat[i];
-}
-
-// x += alpha phat; x += omega shat; r = s; r += (-omega) t (:132-137);
-// sums r^2, rtilde*r for the next loop head
+// ++iter; Finished(s) from the |s|^2 partials; when it ends the solve,
+// x += alpha phat (:115-121).  Else x += alpha phat; x += omega shat; r = s;
+// r += (-omega) t (:132-137); sums r^2, rtilde*r for the next loop head
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_bi_xr(int64_t n, const T *__restrict__ phat, const T *__restrict__ shat, const T *__restrict__ s,
                                                   const T *__restrict__ t, const T *__restrict__ rt, T *__restrict__ x, T *__restrict__ r, KState<T> *st,
-                                                  const T *prev, int prev_nb, T *partials)
+                                                  const T *prev, int prev_nb, const T *sprev, int sprev_nb,
+                                                  T *partials)
 {
     if (st->skip) return;
     // six vectors: half the usual number of elements ahead of the fold
@@ -516,16 +511,30 @@ __global__ __launch_bounds__(kBlock) void k_bi_xr(int64_t n, const T *__restrict
             rtp[u] = rt[i];
         }
     }
-    // omega = (t, s) / (t, t) from the SpMV's partials (:129), folded in
+    // Finished(s), then omega = (t, s) / (t, t) from the SpMV's partials
+    // (:129), both folded in
     __shared__ T omega_sh;
+    __shared__ int stop_sh;
     {
-        T tot[2];
+        T tot[2], ss[2];
+        grid_total<T>(sprev, sprev_nb, ss);
         grid_total<T>(prev, prev_nb, tot);
         if (threadIdx.x == 0) {
+            const double reste = st->facteur * (double)sqrt_t(ss[0]);
+            stop_sh = (reste < st->tol) || (st->bi_nb >= st->max_iter);
             omega_sh = tot[0] / tot[1];
-            if (blockIdx.x == 0) FinBiOmega<T>{st}(tot);
+            if (blockIdx.x == 0) {
+                FinBiS<T>{st}(ss[0]);
+                if (!stop_sh) FinBiOmega<T>{st}(tot);
+            }
         }
         __syncthreads();
+    }
+    if (stop_sh) {
+        const T a = st->alpha;
+        if (a == (T)0) return;
+        for (int64_t i = i0; i < n; i += stride) x[i] += a * phat[i];
+        return;
     }
     const T alpha = st->alpha, omega = omega_sh, momega = -omega_sh;
     const bool aa = alpha != (T)0, ao = omega != (T)0, am = momega != (T)0;
@@ -2409,16 +2418,17 @@ struct Solve {
         return launch_spmv<T, Fin>(A, a, fin);
     }
 
-    // The iteration loop: body(stream) enqueues one chunk of iterations on
-    // the context's stream and the state is read back after each chunk,
-    // until the solve stops or `limit` iterations have been enqueued.
+    // The iteration loop: body(stream, count) enqueues one chunk of count
+    // iterations on the context's stream and the state is read back after each
+    // chunk, until the solve stops or `limit` iterations have been enqueued
+    // (the last chunk holds what is left of them, one at least).
     // (Recording the chunk once into a hipGraph and replaying it was
     // measured: no gain, the per-kernel cost is on the device side.)
     template <class Body>
     int run_chunks(int64_t limit, int chunk, Body body)
     {
         for (int64_t done_its = 0; done_its <= limit; done_its += chunk) {
-            SHK_TRY(body(ctx->stream));
+            SHK_TRY(body(ctx->stream, (int)std::min<int64_t>(chunk, std::max<int64_t>(limit - done_its, 1))));
             SHK_TRY(read_state());
             if (hst->done) break;
         }
@@ -2482,12 +2492,12 @@ int cg_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration *i
     if (S.hst->res_stall)  // a member waited too long for the others (a shared GPU): x is as it was, start over
         return cg_impl<T>(ctx, A, x, b, prec, it, code, ext, ext_cap, false);
     const int64_t limit = (int64_t)std::max(it->max_iter, 0) + 2;
-    // the loop head of iterations 1 .. kChunk - 1 of a chunk is folded into
+    // the loop head of iterations 1 .. of a chunk is folded into
     // the next kernel (identity: k_cg_p_top; Jacobi: k_cg_z_top, and rho =
     // (r, z) into k_cg_p_rho); the head before a chunk's first iteration runs
     // as its own finish (slot 0), so each chunk ends with the state read back
-    SHK_TRY(S.run_chunks(limit, kChunk, [&](hipStream_t cs) -> int {
-        for (int k = 0; k < kChunk; k++) {
+    SHK_TRY(S.run_chunks(limit, kChunk, [&](hipStream_t cs, int count) -> int {
+        for (int k = 0; k < count; k++) {
             if (jac) {
                 if (k == 0)
                     hipLaunchKernelGGL(k_cg_z<T>, g, blk, 0, cs, n, r, dg, z, S.dst, S.part[0]);
@@ -2508,7 +2518,7 @@ int cg_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration *i
             SHK_TRY(S.spmv(a, FinDefer{}));  // (p, q): finished inside k_cg_xr
             hipLaunchKernelGGL(k_cg_xr<T>, g, blk, 0, cs, n, p, q, x, r, S.dst, (const T *)S.part[0],
                                a.grid_used, S.part[1]);
-            if (k == kChunk - 1)
+            if (k == count - 1)
                 grid_finish<T>(cs, (const T *)S.part[1], S.nb, (const int *)&S.dst->skip,
                                FinCgTop<T>{S.dst, 1, jac ? 0 : 1, 0});
         }
@@ -2544,12 +2554,9 @@ int bicgstab_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iterat
     S.fin(FinBiTop<T>{S.dst, 0, 0});
     SHK_HIP(hipGetLastError());
     const int64_t limit = (int64_t)std::max(it->max_iter, 0) / 2 + 2;
-    // a loop's slot (its place in the chunk) names the Finished(s) that
-    // stopped the solve; the chunk is replayed, so slots repeat across
-    // chunks, but a stopped solve replays no further chunk
-    SHK_TRY(S.run_chunks(limit, kChunk, [&](hipStream_t cs) -> int {
-        for (int slot = 0; slot < kChunk; slot++) {
-            // the loop head of slots 1 .. kChunk - 1 is folded into k_bi_p_top;
+    SHK_TRY(S.run_chunks(limit, kChunk, [&](hipStream_t cs, int count) -> int {
+        for (int slot = 0; slot < count; slot++) {
+            // the loop head of a chunk's later slots is folded into k_bi_p_top;
             // the head before a chunk's first slot runs as its own finish
             if (slot == 0)
                 hipLaunchKernelGGL(k_bi_p<T>, g, blk, 0, cs, n, r, v, p, dg, phat, S.dst);
@@ -2562,17 +2569,15 @@ int bicgstab_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iterat
             a.partials = S.part[0];
             SHK_TRY(S.spmv(a, FinDefer{}));  // sigma: finished inside k_bi_s
             hipLaunchKernelGGL(k_bi_s<T>, g, blk, 0, cs, n, r, v, s, dg, shat, S.dst, (const T *)S.part[0],
-                               a.grid_used, S.part[1]);
-            grid_finish<T>(cs, (const T *)S.part[1], S.nb, (const int *)&S.dst->skip, FinBiS<T>{S.dst, slot});
-            hipLaunchKernelGGL(k_bi_fix<T>, g, blk, 0, cs, n, phat, x, S.dst, slot);
+                               a.grid_used, S.part[2]);
             SpmvArgs<T> b2{};
             b2.x = shat; b2.y_out = t; b2.alpha = (T)1; b2.mlt = 1;
             b2.dot0 = kDotVec; b2.u0 = s; b2.dot1 = kDotSelf; b2.skip = &S.dst->skip;
             b2.partials = S.part[0];
             SHK_TRY(S.spmv(b2, FinDefer{}));  // omega: finished inside k_bi_xr
             hipLaunchKernelGGL(k_bi_xr<T>, g, blk, 0, cs, n, phat, shat, s, t, rt, x, r, S.dst,
-                               (const T *)S.part[0], b2.grid_used, S.part[1]);
-            if (slot == kChunk - 1)
+                               (const T *)S.part[0], b2.grid_used, (const T *)S.part[2], S.nb, S.part[1]);
+            if (slot == count - 1)
                 grid_finish<T>(cs, (const T *)S.part[1], S.nb, (const int *)&S.dst->skip,
                                FinBiTop<T>{S.dst, 1, 0});
         }
@@ -2746,8 +2751,8 @@ int cgs_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration *
     S.fin(FinLanczosTop<T>{S.dst, 0});
     SHK_HIP(hipGetLastError());
     const int64_t limit = (int64_t)std::max(it->max_iter, 0) / 2 + 2;
-    SHK_TRY(S.run_chunks(limit, kChunk, [&](hipStream_t cs) -> int {
-        for (int k = 0; k < kChunk; k++) {
+    SHK_TRY(S.run_chunks(limit, kChunk, [&](hipStream_t cs, int count) -> int {
+        for (int k = 0; k < count; k++) {
             hipLaunchKernelGGL(k_cgs_pu<T>, g, blk, 0, cs, n, r, q, p, u, dg, phat, S.dst);
             SpmvArgs<T> a{};
             a.x = phat; a.y_out = vhat; a.alpha = (T)1; a.mlt = 1;
@@ -2799,8 +2804,8 @@ int bicg_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration 
     S.fin(FinLanczosTop<T>{S.dst, 0});
     SHK_HIP(hipGetLastError());
     const int64_t limit = (int64_t)std::max(it->max_iter, 0) / 2 + 2;
-    SHK_TRY(S.run_chunks(limit, kChunk, [&](hipStream_t cs) -> int {
-        for (int k = 0; k < kChunk; k++) {
+    SHK_TRY(S.run_chunks(limit, kChunk, [&](hipStream_t cs, int count) -> int {
+        for (int k = 0; k < count; k++) {
             hipLaunchKernelGGL(k_bicg_p<T>, g, blk, 0, cs, n, z, zt, p, pt, S.dst);
             SpmvArgs<T> a{};
             a.x = p; a.y_out = q; a.alpha = (T)1; a.mlt = 1;
@@ -2855,8 +2860,8 @@ int tfqmr_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration
     hipLaunchKernelGGL(k_tq_v<T>, g_, blk, 0, st, n, tmp, dg, g, v, (const T *)h, rt, 1, S.dst, S.partials);
     SHK_HIP(hipGetLastError());
     const int64_t limit = (int64_t)std::max(it->max_iter, 0) / 2 + 2;
-    SHK_TRY(S.run_chunks(limit, kChunk, [&](hipStream_t cs) -> int {
-        for (int slot = 0; slot < kChunk; slot++) {
+    SHK_TRY(S.run_chunks(limit, kChunk, [&](hipStream_t cs, int count) -> int {
+        for (int slot = 0; slot < count; slot++) {
             S.fin(FinTqSigma<T>{S.dst});
             hipLaunchKernelGGL(k_tq_y0<T>, g_, blk, 0, cs, n, y1, v, y0, S.dst);
             SpmvArgs<T> a{};
@@ -2915,8 +2920,8 @@ int qmr_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration *
     S.fin(FinQmrTop<T>{S.dst, 1});
     SHK_HIP(hipGetLastError());
     const int64_t limit = (int64_t)std::max(it->max_iter, 0) / 2 + 2;
-    SHK_TRY(S.run_chunks(limit, kChunk, [&](hipStream_t cs) -> int {
-        for (int k = 0; k < kChunk; k++) {
+    SHK_TRY(S.run_chunks(limit, kChunk, [&](hipStream_t cs, int count) -> int {
+        for (int k = 0; k < count; k++) {
             hipLaunchKernelGGL(k_qmr_scale<T>, g, blk, 0, cs, n, v, y, w, dg, z, S.dst, S.partials);
             S.fin(FinQmrDelta<T>{S.dst});
             hipLaunchKernelGGL(k_qmr_pq<T>, g, blk, 0, cs, n, y, zsrc, p, q, S.dst);
@@ -2975,8 +2980,8 @@ int cgne_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration 
     hipLaunchKernelGGL(k_cgne_r0<T>, g, blk, 0, st, n, (const T *)q, r, x, it->init_guess_null ? 1 : 0, S.dst);
     SHK_HIP(hipGetLastError());
     const int64_t limit = (int64_t)std::max(it->max_iter, 0) / 2 + 2;
-    SHK_TRY(S.run_chunks(limit, kChunk, [&](hipStream_t cs) -> int {
-        for (int k = 0; k < kChunk; k++) {
+    SHK_TRY(S.run_chunks(limit, kChunk, [&](hipStream_t cs, int count) -> int {
+        for (int k = 0; k < count; k++) {
             hipLaunchKernelGGL(k_cgne_z<T>, g, blk, 0, cs, n, (const T *)r, dg, z, S.dst, S.partials);
             S.fin(FinCgneRho<T>{S.dst});
             hipLaunchKernelGGL(k_cgne_p<T>, g, blk, 0, cs, n, zsrc, p, S.dst);
@@ -3041,8 +3046,8 @@ int lsqr_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, shk_iteration *it, int *
     hipLaunchKernelGGL(k_lsqr_v0<T>, g, blk, 0, st, n, v, w, S.dst);
     SHK_HIP(hipGetLastError());
     const int64_t limit = (int64_t)std::max(it->max_iter, 0) / 2 + 2;
-    SHK_TRY(S.run_chunks(limit, kChunk, [&](hipStream_t cs) -> int {
-        for (int k = 0; k < kChunk; k++) {
+    SHK_TRY(S.run_chunks(limit, kChunk, [&](hipStream_t cs, int count) -> int {
+        for (int k = 0; k < count; k++) {
             // Swap(u1, u); Swap(v1, v) after every loop: even slots use the
             // first assignment, odd ones the other (a chunk has an even count)
             T *uc = (k & 1) ? u1 : u, *un = (k & 1) ? u : u1;
@@ -3105,8 +3110,8 @@ int bicgcr_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteratio
     grid_finish<T>(st, (const T *)S.part[0], S.nb, (const int *)&S.dst->skip, FinBcrTop<T>{S.dst, 1});
     SHK_HIP(hipGetLastError());
     const int64_t limit = (int64_t)std::max(it->max_iter, 0) + 2;
-    SHK_TRY(S.run_chunks(limit, kChunk, [&](hipStream_t cs) -> int {
-        for (int k = 0; k < kChunk; k++) {
+    SHK_TRY(S.run_chunks(limit, kChunk, [&](hipStream_t cs, int count) -> int {
+        for (int k = 0; k < count; k++) {
             grid_finish<T>(cs, (const T *)S.part[1], S.nb, (const int *)&S.dst->skip, FinBcrMu<T>{S.dst});
             hipLaunchKernelGGL(k_bcr_xvs<T>, g, blk, 0, cs, n, (const T *)p, (const T *)a, (const T *)w, x, v, s,
                                S.dst, S.part[0]);
@@ -3158,8 +3163,8 @@ int qmrsym_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteratio
     S.fin(FinQmsTop<T>{S.dst, 1});
     SHK_HIP(hipGetLastError());
     const int64_t limit = (int64_t)std::max(it->max_iter, 0) + 2;
-    SHK_TRY(S.run_chunks(limit, kChunk, [&](hipStream_t cs) -> int {
-        for (int k = 0; k < kChunk; k++) {
+    SHK_TRY(S.run_chunks(limit, kChunk, [&](hipStream_t cs, int count) -> int {
+        for (int k = 0; k < count; k++) {
             hipLaunchKernelGGL(k_qms_scale<T>, g, blk, 0, cs, n, v, y, S.dst, S.partials);
             S.fin(FinQmsDelta<T>{S.dst});
             hipLaunchKernelGGL(k_qms_p<T>, g, blk, 0, cs, n, (const T *)y, p, S.dst);
@@ -3218,8 +3223,8 @@ int minres_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteratio
     SHK_HIP(hipGetLastError());
     int64_t t = 0;  // iterations enqueued: the buffers' rotation
     const int64_t limit = (int64_t)std::max(it->max_iter, 0) + 2;
-    SHK_TRY(S.run_chunks(limit, kChunk, [&](hipStream_t cs) -> int {
-        for (int k = 0; k < kChunk; k++, t++) {
+    SHK_TRY(S.run_chunks(limit, kChunk, [&](hipStream_t cs, int count) -> int {
+        for (int k = 0; k < count; k++, t++) {
             T *u = ub[t % 2], *u_old = ub[(t + 1) % 2], *v = vb[t % 2], *v_old = vb[(t + 1) % 2];
             T *w = wb[t % 3], *w_old = wb[(t + 2) % 3], *w_new = wb[(t + 1) % 3];
             SpmvArgs<T> a{};
@@ -3276,8 +3281,8 @@ int symmlq_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteratio
     SHK_HIP(hipGetLastError());
     int64_t t = 0;  // iterations enqueued: the v / u buffers' rotation
     const int64_t limit = (int64_t)std::max(it->max_iter, 0) + 2;
-    SHK_TRY(S.run_chunks(limit, kChunk, [&](hipStream_t cs) -> int {
-        for (int k = 0; k < kChunk; k++, t++) {
+    SHK_TRY(S.run_chunks(limit, kChunk, [&](hipStream_t cs, int count) -> int {
+        for (int k = 0; k < count; k++, t++) {
             T *u = ub[t % 2], *u_old = ub[(t + 1) % 2], *v = vb[t % 2], *v_old = vb[(t + 1) % 2];
             if (t > 0)
                 hipLaunchKernelGGL(k_sy_upd<T>, g, blk, 0, cs, n, (const T *)r, (const T *)z, v, u, w_bar, x,
@@ -3334,8 +3339,8 @@ int qcgs_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration 
     SHK_HIP(hipGetLastError());
     const int64_t limit = (int64_t)std::max(it->max_iter, 0) / 2 + 2;
     bool first = true;
-    SHK_TRY(S.run_chunks(limit, kChunk, [&](hipStream_t cs) -> int {
-        for (int k = 0; k < kChunk; k++) {
+    SHK_TRY(S.run_chunks(limit, kChunk, [&](hipStream_t cs, int count) -> int {
+        for (int k = 0; k < count; k++) {
             grid_finish<T>(cs, (const T *)S.part[0], S.nb, (const int *)&S.dst->skip,
                            FinQcTop<T>{S.dst, first ? 1 : 0});
             first = false;
@@ -3412,7 +3417,7 @@ int gcr_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration *
     const int ni = (m + 1) / 2;  // inner iterations of a full cycle
     const int cycles = std::max(1, kChunk / ni);
     const int64_t limit = (int64_t)std::max(it->max_iter, 0) / m + 2;
-    SHK_TRY(S.run_chunks(limit, cycles, [&](hipStream_t cs) -> int {
+    SHK_TRY(S.run_chunks(limit, cycles, [&](hipStream_t cs, int) -> int {
         for (int c = 0; c < cycles; c++) {
             grid_finish<T>(cs, (const T *)S.part[0], S.nb, (const int *)&S.dst->skip, FinGcOuter<T>{S.dst, m});
             hipLaunchKernelGGL(k_gc_p0<T>, g, blk, 0, cs, n, (const T *)r, pbase, S.dst);
@@ -3512,7 +3517,7 @@ int bicgstabl_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_itera
     SHK_HIP(hipGetLastError());
     const int cycles = std::max(1, kChunk / l);
     const int64_t limit = (int64_t)std::max(it->max_iter, 0) / (2 * l) + 2;
-    SHK_TRY(S.run_chunks(limit, cycles, [&](hipStream_t cs) -> int {
+    SHK_TRY(S.run_chunks(limit, cycles, [&](hipStream_t cs, int) -> int {
         const int *skip = (const int *)&S.dst->skip;
         for (int c = 0; c < cycles; c++) {
             grid_finish<T>(cs, (const T *)S.part[0], S.nb, skip, FinBlTop<T>{S.dst});

@@ -33,8 +33,8 @@
 // What bounds it is latency: the two exchanges, the two divisions and the
 // square root behind them, and, on 3-D grids, the halo (two planes per
 // member).  Cg per iteration, launched kernels -> this (FP64): 2-D Laplacian
-// 64^2 16 -> 3.5 us, 256^2 16.2 -> 4.4, 512^2 20 -> 6.1, 1000^2 35 -> 11; 3-D
-// diffusion with Jacobi 40^3 22 -> 8.2, 64^3 26 -> 15.6, 78^3 34 -> 23.
+// 64^2 16 -> 4.0 us, 256^2 16.2 -> 4.0, 512^2 20 -> 5.5, 1000^2 35 -> 10; 3-D
+// diffusion with Jacobi 40^3 22 -> 7.4, 64^3 26 -> 13.2, 78^3 34 -> 19.7.
 #pragma once
 
 #include "shk_kernels.hpp"
@@ -54,36 +54,91 @@ typedef unsigned ll_u4 __attribute__((ext_vector_type(4)));
 typedef unsigned ll_u2 __attribute__((ext_vector_type(2)));
 
 struct LlBuf {
+    template <typename T>
+    using Raw = typename std::conditional<sizeof(T) == 8, ll_u4, ll_u2>::type;
     __amdgpu_buffer_rsrc_t rsrc;
     __device__ __forceinline__ LlBuf(ll_word *base, int64_t words)
         : rsrc(__builtin_amdgcn_make_buffer_rsrc(base, (short)0, (int)(words * 8), 0x00020000))
     {
     }
+    // a value's words as they stand, and the value they hold (false: not of
+    // this epoch)
+    template <typename T>
+    __device__ __forceinline__ Raw<T> read(int64_t w) const
+    {
+        if constexpr (sizeof(T) == 8) return __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)w * 8, 0, kLlAux);
+        else return __builtin_amdgcn_raw_buffer_load_b64(rsrc, (int)w * 8, 0, kLlAux);
+    }
+    static __device__ __forceinline__ bool value(const ll_u4 &q, double &v, unsigned epoch)
+    {
+        v = __builtin_bit_cast(double, (uint64_t)q[0] | ((uint64_t)q[2] << 32));
+        return (q[1] == epoch) & (q[3] == epoch);
+    }
+    static __device__ __forceinline__ bool value(const ll_u2 &q, float &v, unsigned epoch)
+    {
+        v = __builtin_bit_cast(float, q[0]);
+        return q[1] == epoch;
+    }
 };
 
 // word index w of the buffer (of a double's first word)
-__device__ __forceinline__ void ll_put(const LlBuf &b, int w, double v, unsigned epoch)
+__device__ __forceinline__ void ll_put(const LlBuf &b, int64_t w, double v, unsigned epoch)
 {
     const uint64_t bits = __builtin_bit_cast(uint64_t, v);
     const ll_u4 q = {(unsigned)bits, epoch, (unsigned)(bits >> 32), epoch};
-    __builtin_amdgcn_raw_buffer_store_b128(q, b.rsrc, w * 8, 0, kLlAux);
+    __builtin_amdgcn_raw_buffer_store_b128(q, b.rsrc, (int)w * 8, 0, kLlAux);
 }
-__device__ __forceinline__ void ll_put(const LlBuf &b, int w, float v, unsigned epoch)
+__device__ __forceinline__ void ll_put(const LlBuf &b, int64_t w, float v, unsigned epoch)
 {
     const ll_u2 q = {__builtin_bit_cast(unsigned, v), epoch};
-    __builtin_amdgcn_raw_buffer_store_b64(q, b.rsrc, w * 8, 0, kLlAux);
+    __builtin_amdgcn_raw_buffer_store_b64(q, b.rsrc, (int)w * 8, 0, kLlAux);
 }
-__device__ __forceinline__ bool ll_get(const LlBuf &b, int w, double &v, unsigned epoch)
+// The same words past a buffer's 2 GiB: 8-byte atomics on 64-bit addresses.
+struct LlPtr {
+    ll_word *p;
+    __device__ __forceinline__ LlPtr(ll_word *base, int64_t) : p(base) {}
+    __device__ __forceinline__ void store(int64_t w, unsigned v, unsigned epoch) const
+    {
+        __hip_atomic_store(p + w, (ll_word)epoch << 32 | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    template <typename T>
+    struct Raw {
+        ll_word q[ll_words<T>()];
+    };
+    template <typename T>
+    __device__ __forceinline__ Raw<T> read(int64_t w) const
+    {
+        Raw<T> r;
+#pragma unroll
+        for (int i = 0; i < ll_words<T>(); i++)
+            r.q[i] = __hip_atomic_load(p + w + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return r;
+    }
+    static __device__ __forceinline__ bool value(const Raw<double> &r, double &v, unsigned epoch)
+    {
+        v = __builtin_bit_cast(double, (r.q[0] & 0xffffffffull) | (r.q[1] << 32));
+        return ((unsigned)(r.q[0] >> 32) == epoch) & ((unsigned)(r.q[1] >> 32) == epoch);
+    }
+    static __device__ __forceinline__ bool value(const Raw<float> &r, float &v, unsigned epoch)
+    {
+        v = __builtin_bit_cast(float, (unsigned)r.q[0]);
+        return (unsigned)(r.q[0] >> 32) == epoch;
+    }
+};
+__device__ __forceinline__ void ll_put(const LlPtr &b, int64_t w, double v, unsigned epoch)
 {
-    const ll_u4 q = __builtin_amdgcn_raw_buffer_load_b128(b.rsrc, w * 8, 0, kLlAux);
-    v = __builtin_bit_cast(double, (uint64_t)q[0] | ((uint64_t)q[2] << 32));
-    return (q[1] == epoch) & (q[3] == epoch);
+    const uint64_t bits = __builtin_bit_cast(uint64_t, v);
+    b.store(w, (unsigned)bits, epoch);
+    b.store(w + 1, (unsigned)(bits >> 32), epoch);
 }
-__device__ __forceinline__ bool ll_get(const LlBuf &b, int w, float &v, unsigned epoch)
+__device__ __forceinline__ void ll_put(const LlPtr &b, int64_t w, float v, unsigned epoch)
 {
-    const ll_u2 q = __builtin_amdgcn_raw_buffer_load_b64(b.rsrc, w * 8, 0, kLlAux);
-    v = __builtin_bit_cast(float, q[0]);
-    return q[1] == epoch;
+    b.store(w, __builtin_bit_cast(unsigned, v), epoch);
+}
+template <class Words, typename T>
+__device__ __forceinline__ bool ll_get(const Words &b, int64_t w, T &v, unsigned epoch)
+{
+    return Words::value(b.template read<T>(w), v, epoch);
 }
 
 // Sum over each 16-lane row, in every lane, by DPP (no LDS round trip).
@@ -213,9 +268,12 @@ __device__ __forceinline__ bool res_wait(T (&v)[NV], ResTeam &t, ResShared<T> &s
         if (q < t.k) {
             const int from = (int)(ph * t.k + q) * res_slot_words<T>();
             const bool ok = res_poll(t, [&]() {
+                LlBuf::Raw<T> raw[NV];
+#pragma unroll
+                for (int i = 0; i < NV; i++) raw[i] = t.slot.template read<T>(from + i * ll_words<T>());
                 bool all = true;
 #pragma unroll
-                for (int i = 0; i < NV; i++) all &= ll_get(t.slot, from + i * ll_words<T>(), s[i], t.epoch);
+                for (int i = 0; i < NV; i++) all &= LlBuf::value(raw[i], s[i], t.epoch);
                 return all;
             });
             if (!ok) sh.bad = 1;
@@ -328,19 +386,25 @@ __device__ __forceinline__ bool res_cg(const ResRows &R, const T *val, const T *
         if (row < R.m1) publish(row, z[u]);
     }
     bool ok = true;
-    // N halo values from element h0 on: every word is loaded before the first
-    // is looked at; lanes past the halo's end poll its last element
+    // N halo values from element h0 on: every word is on its way before the
+    // first is looked at (checked one by one, the loads took turns: 64^3 15.6
+    // instead of 13.2 us per iteration); lanes past the halo's end poll its
+    // last element
     auto fetch = [&](auto &zh, int h0) {
         constexpr int N = sizeof(zh) / sizeof(T);
         if (h0 >= nhalo) return;
         const bool got = res_poll(t, [&]() {
-            bool all = true;
+            LlBuf::Raw<T> raw[N];
 #pragma unroll
             for (int q = 0; q < N; q++)
                 if (h0 + q * NT < nhalo) {
                     const int h = min(h0 + q * NT + tid, nhalo - 1);
-                    all &= ll_get(zw, halo_row(h) * ll_words<T>(), zh[q], zepoch);
+                    raw[q] = zw.template read<T>(halo_row(h) * ll_words<T>());
                 }
+            bool all = true;
+#pragma unroll
+            for (int q = 0; q < N; q++)
+                if (h0 + q * NT < nhalo) all &= LlBuf::value(raw[q], zh[q], zepoch);
             return all;
         });
         if (!got) sh.bad = 1;

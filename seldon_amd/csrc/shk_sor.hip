@@ -1,4 +1,4 @@
-// shk_sor.hip -- Seldon's SOR / SSOR sweeps on the device, level-scheduled.
+// shk_sor.hip -- Seldon's SOR / SSOR sweeps on the device.
 //
 // SOR(A, X, B, omega, iter, type_ssor) runs iter forward sweeps when
 // type_ssor % 2 == 0, then iter backward sweeps when type_ssor % 3 == 0.
@@ -10,12 +10,28 @@
 //   X(j) = (1 - omega) * X(j) + omega * temp / ajj
 // with the rows in increasing order (forward) or decreasing (backward).  A
 // row reads the new X of the rows swept before it and the old X of the
-// others.  Rows are grouped in levels such that a row comes after every
-// earlier-swept row whose X it reads and before every later-swept row that
-// reads its X (both directions of each stored entry count); rows of one level
-// then neither read nor write each other's X, so a level runs in parallel,
-// one thread per row, and every row sees exactly the operands of the
-// sequential sweep: the results are bitwise Seldon's.
+// others.
+//
+// A sweep is one kernel.  The new values go to words that say which sweep
+// wrote them ({sweep number, 32 bits of the value}, as in shk_resident.hpp);
+// a row polls the words of the rows it needs, forms its own value and writes
+// its word.  X itself, which holds every old value, is only read during the
+// sweep and takes the new values after it, so a row never has to wait for the
+// readers of its old value.  Rows are taken in the order of the dependence
+// levels (a row's level is one more than the highest it reads a new value
+// from), 64 rows of one level at most at a time, by wavefronts that draw the
+// next piece from a counter: the lowest unfinished piece is always being
+// worked on and needs only finished ones, so every wait ends whatever part of
+// the GPU the kernel gets.  Every row sees exactly the operands of the
+// sequential sweep, in its order: the results are bitwise Seldon's.
+//
+// Bound by the chain of levels: a word's way from one work-group to another
+// and the division behind it, 1.0 us per level on 2-D grids, 1.7 on the 128^3
+// one.  (A launch per level cost 9 us, one work-group stepping through small
+// levels 2.5.)  Symmetric sweep, FP64, before -> after: 128^3
+// convection-diffusion (2 x 382 levels) 5.81 -> 1.36 ms, 64^3 2.51 -> 0.54,
+// 16^3 0.194 -> 0.135; 256^2 Laplacian RowSparse 2.56 -> 1.09, RowSymSparse
+// 2.02 -> 1.04; 50K-row power-law matrix 85.6 -> 43.7.
 //
 // RowSymSparse (:179-300, upper triangle stored) splits each sweep in two
 // passes.  Forward: Z(j) = (1-w)/w ajj X(j) + (B(j) - sum_{p>j} a_jp X(p))
@@ -32,20 +48,16 @@
 #include <string>
 #include <vector>
 
-#include "shk_kernels.hpp"
+#include "shk_resident.hpp"
 
 namespace shk {
 
-// Consecutive levels of at most kRunRows rows are run by one work-group of
-// kRunThreads threads, level after level with a barrier between them (the
-// barrier orders each level's X stores before the next level's loads within
-// the work-group); larger levels get a launch each.
-constexpr int kRunThreads = 1024;
-constexpr int kRunRows = 1024;
+constexpr int kSorBatch = 8;              // entries of a row in flight at a time
+constexpr long long kSorWaitSeconds = 4;  // a wait before the sweep is left to one work-group
 
-struct LevelSeg {
-    int l0, l1;  // levels [l0, l1)
-    bool run;    // one work-group steps through them; else one level, one launch
+// device counters of a plan's sweeps
+struct SorState {
+    unsigned ticket, stall, sweep, rescue_ticket;
 };
 
 struct SorPlan {
@@ -54,44 +66,67 @@ struct SorPlan {
     void *val = nullptr, *diag = nullptr;
     int *tptr = nullptr, *tind = nullptr;  // RowSymSparse: strict upper entries by column
     void *tval = nullptr, *z = nullptr;    // (rows increasing), and the half-step vector
-    int *rows[2] = {nullptr, nullptr};     // forward, backward: rows grouped by level
-    int *doff[2] = {nullptr, nullptr};     // level offsets into rows[d] (device)
-    std::vector<int> off[2];               // the same (host)
-    std::vector<LevelSeg> segs[2];         // launches of direction d
+    int *rows[2] = {nullptr, nullptr};     // forward, backward: rows by level
+    int *pos[2] = {nullptr, nullptr};      // where each row stands in rows[d]
+    int2 *piece[2] = {nullptr, nullptr};   // {first of rows[d], count}: up to 64 rows of one level
+    int npiece[2] = {0, 0};
+    // the new value of each row, in the order of rows[d]: a piece writes
+    // consecutive words, and the rows it waits for stand close together in the
+    // levels before it (by row number a 64-row piece of a 3-D grid polls up to
+    // 192 cache lines: 2.18 instead of 1.36 ms at 128^3)
+    ll_word *word = nullptr;
+    SorState *state = nullptr;
+    long long limit = 0;
 };
 
 // ---- row operations ------------------------------------------------------
+// Each names its rows' entries (ptr, ind, val), says whether entry column c
+// is read new, old or not at all, loads what else a row needs (before it
+// waits), and forms the row's value from the sum of its entries in stored
+// order.
+enum SorRead { kSorOld, kSorNew, kSorNone };
+
 // general storages: one row of the sweep
 template <typename T, typename W>
 struct SorRow {
     const int *ptr, *ind;
     const T *val, *diag, *B;
-    T *X;
+    const T *X;
     W omega;
-    __device__ __forceinline__ void operator()(int j) const
+    bool forward;
+    static constexpr bool kSubtract = false;
+    __device__ __forceinline__ SorRead read(int j, int c) const
     {
-        T temp = (T)0;
-        for (int k = ptr[j]; k < ptr[j + 1]; k++) temp += val[k] * X[ind[k]];
-        const T ajj = diag[j];
-        const T xj = X[j];
-        temp = B[j] - temp + ajj * xj;
-        X[j] = (T)(((W)1 - omega) * (W)xj + omega * (W)temp / (W)ajj);
+        return (forward ? c < j : c > j) ? kSorNew : kSorOld;
+    }
+    struct Row {
+        T ajj, xj, b;
+    };
+    __device__ __forceinline__ Row load(int j) const { return Row{diag[j], X[j], B[j]}; }
+    __device__ __forceinline__ T start(const Row &) const { return (T)0; }
+    __device__ __forceinline__ T value(const Row &r, T temp) const
+    {
+        temp = r.b - temp + r.ajj * r.xj;
+        return (T)(((W)1 - omega) * (W)r.xj + omega * (W)temp / (W)r.ajj);
     }
 };
 
 // RowSymSparse forward solve: X(p) = (Z(p) - sum_j a_jp X(j)) * (w / ajj)
 template <typename T, typename W>
 struct SymForward {
-    const int *tptr, *tind;
-    const T *tval, *diag, *Z;
-    T *X;
+    const int *ptr, *ind;  // strict upper entries by column
+    const T *val, *diag, *Z;
+    const T *X;
     W omega;
-    __device__ __forceinline__ void operator()(int p) const
-    {
-        T x = Z[p];
-        for (int k = tptr[p]; k < tptr[p + 1]; k++) x -= tval[k] * X[tind[k]];
-        X[p] = (T)((W)x * (omega / (W)diag[p]));
-    }
+    static constexpr bool kSubtract = true;
+    __device__ __forceinline__ SorRead read(int, int) const { return kSorNew; }
+    struct Row {
+        T z;
+        W f;
+    };
+    __device__ __forceinline__ Row load(int p) const { return Row{Z[p], omega / (W)diag[p]}; }
+    __device__ __forceinline__ T start(const Row &r) const { return r.z; }
+    __device__ __forceinline__ T value(const Row &r, T x) const { return (T)((W)x * r.f); }
 };
 
 // RowSymSparse backward solve: X(j) = (Z(j) - sum_{p != j} a_jp X(p)) w / ajj
@@ -99,35 +134,128 @@ template <typename T, typename W>
 struct SymBackward {
     const int *ptr, *ind;
     const T *val, *diag, *Z;
-    T *X;
+    const T *X;
     W omega;
-    __device__ __forceinline__ void operator()(int j) const
+    static constexpr bool kSubtract = false;
+    __device__ __forceinline__ SorRead read(int j, int c) const { return c == j ? kSorNone : kSorNew; }
+    struct Row {
+        T z, ajj;
+    };
+    __device__ __forceinline__ Row load(int j) const { return Row{Z[j], diag[j]}; }
+    __device__ __forceinline__ T start(const Row &) const { return (T)0; }
+    __device__ __forceinline__ T value(const Row &r, T temp) const
     {
-        T temp = (T)0;
-        for (int k = ptr[j]; k < ptr[j + 1]; k++)
-            if (ind[k] != j) temp += val[k] * X[ind[k]];
-        X[j] = (T)((W)(Z[j] - temp) * omega / (W)diag[j]);
+        return (T)((W)(r.z - temp) * omega / (W)r.ajj);
     }
 };
 
-// one level, one thread per row
-template <class Op>
-__global__ __launch_bounds__(kBlock) void k_level(const int *__restrict__ rows, int count, Op op)
+// the next sweep: its number, and its counters to their start
+__global__ void k_sor_begin(SorState *st)
 {
-    const int t = blockIdx.x * kBlock + threadIdx.x;
-    if (t < count) op(rows[t]);
+    st->ticket = 0u;
+    st->rescue_ticket = 0u;
+    st->stall = 0u;
+    st->sweep++;
 }
 
-// levels [l0, l1) in one work-group
-template <class Op>
-__global__ __launch_bounds__(kRunThreads) void k_level_run(const int *__restrict__ rows, const int *__restrict__ off,
-                                                           int l0, int l1, Op op)
+// One sweep: wavefronts draw pieces until none is left.  `rescue`: only when
+// the sweep before it gave up waiting (a GPU shared with long-running work),
+// by one work-group, whose wavefronts are all there, without a limit.
+template <typename T, class Words, class Op>
+__global__ __launch_bounds__(kBlock) void k_sor_sweep(int m, const int *__restrict__ rows, const int *__restrict__ pos,
+                                                      const int2 *__restrict__ piece, int npiece, Op op,
+                                                      ll_word *words, SorState *st, long long limit, bool rescue)
 {
-    for (int l = l0; l < l1; l++) {
-        const int end = off[l + 1];
-        for (int t = off[l] + (int)threadIdx.x; t < end; t += kRunThreads) op(rows[t]);
-        __syncthreads();
+    if (rescue && !st->stall) return;
+    const unsigned sweep = st->sweep;
+    unsigned *ticket = rescue ? &st->rescue_ticket : &st->ticket;
+    const Words w(words, (int64_t)m * ll_words<T>());
+    const int lane = threadIdx.x & (kWave - 1);
+    auto draw = [&]() {
+        int q = 0;
+        if (lane == 0) q = (int)atomicAdd(ticket, 1u);
+        return __builtin_amdgcn_readfirstlane(q);
+    };
+    for (int q = draw(); q < npiece;) {
+        const int next = draw();  // on its way while this piece waits
+        const int2 pc = piece[q];
+        const bool in = lane < pc.y;
+        const int j = rows[pc.x + (in ? lane : 0)];
+        const int p0 = op.ptr[j], len = in ? op.ptr[j + 1] - p0 : 0;
+        int most = len;
+        for (int o = 32; o > 0; o >>= 1) most = max(most, __shfl_xor(most, o, kWave));
+        const typename Op::Row row = op.load(j);
+        T acc = op.start(row);
+        for (int k0 = 0; k0 < most; k0 += kSorBatch) {
+            int c[kSorBatch], how[kSorBatch];
+            T v[kSorBatch], x[kSorBatch];
+#pragma unroll
+            for (int u = 0; u < kSorBatch; u++) {
+                const int k = k0 + u < len ? p0 + k0 + u : 0;
+                c[u] = op.ind[k];
+                v[u] = op.val[k];
+            }
+            unsigned need = 0u;  // entries some lane reads new
+#pragma unroll
+            for (int u = 0; u < kSorBatch; u++) {
+                how[u] = k0 + u < len ? (int)op.read(j, c[u]) : (int)kSorNone;
+                if (__builtin_amdgcn_ballot_w64(how[u] == kSorNew)) need |= 1u << u;
+                x[u] = how[u] == kSorOld ? op.X[c[u]] : (T)0;
+                c[u] = how[u] == kSorNew ? pos[c[u]] : pc.x;  // the word to poll
+            }
+            if (need) {
+                const long long t0 = wall_clock64();
+                for (int n = 1;; n++) {
+                    asm volatile("" ::: "memory");  // the words are read again
+                    // every word is on its way before the first is looked at
+                    typename Words::template Raw<T> raw[kSorBatch];
+#pragma unroll
+                    for (int u = 0; u < kSorBatch; u++)
+                        if (need >> u & 1u)
+                            raw[u] = w.template read<T>((int64_t)c[u] * ll_words<T>());
+                    bool all = true;
+#pragma unroll
+                    for (int u = 0; u < kSorBatch; u++)
+                        if (need >> u & 1u) {
+                            T y;
+                            const bool got = Words::value(raw[u], y, sweep);
+                            if (how[u] == kSorNew) {
+                                x[u] = y;
+                                all &= got;
+                            }
+                        }
+                    if (!__builtin_amdgcn_ballot_w64(!all)) break;
+                    if (!rescue && (n & 255) == 0) {
+                        const bool late = wall_clock64() - t0 > limit;
+                        if (late) __hip_atomic_store(&st->stall, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        if (late || __hip_atomic_load(&st->stall, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
+                    }
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < kSorBatch; u++)
+                if (how[u] != kSorNone) {
+                    const T t = v[u] * x[u];
+                    acc = Op::kSubtract ? acc - t : acc + t;
+                }
+        }
+        if (in) ll_put(w, (int64_t)(pc.x + lane) * ll_words<T>(), op.value(row, acc), sweep);
+        q = next;
     }
+}
+
+// X from the sweep's words
+template <typename T, class Words>
+__global__ __launch_bounds__(kBlock) void k_sor_out(int m, const int *__restrict__ pos, ll_word *words,
+                                                    T *__restrict__ X, const SorState *st)
+{
+    const Words w(words, (int64_t)m * ll_words<T>());
+    const unsigned sweep = st->sweep;
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= m) return;
+    T v;
+    ll_get(w, (int64_t)pos[i] * ll_words<T>(), v, sweep);
+    X[i] = v;
 }
 
 // ---- RowSymSparse explicit halves ----------------------------------------
@@ -162,15 +290,16 @@ __global__ __launch_bounds__(kBlock) void k_sor_sym_b1(int m, const int *__restr
 }
 
 // ---- plan ----------------------------------------------------------------
-// Levels of one sweep direction (dir 0: rows 0..m-1, dir 1: m-1..0).
+// Rows of one sweep direction (dir 0: rows 0..m-1, dir 1: m-1..0) by level,
+// and the levels cut into pieces of up to 64 rows.
 static void sor_levels(int m, const std::vector<int> &ptr, const std::vector<int> &ind, int dir,
-                       std::vector<int> &rows, std::vector<int> &off)
+                       std::vector<int> &rows, std::vector<int> &pos, std::vector<int2> &piece)
 {
-    std::vector<int> lev(m, 0), minlev(m, 0);
+    std::vector<int> lev(m, 0);
     int nlev = 0;
     for (int q = 0; q < m; q++) {
         const int j = dir == 0 ? q : m - 1 - q;
-        int L = minlev[j];
+        int L = 0;
         for (int k = ptr[j]; k < ptr[j + 1]; k++) {
             const int c = ind[k];
             const bool before = dir == 0 ? c < j : c > j;  // swept before j: read new
@@ -178,37 +307,21 @@ static void sor_levels(int m, const std::vector<int> &ptr, const std::vector<int
         }
         lev[j] = L;
         nlev = std::max(nlev, L + 1);
-        for (int k = ptr[j]; k < ptr[j + 1]; k++) {
-            const int c = ind[k];
-            const bool after = dir == 0 ? c > j : c < j;  // swept after j: read old
-            if (after) minlev[c] = std::max(minlev[c], L + 1);
-        }
     }
-    off.assign((size_t)nlev + 1, 0);
+    std::vector<int> off((size_t)nlev + 1, 0);
     for (int j = 0; j < m; j++) off[(size_t)lev[j] + 1]++;
     for (int l = 0; l < nlev; l++) off[(size_t)l + 1] += off[l];
     std::vector<int> next(off.begin(), off.end() - 1);
     rows.assign(m, 0);
-    for (int j = 0; j < m; j++) rows[next[lev[j]]++] = j;
-}
-
-// Launches of one direction: runs of consecutive small levels, and the
-// larger levels one by one.
-static void level_segments(const std::vector<int> &off, std::vector<LevelSeg> &segs)
-{
-    segs.clear();
-    const int nlev = (int)off.size() - 1;
-    for (int l = 0; l < nlev;) {
-        int e = l;
-        while (e < nlev && off[(size_t)e + 1] - off[e] <= kRunRows) e++;
-        if (e - l >= 2) {
-            segs.push_back({l, e, true});
-            l = e;
-        } else {
-            segs.push_back({l, l + 1, false});
-            l++;
-        }
+    pos.assign(m, 0);
+    for (int j = 0; j < m; j++) {
+        pos[j] = next[lev[j]]++;
+        rows[pos[j]] = j;
     }
+    piece.clear();
+    for (int l = 0; l < nlev; l++)
+        for (int q = off[l]; q < off[(size_t)l + 1]; q += kWave)
+            piece.push_back(make_int2(q, std::min(kWave, off[(size_t)l + 1] - q)));
 }
 
 // Seldon's A(j, j) on RowSparse (matrix_sparse/Matrix_Sparse.cxx:1054-1084):
@@ -254,9 +367,9 @@ static int sor_build(shk_csr A, SorPlan **out)
             if (ind[k] == j) diag[j] += val[k];
         }
     }
-    std::vector<int> rows[2], tptr, tind;
+    std::vector<int> rows[2], pos[2], tptr, tind;
     std::vector<T> tval;
-    std::vector<int> off[2];
+    std::vector<int2> piece[2];
     if (sym) {
         // strict upper entries gathered by column, rows increasing (a stable
         // counting sort of the row-major entries)
@@ -277,25 +390,30 @@ static int sor_build(shk_csr A, SorPlan **out)
                 }
         // the forward solve's row p reads the X(j) of its column entries, the
         // backward solve's row j the X(p) of its row entries
-        sor_levels(m, tptr, tind, 0, rows[0], off[0]);
-        sor_levels(m, ptr, ind, 1, rows[1], off[1]);
+        sor_levels(m, tptr, tind, 0, rows[0], pos[0], piece[0]);
+        sor_levels(m, ptr, ind, 1, rows[1], pos[1], piece[1]);
     } else {
-        for (int d = 0; d < 2; d++) sor_levels(m, ptr, ind, d, rows[d], off[d]);
+        for (int d = 0; d < 2; d++) sor_levels(m, ptr, ind, d, rows[d], pos[d], piece[d]);
     }
     SorPlan *P = new SorPlan;
     P->m = m;
     P->storage = A->storage;
     P->dtype = A->dtype;
-    P->off[0] = std::move(off[0]);
-    P->off[1] = std::move(off[1]);
-    for (int d = 0; d < 2; d++) level_segments(P->off[d], P->segs[d]);
+    for (int d = 0; d < 2; d++) P->npiece[d] = (int)piece[d].size();
     hipStream_t s = A->ctx->stream;
     hipError_t e = put(&P->ptr, ptr, s);
     if (e == hipSuccess) e = put(&P->ind, ind, s);
     if (e == hipSuccess) e = put((T **)&P->val, val, s);
     if (e == hipSuccess) e = put((T **)&P->diag, diag, s);
     for (int d = 0; d < 2 && e == hipSuccess; d++) e = put(&P->rows[d], rows[d], s);
-    for (int d = 0; d < 2 && e == hipSuccess; d++) e = put(&P->doff[d], P->off[d], s);
+    for (int d = 0; d < 2 && e == hipSuccess; d++) e = put(&P->pos[d], pos[d], s);
+    for (int d = 0; d < 2 && e == hipSuccess; d++) e = put(&P->piece[d], piece[d], s);
+    // no word carries a sweep number yet: sweeps count from 1
+    const size_t wb = sizeof(ll_word) * ll_words<T>() * (size_t)std::max(m, 1);
+    if (e == hipSuccess) e = hipMalloc((void **)&P->word, wb);
+    if (e == hipSuccess) e = hipMemsetAsync(P->word, 0, wb, s);
+    if (e == hipSuccess) e = hipMalloc((void **)&P->state, sizeof(SorState));
+    if (e == hipSuccess) e = hipMemsetAsync(P->state, 0, sizeof(SorState), s);
     if (sym) {
         if (e == hipSuccess) e = put(&P->tptr, tptr, s);
         if (e == hipSuccess) e = put(&P->tind, tind, s);
@@ -306,6 +424,11 @@ static int sor_build(shk_csr A, SorPlan **out)
     if (e != hipSuccess) {
         sor_free(P);
         return fail(SHK_ERR_NOMEM, std::string("sor: device memory: ") + hipGetErrorString(e));
+    }
+    const int st = wall_clock_ticks(A->ctx, kSorWaitSeconds, &P->limit);
+    if (st != SHK_OK) {
+        sor_free(P);
+        return st;
     }
     *out = P;
     return SHK_OK;
@@ -324,26 +447,43 @@ void sor_free(SorPlan *P)
     hipFree(P->z);
     hipFree(P->rows[0]);
     hipFree(P->rows[1]);
-    hipFree(P->doff[0]);
-    hipFree(P->doff[1]);
+    hipFree(P->pos[0]);
+    hipFree(P->pos[1]);
+    hipFree(P->piece[0]);
+    hipFree(P->piece[1]);
+    hipFree(P->word);
+    hipFree(P->state);
     delete P;
 }
 
 static inline dim3 grid_for(int count) { return dim3((count + kBlock - 1) / kBlock); }
 
-template <class Op>
-static void run_levels(const SorPlan *P, int d, const Op &op, hipStream_t s)
+// One sweep's triangular part.  Four wavefronts per work-group and one
+// work-group per CU at most: more of them than the levels can use only poll
+// (128^3 with 64 / 128 / 256 / 512 work-groups: 1.78 / 1.40 / 1.36 / 1.45 ms).
+template <typename T, class Words, class Op>
+static void launch_sweep(shk_ctx ctx, const SorPlan *P, int d, const Op &op, T *X)
 {
-    for (const LevelSeg &g : P->segs[d]) {
-        if (g.run) {
-            hipLaunchKernelGGL(k_level_run<Op>, dim3(1), dim3(kRunThreads), 0, s, (const int *)P->rows[d],
-                               (const int *)P->doff[d], g.l0, g.l1, op);
-        } else {
-            const int first = P->off[d][g.l0], count = P->off[d][g.l1] - first;
-            hipLaunchKernelGGL(k_level<Op>, grid_for(count), dim3(kBlock), 0, s, (const int *)P->rows[d] + first,
-                               count, op);
-        }
-    }
+    hipStream_t s = ctx->stream;
+    const int np = P->npiece[d], waves = kBlock / kWave;
+    const dim3 grid(std::max(1, std::min((np + waves - 1) / waves, ctx->num_cus))), blk(kBlock);
+    hipLaunchKernelGGL(k_sor_begin, dim3(1), dim3(1), 0, s, P->state);
+    hipLaunchKernelGGL((k_sor_sweep<T, Words, Op>), grid, blk, 0, s, P->m, (const int *)P->rows[d],
+                       (const int *)P->pos[d], (const int2 *)P->piece[d], np, op, P->word, P->state, P->limit, false);
+    hipLaunchKernelGGL((k_sor_sweep<T, Words, Op>), dim3(1), blk, 0, s, P->m, (const int *)P->rows[d],
+                       (const int *)P->pos[d], (const int2 *)P->piece[d], np, op, P->word, P->state, P->limit, true);
+    hipLaunchKernelGGL((k_sor_out<T, Words>), grid_for(P->m), blk, 0, s, P->m, (const int *)P->pos[d], P->word, X,
+                       (const SorState *)P->state);
+}
+
+// 32-bit buffer offsets reach 2 GiB of words (134M FP64 rows)
+template <typename T, class Op>
+static void run_sweep(shk_ctx ctx, const SorPlan *P, int d, const Op &op, T *X)
+{
+    if ((int64_t)P->m * ll_words<T>() * (int64_t)sizeof(ll_word) < INT32_MAX)
+        launch_sweep<T, LlBuf>(ctx, P, d, op, X);
+    else
+        launch_sweep<T, LlPtr>(ctx, P, d, op, X);
 }
 
 template <typename T, typename W>
@@ -354,15 +494,15 @@ static int sor_run(shk_ctx ctx, const SorPlan *P, T *X, const T *B, W omega, int
     T *Z = (T *)P->z;
     auto sweep = [&](int d) {
         if (P->storage != SHK_ROWSYMSPARSE) {
-            run_levels(P, d, SorRow<T, W>{P->ptr, P->ind, val, diag, B, X, omega}, s);
+            run_sweep<T>(ctx, P, d, SorRow<T, W>{P->ptr, P->ind, val, diag, B, X, omega, d == 0}, X);
         } else if (d == 0) {
             hipLaunchKernelGGL((k_sor_sym_f1<T, W>), grid_for(P->m), dim3(kBlock), 0, s, P->m, P->ptr, P->ind, val,
                                diag, B, (const T *)X, Z, omega);
-            run_levels(P, 0, SymForward<T, W>{P->tptr, P->tind, tval, diag, Z, X, omega}, s);
+            run_sweep<T>(ctx, P, 0, SymForward<T, W>{P->tptr, P->tind, tval, diag, Z, X, omega}, X);
         } else {
             hipLaunchKernelGGL((k_sor_sym_b1<T, W>), grid_for(P->m), dim3(kBlock), 0, s, P->m, P->tptr, P->tind,
                                tval, diag, B, (const T *)X, Z, omega);
-            run_levels(P, 1, SymBackward<T, W>{P->ptr, P->ind, val, diag, Z, X, omega}, s);
+            run_sweep<T>(ctx, P, 1, SymBackward<T, W>{P->ptr, P->ind, val, diag, Z, X, omega}, X);
         }
     };
     if (type_ssor % 2 == 0)

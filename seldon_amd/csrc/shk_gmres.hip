@@ -14,9 +14,10 @@
 //
 // Bound by the sum (3.2 us over 128 work-groups) and, at 2M rows and more, by
 // reading V_k.  Per iteration of GMRES(30) + Jacobi, FP64, a kernel per pass
-// -> this: 24^3 rows 104 -> 38 us, 64^3 119 -> 51, 100^3 170 -> 80, 128^3
-// 335 -> 134; GMRES(50) on the 4M-row power-law matrix 800 -> 455 (its SpMV
-// 290 of them), FP32 390 -> 253.
+// -> this: 24^3 rows 104 -> 38 us, 64^3 119 -> 50, 100^3 170 -> 75, 128^3
+// 335 -> 120; GMRES(50) on the 4M-row power-law matrix 800 -> 440 (its SpMV
+// 290 of them), FP32 390 -> 244.  (A ninth wavefront for the sums alone, V two
+// passes ahead: 47 at 64^3, 124 at 128^3, and 16 vectors no longer fit.)
 #include <algorithm>
 
 #include "shk_resident.hpp"
@@ -96,10 +97,16 @@ __global__ __launch_bounds__(kGoThreads, 2) void k_gm_ortho(GmOrtho<T> a)
         for (int q = 0; q < NV; q++)
 #pragma unroll
             for (int e = 0; e < N; e++) c[0] += cur[q][e] * w[q][e];
+        // many loads hold the post up behind them in the CU's memory pipeline
+        // (16 vectors: 128.7 us per iteration at 128^3 rows, 120.2 with the
+        // post first), few are better on their way while the work-group meets
+        // (2 vectors, 64^3 rows: 50.0 against 52.2)
+        constexpr bool kPostFirst = NV >= 8;
+        if constexpr (kPostFirst) res_post<T, 1, kGoThreads>(c, t, sh);
         __builtin_amdgcn_sched_barrier(0);
         load(a.V + (size_t)min(k + 1, i) * a.ldv, next);  // the last pass reads its own V_i again, unused
         __builtin_amdgcn_sched_barrier(0);
-        res_post<T, 1, kGoThreads>(c, t, sh);
+        if constexpr (!kPostFirst) res_post<T, 1, kGoThreads>(c, t, sh);
         if (!res_wait<T, 1, kGoThreads>(c, t, sh)) return false;
         const double h = (double)c[0];
         if (lead && tid == 0) hc[k] = h;

@@ -1171,13 +1171,6 @@ struct FinGmOuter {  // true residual after the update (Gmres.cxx:173-178)
     __device__ void operator()(const T (&s)[2]) const { gm_outer_check(st, (double)sqrt_t(s[0])); }
 };
 
-template <typename T>
-struct FinGmH {  // H(k, i) = (V_k, w)
-    KState<T> *st;
-    int k, i;
-    __device__ void operator()(const T (&s)[2]) const { st->H[i * (st->gm_m + 1) + k] = (double)s[0]; }
-};
-
 // End of Arnoldi step i (Gmres.cxx:135-162).
 template <typename T>
 struct FinGmStep {

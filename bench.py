@@ -367,9 +367,9 @@ def convdiff_solves(K, wl, np, torch, cpu=True, layout="auto"):
     sb = Ad.spmv_bytes(False)
     out["spmv"] = {"kernel_ms": round(avg.value, 5), "GBs": round(sb / (avg.value * 1e-3) / 1e9, 2),
                    "frac": round(sb / (avg.value * 1e-3) / 1e9 / HBM_PEAK_GBS, 4), "bytes": sb}
-    # one symmetric SOR sweep (forward then backward, omega 1), level-scheduled
+    # one symmetric SOR sweep (forward then backward, omega 1)
     x = torch.zeros_like(bg)
-    K.SOR(Ad, x, bg, 1.0, 1, 0)  # builds the level plan
+    K.SOR(Ad, x, bg, 1.0, 1, 0)  # builds the plan
     torch.cuda.synchronize()
     t0 = time.perf_counter()
     for _ in range(5):

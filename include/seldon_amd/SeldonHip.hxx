@@ -471,7 +471,7 @@ namespace Seldon
 
   // SOR(A, X, B, omega, iter, type_ssor) (matrix_sparse/Relaxation_MatVect.cxx:
   // 41-95 RowSparse, :106-167 ArrayRowSparse, :179-300 RowSymSparse),
-  // level-scheduled on the GPU and
+  // in level order on the GPU and
   // bitwise Seldon's sweeps; with it Seldon's own SorPreconditioner
   // (Precond_Ssor.cxx), which calls Seldon::SOR, runs on the GPU storages.
   template <class T0, class Prop0, class Storage0, class Allocator0, class T1, class Allocator1, class T2,

@@ -190,9 +190,9 @@ int shk_mlt_dot(shk_ctx ctx, shk_csr A, const void *dx, void *dy, double *result
 /* SOR(A, X, B, omega, iter, type_ssor): type_ssor 2 forward sweeps, 3
  * backward, 0 both (all forward sweeps, then all backward ones), bitwise
  * Seldon's (matrix_sparse/Relaxation_MatVect.cxx:41-95 RowSparse, :106-167
- * ArrayRowSparse, :179-300 RowSymSparse).  Rows run level by level (no row
- * of a level reads another's X); the levels are built on the first call and
- * kept with A.  omega_type is the C++ type of Seldon's omega argument:
+ * ArrayRowSparse, :179-300 RowSymSparse).  A sweep is one launch: rows in
+ * level order wait for the values they need; the order is built on the first
+ * call and kept with A.  omega_type is the C++ type of Seldon's omega argument:
  * SHK_F64 with float values makes each relaxation step double, as C++
  * promotion does; SHK_F32 keeps it in float.  Seldon's SorPreconditioner
  * (computation/solver/preconditioner/Precond_Ssor.cxx:24-90) calls SOR with

@@ -2,8 +2,10 @@
 
 ``stack(systems)`` lays the systems out block-diagonally in one CSR;
 ``cg_batched`` runs Seldon's Cg (identity preconditioner) on every system
-in one launch of the library's persistent kernel (work-group per system,
+in one launch of the library's persistent kernel (teams of work-groups,
 device work queue, largest systems first), optionally captured in a hipGraph;
+systems that repeat a few column offsets are held on the chip for the whole
+solve, and "group" and "rows_per_pass" below apply to the others;
 ``cg_batched_ir`` is the FP32-inner / FP64-refinement variant.
 
 The stacked matrices must use the row layout: ``K.Matrix(A, layout="rows")``.

@@ -59,7 +59,7 @@ struct RedSlot {
 }  // namespace shk
 
 namespace shk {
-struct SorPlan;  // level-scheduled SOR sweeps (shk_sor.hip)
+struct SorPlan;  // SOR sweeps in level order (shk_sor.hip)
 void sor_free(SorPlan *P);
 }  // namespace shk
 
@@ -145,8 +145,8 @@ struct shk_csr_s {
     // first use as an ArrayRowSparse matrix whose rows list, for each column
     // c of A, the entries (i, c) in increasing i
     shk_csr_s *trans = nullptr;
-    // SOR / SSOR sweeps: the caller's CSR and the row levels of both sweep
-    // directions, built on first use
+    // SOR / SSOR sweeps: the caller's CSR and the rows in level order for both
+    // sweep directions, built on first use
     shk::SorPlan *sor = nullptr;
 };
 

@@ -192,7 +192,10 @@ int shk_mlt_dot(shk_ctx ctx, shk_csr A, const void *dx, void *dy, double *result
  * Seldon's (matrix_sparse/Relaxation_MatVect.cxx:41-95 RowSparse, :106-167
  * ArrayRowSparse, :179-300 RowSymSparse).  A sweep is one launch: rows in
  * level order wait for the values they need; the order is built on the first
- * call and kept with A.  omega_type is the C++ type of Seldon's omega argument:
+ * call and kept with A.  A call can be captured once the order is there;
+ * replays may overlap direct calls with A and replays of other captures.  Each
+ * stream of a capture takes up to 24 bytes a row of device memory, kept until
+ * A's values change or it is destroyed.  omega_type is the C++ type of Seldon's omega argument:
  * SHK_F64 with float values makes each relaxation step double, as C++
  * promotion does; SHK_F32 keeps it in float.  Seldon's SorPreconditioner
  * (computation/solver/preconditioner/Precond_Ssor.cxx:24-90) calls SOR with

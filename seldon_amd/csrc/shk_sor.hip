@@ -25,6 +25,10 @@
 // the GPU the kernel gets.  Every row sees exactly the operands of the
 // sequential sweep, in its order: the results are bitwise Seldon's.
 //
+// The words and counters of a sweep are of one call at a time (SorWork): a
+// context's direct calls follow each other and share one set, and every
+// capture has its own, since replays may overlap direct calls and each other.
+//
 // Bound by the chain of levels: a word's way from one work-group to another
 // and the division behind it, 1.0 us per level on 2-D grids, 1.7 on the 128^3
 // one.  (A launch per level cost 9 us, one work-group stepping through small
@@ -55,9 +59,24 @@ namespace shk {
 constexpr int kSorBatch = 8;              // entries of a row in flight at a time
 constexpr long long kSorWaitSeconds = 4;  // a wait before the sweep is left to one work-group
 
-// device counters of a plan's sweeps
+constexpr int kSorOwnPolls = 1 << 20;     // looks at a word the wavefront wrote itself, at most
+
+// device counters of the sweeps
 struct SorState {
-    unsigned ticket, stall, sweep, rescue_ticket;
+    unsigned ticket, stall, sweep;
+};
+
+// What a sweep writes besides X, in one allocation.
+struct SorWork {
+    SorState *state = nullptr;
+    // the new value of each row, in the order of rows[d]: a piece writes
+    // consecutive words, and the rows it waits for stand close together in the
+    // levels before it (by row number a 64-row piece of a 3-D grid polls up to
+    // 192 cache lines: 2.18 instead of 1.36 ms at 128^3)
+    ll_word *word = nullptr;
+    void *z = nullptr;                // RowSymSparse: the half-step vector
+    unsigned long long capture = 0;   // the capture it is of (0: direct calls),
+    hipStream_t stream = nullptr;     // on this stream of it
 };
 
 struct SorPlan {
@@ -65,17 +84,12 @@ struct SorPlan {
     int *ptr = nullptr, *ind = nullptr;  // the stored rows
     void *val = nullptr, *diag = nullptr;
     int *tptr = nullptr, *tind = nullptr;  // RowSymSparse: strict upper entries by column
-    void *tval = nullptr, *z = nullptr;    // (rows increasing), and the half-step vector
+    void *tval = nullptr;                  // (rows increasing)
     int *rows[2] = {nullptr, nullptr};     // forward, backward: rows by level
     int *pos[2] = {nullptr, nullptr};      // where each row stands in rows[d]
     int2 *piece[2] = {nullptr, nullptr};   // {first of rows[d], count}: up to 64 rows of one level
     int npiece[2] = {0, 0};
-    // the new value of each row, in the order of rows[d]: a piece writes
-    // consecutive words, and the rows it waits for stand close together in the
-    // levels before it (by row number a 64-row piece of a 3-D grid polls up to
-    // 192 cache lines: 2.18 instead of 1.36 ms at 128^3)
-    ll_word *word = nullptr;
-    SorState *state = nullptr;
+    std::vector<SorWork> work;             // [0]: direct calls
     long long limit = 0;
 };
 
@@ -149,18 +163,26 @@ struct SymBackward {
     }
 };
 
+// no word carries a sweep number yet: sweeps count from 1
+__global__ __launch_bounds__(kBlock) void k_sor_clear(int64_t n, ll_word *words, SorState *st)
+{
+    const int64_t i0 = blockIdx.x * (int64_t)kBlock + threadIdx.x;
+    if (i0 == 0) *st = SorState{0u, 0u, 0u};
+    for (int64_t i = i0; i < n; i += (int64_t)gridDim.x * kBlock) words[i] = 0;
+}
+
 // the next sweep: its number, and its counters to their start
 __global__ void k_sor_begin(SorState *st)
 {
     st->ticket = 0u;
-    st->rescue_ticket = 0u;
     st->stall = 0u;
     st->sweep++;
 }
 
 // One sweep: wavefronts draw pieces until none is left.  `rescue`: only when
 // the sweep before it gave up waiting (a GPU shared with long-running work),
-// by one work-group, whose wavefronts are all there, without a limit.
+// by a single wavefront, which takes the pieces in order: every word it needs
+// is one it has written itself, so it waits for nobody.
 template <typename T, class Words, class Op>
 __global__ __launch_bounds__(kBlock) void k_sor_sweep(int m, const int *__restrict__ rows, const int *__restrict__ pos,
                                                       const int2 *__restrict__ piece, int npiece, Op op,
@@ -168,16 +190,16 @@ __global__ __launch_bounds__(kBlock) void k_sor_sweep(int m, const int *__restri
 {
     if (rescue && !st->stall) return;
     const unsigned sweep = st->sweep;
-    unsigned *ticket = rescue ? &st->rescue_ticket : &st->ticket;
     const Words w(words, (int64_t)m * ll_words<T>());
     const int lane = threadIdx.x & (kWave - 1);
-    auto draw = [&]() {
+    auto draw = [&](int after) {
+        if (rescue) return after + 1;
         int q = 0;
-        if (lane == 0) q = (int)atomicAdd(ticket, 1u);
+        if (lane == 0) q = (int)atomicAdd(&st->ticket, 1u);
         return __builtin_amdgcn_readfirstlane(q);
     };
-    for (int q = draw(); q < npiece;) {
-        const int next = draw();  // on its way while this piece waits
+    for (int q = draw(-1); q < npiece;) {
+        const int next = draw(q);  // on its way while this piece waits
         const int2 pc = piece[q];
         const bool in = lane < pc.y;
         const int j = rows[pc.x + (in ? lane : 0)];
@@ -225,7 +247,9 @@ __global__ __launch_bounds__(kBlock) void k_sor_sweep(int m, const int *__restri
                             }
                         }
                     if (!__builtin_amdgcn_ballot_w64(!all)) break;
-                    if (!rescue && (n & 255) == 0) {
+                    if (rescue) {
+                        if (n == kSorOwnPolls) break;
+                    } else if ((n & 255) == 0) {
                         const bool late = wall_clock64() - t0 > limit;
                         if (late) __hip_atomic_store(&st->stall, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                         if (late || __hip_atomic_load(&st->stall, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
@@ -346,6 +370,63 @@ static hipError_t put(V **dst, const std::vector<V> &src, hipStream_t s)
     return e;
 }
 
+// state, words and (RowSymSparse) the half-step vector of P's sweeps
+template <typename T>
+static hipError_t sor_work_alloc(const SorPlan *P, SorWork &w)
+{
+    auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
+    const size_t sb = al(sizeof(SorState)), wb = al(sizeof(ll_word) * ll_words<T>() * (size_t)P->m),
+                 zb = P->storage == SHK_ROWSYMSPARSE ? sizeof(T) * (size_t)P->m : 0;
+    char *p = nullptr;
+    const hipError_t e = hipMalloc((void **)&p, sb + wb + zb);
+    if (e != hipSuccess) return e;
+    w.state = (SorState *)p;
+    w.word = (ll_word *)(p + sb);
+    w.z = p + sb + wb;
+    return hipSuccess;
+}
+
+template <typename T>
+static void sor_clear(const SorPlan *P, const SorWork &w, hipStream_t s)
+{
+    const int64_t n = (int64_t)P->m * ll_words<T>();
+    hipLaunchKernelGGL(k_sor_clear, dim3(red_blocks(n)), dim3(kBlock), 0, s, n, w.word, w.state);
+}
+
+// What a call on the context's stream may write.  Direct calls follow each
+// other: a context has one stream, and is synchronised where that changes.
+// Captured calls of one capture and stream follow each other too; their words
+// start from nothing on every replay.
+template <typename T>
+static int sor_work(shk_ctx ctx, SorPlan *P, SorWork &out)
+{
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    if (hipStreamGetCaptureInfo(ctx->stream, &cs, &id) != hipSuccess) (void)hipGetLastError();
+    if (cs != hipStreamCaptureStatusActive) {
+        out = P->work[0];
+        return SHK_OK;
+    }
+    for (size_t i = 1; i < P->work.size(); i++)
+        if (P->work[i].capture == id && P->work[i].stream == ctx->stream) {
+            out = P->work[i];
+            return SHK_OK;
+        }
+    SorWork w;
+    w.capture = id;
+    w.stream = ctx->stream;
+    // an allocation is no part of the capture
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    SHK_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+    const hipError_t e = sor_work_alloc<T>(P, w);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess) return fail(SHK_ERR_NOMEM, std::string("sor: device memory: ") + hipGetErrorString(e));
+    sor_clear<T>(P, w, ctx->stream);
+    P->work.push_back(w);
+    out = w;
+    return SHK_OK;
+}
+
 template <typename T>
 static int sor_build(shk_csr A, SorPlan **out)
 {
@@ -408,17 +489,13 @@ static int sor_build(shk_csr A, SorPlan **out)
     for (int d = 0; d < 2 && e == hipSuccess; d++) e = put(&P->rows[d], rows[d], s);
     for (int d = 0; d < 2 && e == hipSuccess; d++) e = put(&P->pos[d], pos[d], s);
     for (int d = 0; d < 2 && e == hipSuccess; d++) e = put(&P->piece[d], piece[d], s);
-    // no word carries a sweep number yet: sweeps count from 1
-    const size_t wb = sizeof(ll_word) * ll_words<T>() * (size_t)std::max(m, 1);
-    if (e == hipSuccess) e = hipMalloc((void **)&P->word, wb);
-    if (e == hipSuccess) e = hipMemsetAsync(P->word, 0, wb, s);
-    if (e == hipSuccess) e = hipMalloc((void **)&P->state, sizeof(SorState));
-    if (e == hipSuccess) e = hipMemsetAsync(P->state, 0, sizeof(SorState), s);
+    P->work.emplace_back();
+    if (e == hipSuccess) e = sor_work_alloc<T>(P, P->work[0]);
+    if (e == hipSuccess) sor_clear<T>(P, P->work[0], s);
     if (sym) {
         if (e == hipSuccess) e = put(&P->tptr, tptr, s);
         if (e == hipSuccess) e = put(&P->tind, tind, s);
         if (e == hipSuccess) e = put((T **)&P->tval, tval, s);
-        if (e == hipSuccess) e = hipMalloc(&P->z, sizeof(T) * std::max(m, 1));
     }
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) {
@@ -444,15 +521,13 @@ void sor_free(SorPlan *P)
     hipFree(P->tptr);
     hipFree(P->tind);
     hipFree(P->tval);
-    hipFree(P->z);
     hipFree(P->rows[0]);
     hipFree(P->rows[1]);
     hipFree(P->pos[0]);
     hipFree(P->pos[1]);
     hipFree(P->piece[0]);
     hipFree(P->piece[1]);
-    hipFree(P->word);
-    hipFree(P->state);
+    for (const SorWork &w : P->work) hipFree(w.state);
     delete P;
 }
 
@@ -462,47 +537,49 @@ static inline dim3 grid_for(int count) { return dim3((count + kBlock - 1) / kBlo
 // work-group per CU at most: more of them than the levels can use only poll
 // (128^3 with 64 / 128 / 256 / 512 work-groups: 1.78 / 1.40 / 1.36 / 1.45 ms).
 template <typename T, class Words, class Op>
-static void launch_sweep(shk_ctx ctx, const SorPlan *P, int d, const Op &op, T *X)
+static void launch_sweep(shk_ctx ctx, const SorPlan *P, const SorWork &w, int d, const Op &op, T *X)
 {
     hipStream_t s = ctx->stream;
     const int np = P->npiece[d], waves = kBlock / kWave;
     const dim3 grid(std::max(1, std::min((np + waves - 1) / waves, ctx->num_cus))), blk(kBlock);
-    hipLaunchKernelGGL(k_sor_begin, dim3(1), dim3(1), 0, s, P->state);
+    hipLaunchKernelGGL(k_sor_begin, dim3(1), dim3(1), 0, s, w.state);
     hipLaunchKernelGGL((k_sor_sweep<T, Words, Op>), grid, blk, 0, s, P->m, (const int *)P->rows[d],
-                       (const int *)P->pos[d], (const int2 *)P->piece[d], np, op, P->word, P->state, P->limit, false);
-    hipLaunchKernelGGL((k_sor_sweep<T, Words, Op>), dim3(1), blk, 0, s, P->m, (const int *)P->rows[d],
-                       (const int *)P->pos[d], (const int2 *)P->piece[d], np, op, P->word, P->state, P->limit, true);
-    hipLaunchKernelGGL((k_sor_out<T, Words>), grid_for(P->m), blk, 0, s, P->m, (const int *)P->pos[d], P->word, X,
-                       (const SorState *)P->state);
+                       (const int *)P->pos[d], (const int2 *)P->piece[d], np, op, w.word, w.state, P->limit, false);
+    hipLaunchKernelGGL((k_sor_sweep<T, Words, Op>), dim3(1), dim3(kWave), 0, s, P->m, (const int *)P->rows[d],
+                       (const int *)P->pos[d], (const int2 *)P->piece[d], np, op, w.word, w.state, P->limit, true);
+    hipLaunchKernelGGL((k_sor_out<T, Words>), grid_for(P->m), blk, 0, s, P->m, (const int *)P->pos[d], w.word, X,
+                       (const SorState *)w.state);
 }
 
 // 32-bit buffer offsets reach 2 GiB of words (134M FP64 rows)
 template <typename T, class Op>
-static void run_sweep(shk_ctx ctx, const SorPlan *P, int d, const Op &op, T *X)
+static void run_sweep(shk_ctx ctx, const SorPlan *P, const SorWork &w, int d, const Op &op, T *X)
 {
     if ((int64_t)P->m * ll_words<T>() * (int64_t)sizeof(ll_word) < INT32_MAX)
-        launch_sweep<T, LlBuf>(ctx, P, d, op, X);
+        launch_sweep<T, LlBuf>(ctx, P, w, d, op, X);
     else
-        launch_sweep<T, LlPtr>(ctx, P, d, op, X);
+        launch_sweep<T, LlPtr>(ctx, P, w, d, op, X);
 }
 
 template <typename T, typename W>
-static int sor_run(shk_ctx ctx, const SorPlan *P, T *X, const T *B, W omega, int iter, int type_ssor)
+static int sor_run(shk_ctx ctx, SorPlan *P, T *X, const T *B, W omega, int iter, int type_ssor)
 {
     hipStream_t s = ctx->stream;
     const T *val = (const T *)P->val, *diag = (const T *)P->diag, *tval = (const T *)P->tval;
-    T *Z = (T *)P->z;
+    SorWork w;
+    SHK_TRY(sor_work<T>(ctx, P, w));
+    T *Z = (T *)w.z;
     auto sweep = [&](int d) {
         if (P->storage != SHK_ROWSYMSPARSE) {
-            run_sweep<T>(ctx, P, d, SorRow<T, W>{P->ptr, P->ind, val, diag, B, X, omega, d == 0}, X);
+            run_sweep<T>(ctx, P, w, d, SorRow<T, W>{P->ptr, P->ind, val, diag, B, X, omega, d == 0}, X);
         } else if (d == 0) {
             hipLaunchKernelGGL((k_sor_sym_f1<T, W>), grid_for(P->m), dim3(kBlock), 0, s, P->m, P->ptr, P->ind, val,
                                diag, B, (const T *)X, Z, omega);
-            run_sweep<T>(ctx, P, 0, SymForward<T, W>{P->tptr, P->tind, tval, diag, Z, X, omega}, X);
+            run_sweep<T>(ctx, P, w, 0, SymForward<T, W>{P->tptr, P->tind, tval, diag, Z, X, omega}, X);
         } else {
             hipLaunchKernelGGL((k_sor_sym_b1<T, W>), grid_for(P->m), dim3(kBlock), 0, s, P->m, P->tptr, P->tind,
                                tval, diag, B, (const T *)X, Z, omega);
-            run_sweep<T>(ctx, P, 1, SymBackward<T, W>{P->ptr, P->ind, val, diag, Z, X, omega}, X);
+            run_sweep<T>(ctx, P, w, 1, SymBackward<T, W>{P->ptr, P->ind, val, diag, Z, X, omega}, X);
         }
     };
     if (type_ssor % 2 == 0)
@@ -536,7 +613,7 @@ int shk_sor(shk_ctx ctx, shk_csr A, void *dx, const void *db, double omega, shk_
         SHK_TRY(A->dtype == SHK_F64 ? sor_build<double>(A, &P) : sor_build<float>(A, &P));
         A->sor = P;
     }
-    const SorPlan *P = A->sor;
+    SorPlan *P = A->sor;
     if (A->dtype == SHK_F64)
         return sor_run<double, double>(ctx, P, (double *)dx, (const double *)db, omega, iter, type_ssor);
     if (omega_type == SHK_F64)

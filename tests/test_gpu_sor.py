@@ -98,3 +98,56 @@ def test_sor_in_a_graph(gpu):
     finally:
         torch.cuda.synchronize()
         ctx.bind_stream()
+
+
+@pytest.mark.parametrize("st", ["row", "sym"])
+def test_overlapping_sweeps_of_one_matrix(gpu, st):
+    """Two captured sweeps of one matrix replayed side by side on two streams,
+    then one of them beside a direct call on a third: each X is its own
+    sequence of sweeps, whichever way they overlap."""
+    from oracle import oracle as orc
+    from seldon_amd import krylov as K
+    A = wl.diffusion3d(40, wl.normal(40 ** 3, 4, 0.0, 0.5))
+    M = wl.upper(A) if st == "sym" else A
+    Ag = K.Matrix(M, storage=st)
+    b = [wl.uniform(A.m, 6 + k) for k in range(3)]
+    bg = [torch.tensor(v, device="cuda") for v in b]
+    xg = [torch.zeros_like(v) for v in bg]
+    K.SOR(Ag, xg[2], bg[2], 1.2, 1, 0)  # plan
+    ref = [np.zeros(A.m), np.zeros(A.m), orc.sor(M, np.zeros(A.m), b[2], 1.2, 1, 0, storage=st)]
+    ctx = K.Context.default()
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    graphs = [torch.cuda.CUDAGraph() for _ in range(2)]
+    torch.cuda.synchronize()
+
+    def check():
+        torch.cuda.synchronize()
+        for k in range(3):
+            assert np.array_equal(xg[k].cpu().numpy(), ref[k]), k
+
+    try:
+        for k in range(2):
+            with torch.cuda.stream(streams[k]):
+                ctx.bind_stream(streams[k])
+                with torch.cuda.graph(graphs[k], stream=streams[k]):
+                    K.SOR(Ag, xg[k], bg[k], 1.2, 1, 0)
+                    K.SOR(Ag, xg[k], bg[k], 0.9, 1, 2)
+        ctx.bind_stream(streams[2])
+        for _ in range(4):
+            for k in (0, 1, 1, 0):
+                with torch.cuda.stream(streams[k]):
+                    graphs[k].replay()
+                for o, sweep in ((1.2, 0), (0.9, 2)):
+                    ref[k] = orc.sor(M, ref[k], b[k], o, 1, sweep, storage=st)
+            check()
+        for _ in range(4):
+            with torch.cuda.stream(streams[0]):
+                graphs[0].replay()
+            K.SOR(Ag, xg[2], bg[2], 1.2, 1, 0)
+            for o, sweep in ((1.2, 0), (0.9, 2)):
+                ref[0] = orc.sor(M, ref[0], b[0], o, 1, sweep, storage=st)
+            ref[2] = orc.sor(M, ref[2], b[2], 1.2, 1, 0, storage=st)
+            check()
+    finally:
+        torch.cuda.synchronize()
+        ctx.bind_stream()

@@ -91,6 +91,30 @@ int shk_ctx_set_stream(shk_ctx ctx, void *hip_stream);
 int shk_ctx_synchronize(shk_ctx ctx);
 int shk_ctx_device_info(shk_ctx ctx, int *num_cus, int *num_xcds, char *arch, int arch_len);
 
+/* Some kernels' work-groups wait for each other (Cg held on chip, the
+ * orthogonalisation of a Gmres step, SOR sweeps, batched systems on teams).
+ * A wait that runs out (a GPU shared with other work) ends the kernel and the
+ * call takes another way: Cg and Gmres start over with kernels that do not
+ * wait, SOR lets one wavefront do the sweep, a batched solve reports
+ * SHK_ERR_STATE. */
+typedef enum {
+    SHK_OPT_ON_CHIP = 0,     /* 1 (default): kernels that wait, where they fit; 0: Cg and Gmres without them */
+    SHK_OPT_WAIT_US = 1,     /* how long a wait may take, in microseconds: -1 (default) for 2 s (SOR 4, batched
+                                20); 0 gives up after a look or two */
+    SHK_OPT_BUFFER_BYTES = 2 /* SOR: values exchanged through 32-bit offsets up to so many bytes (default
+                                2^31 - 1), through 64-bit addresses past them */
+} shk_option;
+int shk_ctx_set_option(shk_ctx ctx, int option, int64_t value);
+/* What the context's calls did since it was created (synchronises). */
+typedef enum {
+    SHK_COUNT_CG_ON_CHIP = 0,    /* Cg solves held on chip to their end */
+    SHK_COUNT_GMRES_ON_CHIP = 1, /* Gmres solves with the orthogonalisation in one kernel per step */
+    SHK_COUNT_BATCH_ON_CHIP = 2, /* batched calls held on chip */
+    SHK_COUNT_STARTED_OVER = 3,  /* Cg and Gmres solves started over after a wait ran out */
+    SHK_COUNT_SOR_RESCUED = 4    /* SOR sweeps left to one wavefront */
+} shk_counter;
+int shk_ctx_counter(shk_ctx ctx, int counter, int64_t *value);
+
 /* ---- device memory (Allocator role: share/Allocator.cxx:34-65) --------- */
 int shk_malloc(shk_ctx ctx, size_t bytes, void **dptr);
 int shk_free(shk_ctx ctx, void *dptr);

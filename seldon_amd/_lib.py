@@ -50,6 +50,8 @@ SIGNATURES = [
     ("shk_ctx_set_stream", _I, [_P, _P]),
     ("shk_ctx_synchronize", _I, [_P]),
     ("shk_ctx_device_info", _I, [_P, _PI, _PI, ctypes.c_char_p, _I]),
+    ("shk_ctx_set_option", _I, [_P, _I, _I64]),
+    ("shk_ctx_counter", _I, [_P, _I, _PI64]),
     ("shk_malloc", _I, [_P, _U, _PP]),
     ("shk_free", _I, [_P, _P]),
     ("shk_memcpy_h2d", _I, [_P, _P, _P, _U]),

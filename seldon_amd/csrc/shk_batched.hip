@@ -93,7 +93,7 @@ __device__ __forceinline__ void team_wait(Team &t)
         const long long t0 = wall_clock64();
         while (__hip_atomic_load(t.cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
             if (__hip_atomic_load(t.stall, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) break;
-            if (wall_clock64() - t0 > t.limit) {
+            if (wall_clock64() - t0 >= t.limit) {
                 atomicExch(t.stall, 1u);
                 break;
             }
@@ -632,7 +632,8 @@ __global__ __launch_bounds__(kBrThreads, 2) void k_cg_batched_res(ResBatch a)
         R.step = a.step;
         res_window(R);
         const int k = a.team[s];
-        ResTeam t{k, sl.y, LlBuf(a.words + a.slot_off[s], 2 * k * res_slot_words<double>()), 0u, a.stall, a.limit};
+        ResTeam t{k, sl.y, LlBuf(a.words + a.slot_off[s], 2 * k * res_slot_words<double>()), 0u, a.stall, a.limit,
+                  res_every(a.limit)};
         // Init(b); x = 0, r = b (Cg.cxx:58-67)
         double x[RPT], r[RPT], c[1] = {0.0};
 #pragma unroll
@@ -837,7 +838,7 @@ static int batched_resident(shk_ctx ctx, shk_csr A, int count, const int *row_of
     a.steps = flag[0];
     a.queue = ctx->red.ticket + 32;  // a ticket slot of its own
     a.stall = d_flag + 3;
-    SHK_TRY(wall_clock_ticks(ctx, kTeamWaitSeconds, &a.limit));
+    SHK_TRY(wait_ticks(ctx, kTeamWaitSeconds, &a.limit));
     a.tol = tol;
     a.max_iter = max_iter;
     a.its = d_its;
@@ -859,6 +860,7 @@ static int batched_resident(shk_ctx ctx, shk_csr A, int count, const int *row_of
     SHK_HIP(hipStreamSynchronize(st));
     SHK_CHECK(stall == 0u, SHK_ERR_STATE,
               "cg_batched: a team of work-groups waited too long for its members (is the GPU shared?)");
+    ctx->count[SHK_COUNT_BATCH_ON_CHIP]++;
     *solved = true;
     return SHK_OK;
 }
@@ -1034,7 +1036,7 @@ static int batched_common(shk_ctx ctx, shk_csr A64, shk_csr A32, int count, cons
     a.team_cnt = d_tcnt;
     a.team_slot = d_tslot;
     a.stall = d_stall;
-    SHK_TRY(wall_clock_ticks(ctx, kTeamWaitSeconds, &a.limit));
+    SHK_TRY(wait_ticks(ctx, kTeamWaitSeconds, &a.limit));
     a.row_off = d_off;
     a.A64 = SellView{(const int *)A64->ptr, d_boff, d_scol, d_sval};
     if (mixed) a.A32 = SellView{(const int *)A64->ptr, d_boff, d_scol, d_sval32};

@@ -57,11 +57,13 @@ int ensure_ws2(shk_ctx ctx, size_t bytes)
     return SHK_OK;
 }
 
-int wall_clock_ticks(shk_ctx ctx, long long seconds, long long *ticks)
+int wait_ticks(shk_ctx ctx, long long seconds, long long *ticks)
 {
     int khz = 0;
     SHK_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ctx->device));
-    *ticks = (long long)(khz > 0 ? khz : 100000) * 1000LL * seconds;  // 100 MHz where none is reported
+    if (khz <= 0) khz = 100000;  // 100 MHz where none is reported
+    const int64_t us = ctx->opt[SHK_OPT_WAIT_US];
+    *ticks = us >= 0 ? us * khz / 1000 : (long long)khz * 1000 * seconds;
     return SHK_OK;
 }
 
@@ -167,6 +169,33 @@ int shk_ctx_device_info(shk_ctx c, int *num_cus, int *num_xcds, char *arch, int 
         std::strncpy(arch, c->arch, arch_len - 1);
         arch[arch_len - 1] = 0;
     }
+    return SHK_OK;
+}
+
+int shk_ctx_set_option(shk_ctx c, int option, int64_t value)
+{
+    SHK_CHECK(c, SHK_ERR_ARG, "null ctx");
+    bool ok = false;
+    if (option == SHK_OPT_ON_CHIP) ok = value == 0 || value == 1;
+    else if (option == SHK_OPT_WAIT_US) ok = value >= -1 && value <= 3600LL * 1000000;
+    else if (option == SHK_OPT_BUFFER_BYTES) ok = value >= 0 && value <= INT32_MAX;
+    SHK_CHECK(ok, SHK_ERR_ARG, "shk_ctx_set_option: unknown option or value out of range");
+    c->opt[option] = value;
+    return SHK_OK;
+}
+
+int shk_ctx_counter(shk_ctx c, int counter, int64_t *value)
+{
+    SHK_CHECK(c && value, SHK_ERR_ARG, "shk_ctx_counter: null argument");
+    SHK_CHECK(counter >= 0 && counter <= SHK_COUNT_SOR_RESCUED, SHK_ERR_ARG, "shk_ctx_counter: unknown counter");
+    SHK_HIP(hipStreamSynchronize(c->stream));
+    if (counter != SHK_COUNT_SOR_RESCUED) {
+        *value = c->count[counter];
+        return SHK_OK;
+    }
+    unsigned v = 0;
+    SHK_HIP(hipMemcpy(&v, c->red.ticket + kRescuedSlot, sizeof(v), hipMemcpyDeviceToHost));
+    *value = v;
     return SHK_OK;
 }
 

@@ -77,7 +77,8 @@ __global__ __launch_bounds__(kGoThreads, 2) void k_gm_ortho(GmOrtho<T> a)
             gs1 = st->gs[i + 1];
         }
     }
-    ResTeam t{a.k, (int)blockIdx.x, LlBuf(a.slot, 2 * a.k * res_slot_words<T>()), a.epoch, &st->res_stall, a.limit};
+    ResTeam t{a.k, (int)blockIdx.x, LlBuf(a.slot, 2 * a.k * res_slot_words<T>()), a.epoch, &st->res_stall, a.limit,
+               res_every(a.limit)};
     // vector q of this thread: byte q kGoThreads 16 after `at`; past ldv reads
     // are 0 and writes dropped
     const int bytes = (int)(a.ldv * (int64_t)sizeof(T));
@@ -236,7 +237,7 @@ int gm_ortho(shk_ctx ctx, const T *V, int64_t ldv, T *w, int i, unsigned *epoch,
     a.epoch = *epoch;
     a.slot = (ll_word *)slot;
     a.st = st;
-    SHK_TRY(wall_clock_ticks(ctx, kGoWaitSeconds, &a.limit));
+    SHK_TRY(wait_ticks(ctx, kGoWaitSeconds, &a.limit));
     *epoch += (unsigned)i + 2;
     const size_t lds = sizeof(double) * 3 * ((size_t)i + 2);
     const dim3 grid(a.k), blk(kGoThreads);

@@ -84,6 +84,10 @@ struct shk_ctx_s {
     // second arena for drivers that call a solver (iterative refinement)
     void *ws2 = nullptr;
     size_t ws2_cap = 0;
+    // shk_ctx_set_option, shk_ctx_counter (SHK_COUNT_SOR_RESCUED is on the
+    // device: red.ticket[kRescuedSlot])
+    int64_t opt[3] = {1, -1, INT32_MAX};
+    int64_t count[4] = {0, 0, 0, 0};
 };
 
 struct shk_csr_s {
@@ -321,8 +325,10 @@ void sliced_free(shk_csr A);
 // many rows (256 panels of 8192 rows)
 constexpr int kSlAutoMinRows = 1 << 21;
 int check_device_ptr(const void *p, const char *what);
-// wall_clock64 ticks of the given seconds
-int wall_clock_ticks(shk_ctx ctx, long long seconds, long long *ticks);
+// the limit of a wait between work-groups in wall_clock64 ticks: the given
+// seconds, or what SHK_OPT_WAIT_US says
+int wait_ticks(shk_ctx ctx, long long seconds, long long *ticks);
+constexpr int kRescuedSlot = 48;  // of red.ticket
 // Kernels whose work-groups wait for each other need all of them on the GPU
 // at once: two such launches from two threads could each hold half of it.
 // Whoever launches one holds the device's mutex until it has ended.

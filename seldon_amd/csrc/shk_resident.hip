@@ -31,7 +31,7 @@ __global__ __launch_bounds__(kResThreads, 2) void k_cg_resident(ResSolve<T> a)
     if (st->skip) return;
     const int tid = threadIdx.x;
     if (tid == 0) sh.bad = 0;
-    ResTeam t{a.k, (int)blockIdx.x, LlBuf(a.slot, 2 * a.k * res_slot_words<T>()), 0u, &st->res_stall, a.limit};
+    ResTeam t{a.k, (int)blockIdx.x, LlBuf(a.slot, 2 * a.k * res_slot_words<T>()), 0u, &st->res_stall, a.limit, res_every(a.limit)};
     const LlBuf zw(a.zw, (int64_t)a.m * ll_words<T>());
     ResRows R;
     R.r0 = 0;
@@ -167,7 +167,7 @@ int cg_resident(shk_ctx ctx, shk_csr A, const T *diag, T *x, T *r, void *zw, voi
     a.zw = (ll_word *)zw;
     a.slot = (ll_word *)slot;
     a.st = st;
-    SHK_TRY(wall_clock_ticks(ctx, kResWaitSeconds, &a.limit));
+    SHK_TRY(wait_ticks(ctx, kResWaitSeconds, &a.limit));
     const int64_t nz = (int64_t)A->m * ll_words<T>();
     hipLaunchKernelGGL(k_res_clear, dim3(red_blocks(nz)), dim3(kBlock), 0, s, nz, a.zw,
                        2 * a.k * res_slot_words<T>(), a.slot, (const int *)&st->skip);

@@ -193,7 +193,9 @@ struct ResTeam {
     unsigned epoch;       // of the last sum posted (0: none)
     unsigned *stall;
     long long limit;      // wall-clock ticks a wait may take
+    unsigned every;       // looks between two at the clock, less one (2^k - 1)
 };
+__host__ __device__ constexpr unsigned res_every(long long limit) { return limit > 0 ? 63u : 0u; }
 
 // Work-group scratch of the sums.
 template <typename T>
@@ -203,19 +205,20 @@ struct ResShared {
     int bad;              // a wait of this work-group ran out
 };
 
-// A bounded wait: false when the time is up or another member gave up.
+// A bounded wait: false when the time is up (after the first look with a limit
+// of 0) or another member gave up.
 template <class Ready>
 __device__ __forceinline__ bool res_poll(const ResTeam &t, Ready ready)
 {
     asm volatile("" ::: "memory");  // no word read before this call
     if (ready()) return true;
     const long long t0 = wall_clock64();
-    for (int n = 0;; n++) {
+    for (unsigned n = 0;; n++) {
         asm volatile("" ::: "memory");  // the words are read again
         if (ready()) return true;
-        if ((n & 63) == 63) {
+        if ((n & t.every) == t.every) {
             if (__hip_atomic_load(t.stall, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return false;
-            if (wall_clock64() - t0 > t.limit) {
+            if (wall_clock64() - t0 >= t.limit) {
                 __hip_atomic_store(t.stall, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 return false;
             }

@@ -2511,14 +2511,19 @@ int cg_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration *i
     }
     SHK_HIP(hipGetLastError());
     const T *dg = (const T *)A->diag;
-    if (resident && cg_resident_fits(A)) {
+    if (resident && ctx->opt[SHK_OPT_ON_CHIP] && cg_resident_fits(A)) {
         std::lock_guard<std::mutex> lk(resident_mutex(ctx->device));
         SHK_TRY(cg_resident<T>(ctx, A, jac ? dg : nullptr, x, r, p, S.partials, S.dst));
         SHK_TRY(S.read_state());
-        if (!S.hst->res_stall) return S.finish(it, code);
+        if (!S.hst->res_stall) {
+            if (S.hst->res_ran) ctx->count[SHK_COUNT_CG_ON_CHIP]++;
+            return S.finish(it, code);
+        }
     }
-    if (S.hst->res_stall)  // a member waited too long for the others (a shared GPU): x is as it was, start over
+    if (S.hst->res_stall) {  // a member waited too long for the others (a shared GPU): x is as it was, start over
+        ctx->count[SHK_COUNT_STARTED_OVER]++;
         return cg_impl<T>(ctx, A, x, b, prec, it, code, ext, ext_cap, false);
+    }
     const int64_t limit = (int64_t)std::max(it->max_iter, 0) + 2;
     // the loop head of iterations 1 .. of a chunk is folded into
     // the next kernel (identity: k_cg_p_top; Jacobi: k_cg_z_top, and rho =
@@ -2637,7 +2642,7 @@ int gmres_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration
     // columns of V at a stride of whole 256-byte lines (16-byte accesses for
     // every n)
     const int64_t ldv = ((int64_t)A->m + 31) & ~(int64_t)31;
-    resident = resident && gm_ortho_fits<T>(ctx, ldv, m);
+    resident = resident && ctx->opt[SHK_OPT_ON_CHIP] && gm_ortho_fits<T>(ctx, ldv, m);
     const bool keep_x = resident && !it->init_guess_null;  // to start over from
     SHK_TRY(S.setup(ctx, A, (size_t)m + 4 + (keep_x ? 1 : 0), small + 8 * gm_ortho_words() + 256 * (size_t)(m + 2), it));
     const int64_t n = S.n;
@@ -2730,6 +2735,7 @@ int gmres_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration
                 // a work-group waited too long for the others (a shared GPU):
                 // start over with a kernel per pass
                 lk.unlock();
+                ctx->count[SHK_COUNT_STARTED_OVER]++;
                 if (keep_x) SHK_HIP(hipMemcpyAsync(x, x0, sizeof(T) * n, hipMemcpyDeviceToDevice, st));
                 return gmres_impl<T>(ctx, A, x, b, prec, it, code, false);
             }
@@ -2746,6 +2752,7 @@ int gmres_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration
         SHK_HIP(hipGetLastError());
         SHK_TRY(S.read_state());
     }
+    if (resident && epoch) ctx->count[SHK_COUNT_GMRES_ON_CHIP]++;
     return S.finish(it, code);
 }
 

@@ -90,7 +90,6 @@ struct SorPlan {
     int2 *piece[2] = {nullptr, nullptr};   // {first of rows[d], count}: up to 64 rows of one level
     int npiece[2] = {0, 0};
     std::vector<SorWork> work;             // [0]: direct calls
-    long long limit = 0;
 };
 
 // ---- row operations ------------------------------------------------------
@@ -186,9 +185,11 @@ __global__ void k_sor_begin(SorState *st)
 template <typename T, class Words, class Op>
 __global__ __launch_bounds__(kBlock) void k_sor_sweep(int m, const int *__restrict__ rows, const int *__restrict__ pos,
                                                       const int2 *__restrict__ piece, int npiece, Op op,
-                                                      ll_word *words, SorState *st, long long limit, bool rescue)
+                                                      ll_word *words, SorState *st, long long limit, bool rescue,
+                                                      unsigned *rescued)
 {
     if (rescue && !st->stall) return;
+    if (rescue && threadIdx.x == 0) atomicAdd(rescued, 1u);
     const unsigned sweep = st->sweep;
     const Words w(words, (int64_t)m * ll_words<T>());
     const int lane = threadIdx.x & (kWave - 1);
@@ -249,8 +250,8 @@ __global__ __launch_bounds__(kBlock) void k_sor_sweep(int m, const int *__restri
                     if (!__builtin_amdgcn_ballot_w64(!all)) break;
                     if (rescue) {
                         if (n == kSorOwnPolls) break;
-                    } else if ((n & 255) == 0) {
-                        const bool late = wall_clock64() - t0 > limit;
+                    } else if ((n & 255) == 0 || limit <= 0) {
+                        const bool late = wall_clock64() - t0 >= limit;
                         if (late) __hip_atomic_store(&st->stall, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                         if (late || __hip_atomic_load(&st->stall, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
                     }
@@ -502,11 +503,6 @@ static int sor_build(shk_csr A, SorPlan **out)
         sor_free(P);
         return fail(SHK_ERR_NOMEM, std::string("sor: device memory: ") + hipGetErrorString(e));
     }
-    const int st = wall_clock_ticks(A->ctx, kSorWaitSeconds, &P->limit);
-    if (st != SHK_OK) {
-        sor_free(P);
-        return st;
-    }
     *out = P;
     return SHK_OK;
 }
@@ -537,28 +533,29 @@ static inline dim3 grid_for(int count) { return dim3((count + kBlock - 1) / kBlo
 // work-group per CU at most: more of them than the levels can use only poll
 // (128^3 with 64 / 128 / 256 / 512 work-groups: 1.78 / 1.40 / 1.36 / 1.45 ms).
 template <typename T, class Words, class Op>
-static void launch_sweep(shk_ctx ctx, const SorPlan *P, const SorWork &w, int d, const Op &op, T *X)
+static void launch_sweep(shk_ctx ctx, const SorPlan *P, const SorWork &w, long long limit, int d, const Op &op, T *X)
 {
     hipStream_t s = ctx->stream;
     const int np = P->npiece[d], waves = kBlock / kWave;
     const dim3 grid(std::max(1, std::min((np + waves - 1) / waves, ctx->num_cus))), blk(kBlock);
+    unsigned *rescued = ctx->red.ticket + kRescuedSlot;
     hipLaunchKernelGGL(k_sor_begin, dim3(1), dim3(1), 0, s, w.state);
     hipLaunchKernelGGL((k_sor_sweep<T, Words, Op>), grid, blk, 0, s, P->m, (const int *)P->rows[d],
-                       (const int *)P->pos[d], (const int2 *)P->piece[d], np, op, w.word, w.state, P->limit, false);
+                       (const int *)P->pos[d], (const int2 *)P->piece[d], np, op, w.word, w.state, limit, false, rescued);
     hipLaunchKernelGGL((k_sor_sweep<T, Words, Op>), dim3(1), dim3(kWave), 0, s, P->m, (const int *)P->rows[d],
-                       (const int *)P->pos[d], (const int2 *)P->piece[d], np, op, w.word, w.state, P->limit, true);
+                       (const int *)P->pos[d], (const int2 *)P->piece[d], np, op, w.word, w.state, limit, true, rescued);
     hipLaunchKernelGGL((k_sor_out<T, Words>), grid_for(P->m), blk, 0, s, P->m, (const int *)P->pos[d], w.word, X,
                        (const SorState *)w.state);
 }
 
 // 32-bit buffer offsets reach 2 GiB of words (134M FP64 rows)
 template <typename T, class Op>
-static void run_sweep(shk_ctx ctx, const SorPlan *P, const SorWork &w, int d, const Op &op, T *X)
+static void run_sweep(shk_ctx ctx, const SorPlan *P, const SorWork &w, long long limit, int d, const Op &op, T *X)
 {
-    if ((int64_t)P->m * ll_words<T>() * (int64_t)sizeof(ll_word) < INT32_MAX)
-        launch_sweep<T, LlBuf>(ctx, P, w, d, op, X);
+    if ((int64_t)P->m * ll_words<T>() * (int64_t)sizeof(ll_word) < ctx->opt[SHK_OPT_BUFFER_BYTES])
+        launch_sweep<T, LlBuf>(ctx, P, w, limit, d, op, X);
     else
-        launch_sweep<T, LlPtr>(ctx, P, w, d, op, X);
+        launch_sweep<T, LlPtr>(ctx, P, w, limit, d, op, X);
 }
 
 template <typename T, typename W>
@@ -568,18 +565,20 @@ static int sor_run(shk_ctx ctx, SorPlan *P, T *X, const T *B, W omega, int iter,
     const T *val = (const T *)P->val, *diag = (const T *)P->diag, *tval = (const T *)P->tval;
     SorWork w;
     SHK_TRY(sor_work<T>(ctx, P, w));
+    long long limit = 0;
+    SHK_TRY(wait_ticks(ctx, kSorWaitSeconds, &limit));
     T *Z = (T *)w.z;
     auto sweep = [&](int d) {
         if (P->storage != SHK_ROWSYMSPARSE) {
-            run_sweep<T>(ctx, P, w, d, SorRow<T, W>{P->ptr, P->ind, val, diag, B, X, omega, d == 0}, X);
+            run_sweep<T>(ctx, P, w, limit, d, SorRow<T, W>{P->ptr, P->ind, val, diag, B, X, omega, d == 0}, X);
         } else if (d == 0) {
             hipLaunchKernelGGL((k_sor_sym_f1<T, W>), grid_for(P->m), dim3(kBlock), 0, s, P->m, P->ptr, P->ind, val,
                                diag, B, (const T *)X, Z, omega);
-            run_sweep<T>(ctx, P, w, 0, SymForward<T, W>{P->tptr, P->tind, tval, diag, Z, X, omega}, X);
+            run_sweep<T>(ctx, P, w, limit, 0, SymForward<T, W>{P->tptr, P->tind, tval, diag, Z, X, omega}, X);
         } else {
             hipLaunchKernelGGL((k_sor_sym_b1<T, W>), grid_for(P->m), dim3(kBlock), 0, s, P->m, P->tptr, P->tind,
                                tval, diag, B, (const T *)X, Z, omega);
-            run_sweep<T>(ctx, P, w, 1, SymBackward<T, W>{P->ptr, P->ind, val, diag, Z, X, omega}, X);
+            run_sweep<T>(ctx, P, w, limit, 1, SymBackward<T, W>{P->ptr, P->ind, val, diag, Z, X, omega}, X);
         }
     };
     if (type_ssor % 2 == 0)

@@ -54,6 +54,17 @@ class Context:
         L.check(L.load().shk_ctx_device_info(self.h, ctypes.byref(cus), ctypes.byref(xcds), arch, 64))
         return dict(cus=cus.value, xcds=xcds.value, arch=arch.value.decode())
 
+    OPTIONS = {"on_chip": 0, "wait_us": 1, "buffer_bytes": 2}
+    COUNTERS = {"cg_on_chip": 0, "gmres_on_chip": 1, "batch_on_chip": 2, "started_over": 3, "sor_rescued": 4}
+
+    def set_option(self, name: str, value: int):
+        L.check(L.load().shk_ctx_set_option(self.h, self.OPTIONS[name], int(value)))
+
+    def counter(self, name: str) -> int:
+        v = ctypes.c_int64()
+        L.check(L.load().shk_ctx_counter(self.h, self.COUNTERS[name], ctypes.byref(v)))
+        return v.value
+
     def close(self):
         if self.h:
             L.load().shk_ctx_destroy(self.h)

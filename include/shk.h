@@ -21,7 +21,10 @@
  *     the *_device variants leave them in device memory instead.
  *   - A context is single-threaded (Seldon is not thread-safe either,
  *     vector/Vector.hxx:50); separate contexts may be used from separate
- *     threads.  Device memory is owned by the handles.
+ *     threads.  Solves whose work-groups wait for each other (Cg held on chip,
+ *     4 steps of Gmres at a time, batched systems) run side by side while
+ *     their work-groups fit the device together; one that does not fit waits
+ *     in the call for its turn.  Device memory is owned by the handles.
  *   - Arithmetic order: SpMV row sums are taken sequentially in stored order,
  *     exactly as Functions_MatVect.cxx:424-430 does, and FP64/FP32 products
  *     and sums are not contracted into FMAs, so SpMV results are bitwise

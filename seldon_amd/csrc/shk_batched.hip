@@ -844,7 +844,8 @@ static int batched_resident(shk_ctx ctx, shk_csr A, int count, const int *row_of
     a.its = d_its;
     a.codes = d_codes;
     const dim3 grid(std::min(nslot, ctx->num_cus));
-    std::lock_guard<std::mutex> lk(resident_mutex(ctx->device));
+    Seats seats(ctx);
+    seats.take(grid.x);
     SHK_TRY(launch_batch(ctx, st, use_graph, [&](hipStream_t s) -> int {
         hipLaunchKernelGGL(k_batch_res_reset, dim3(red_blocks(zwords + nwords)), dim3(kBlock), 0, s, a.queue, a.stall,
                            zwords + nwords, d_words);
@@ -1052,7 +1053,8 @@ static int batched_common(shk_ctx ctx, shk_csr A64, shk_csr A32, int count, cons
     a.its = d_its;
     a.codes = d_codes;
     a.queue = ctx->red.ticket + 32;  // a ticket slot of its own
-    std::lock_guard<std::mutex> lk(resident_mutex(ctx->device));
+    Seats seats(ctx);
+    seats.take(grid);
     // the queue reset is a kernel node, not a memset node
     SHK_TRY(launch_batch(ctx, st, use_graph, [&](hipStream_t cs) -> int {
         hipLaunchKernelGGL(k_batch_reset, dim3((count + 255) / 256), dim3(256), 0, cs, a.queue, a.stall,

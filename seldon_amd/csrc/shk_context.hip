@@ -1,5 +1,8 @@
 // shk_context.hip -- context, errors and device memory of the shk library.
+#include <algorithm>
+#include <condition_variable>
 #include <cstring>
+#include <mutex>
 
 #include "shk_internal.hpp"
 
@@ -65,6 +68,46 @@ int wait_ticks(shk_ctx ctx, long long seconds, long long *ticks)
     const int64_t us = ctx->opt[SHK_OPT_WAIT_US];
     *ticks = us >= 0 ? us * khz / 1000 : (long long)khz * 1000 * seconds;
     return SHK_OK;
+}
+
+namespace {
+struct SeatQueue {
+    std::mutex mu;
+    std::condition_variable cv;
+    uint64_t next = 0, serving = 0;  // turns given out, and whose it is
+    int used = 0;
+};
+SeatQueue &seat_queue(int device)
+{
+    static SeatQueue q[64];
+    return q[device & 63];
+}
+}  // namespace
+
+void Seats::take(int groups)
+{
+    give();
+    const int need = std::min((groups + kNumXcd - 1) / kNumXcd, most_);
+    SeatQueue &q = seat_queue(device_);
+    std::unique_lock<std::mutex> lk(q.mu);
+    const uint64_t mine = q.next++;
+    q.cv.wait(lk, [&]() { return q.serving == mine && q.used + need <= most_; });
+    q.used += need;
+    q.serving++;
+    held_ = need;
+    q.cv.notify_all();
+}
+
+void Seats::give()
+{
+    if (!held_) return;
+    SeatQueue &q = seat_queue(device_);
+    {
+        std::lock_guard<std::mutex> lk(q.mu);
+        q.used -= held_;
+    }
+    held_ = 0;
+    q.cv.notify_all();
 }
 
 int check_device_ptr(const void *p, const char *what)

@@ -212,6 +212,15 @@ bool gm_ortho_fits(shk_ctx ctx, int64_t ldv, int m)
     return ldv * (int64_t)sizeof(T) / 16 <= (int64_t)kGoMaxVec * kGoThreads * cus && m <= 1000;
 }
 
+// work-groups of a step
+template <typename T>
+int gm_ortho_groups(shk_ctx ctx, int64_t ldv)
+{
+    const int64_t vecs = ldv * (int64_t)sizeof(T) / 16;
+    const int64_t per = (int64_t)go_vectors(vecs, std::min(ctx->num_cus, kResMaxTeam)) * kGoThreads;
+    return (int)((vecs + per - 1) / per);
+}
+
 size_t gm_ortho_words() { return 2 * (size_t)kResMaxTeam * res_slot_words<double>(); }
 
 template <typename T>
@@ -233,7 +242,7 @@ int gm_ortho(shk_ctx ctx, const T *V, int64_t ldv, T *w, int i, unsigned *epoch,
     a.w = w;
     a.ldv = ldv;
     a.i = i;
-    a.k = (int)((vecs + (int64_t)nv * kGoThreads - 1) / ((int64_t)nv * kGoThreads));
+    a.k = gm_ortho_groups<T>(ctx, ldv);
     a.epoch = *epoch;
     a.slot = (ll_word *)slot;
     a.st = st;
@@ -254,6 +263,8 @@ int gm_ortho(shk_ctx ctx, const T *V, int64_t ldv, T *w, int i, unsigned *epoch,
 
 template bool gm_ortho_fits<double>(shk_ctx, int64_t, int);
 template bool gm_ortho_fits<float>(shk_ctx, int64_t, int);
+template int gm_ortho_groups<double>(shk_ctx, int64_t);
+template int gm_ortho_groups<float>(shk_ctx, int64_t);
 template int gm_ortho_start<double>(shk_ctx, void *);
 template int gm_ortho_start<float>(shk_ctx, void *);
 template int gm_ortho<double>(shk_ctx, const double *, int64_t, double *, int, unsigned *, void *, KState<double> *);

@@ -9,7 +9,6 @@
 
 #include <cstdint>
 #include <cstdio>
-#include <mutex>
 #include <string>
 #include <vector>
 
@@ -329,10 +328,26 @@ int check_device_ptr(const void *p, const char *what);
 // seconds, or what SHK_OPT_WAIT_US says
 int wait_ticks(shk_ctx ctx, long long seconds, long long *ticks);
 constexpr int kRescuedSlot = 48;  // of red.ticket
-// Kernels whose work-groups wait for each other need all of them on the GPU
-// at once: two such launches from two threads could each hold half of it.
-// Whoever launches one holds the device's mutex until it has ended.
-std::mutex &resident_mutex(int device);
+// Kernels whose work-groups wait for each other need all of them on the GPU at
+// once: launches from several threads could each hold a part of it and none
+// enough.  Whoever launches one takes seats for its work-groups until it has
+// ended.  A work-group may fill a CU, and an XCD gets every eighth work-group
+// of a launch, so a launch of `groups` takes ceil(groups / 8) of an XCD's CUs;
+// launches that fit together run together, others wait their turn, in order.
+// Kernels of the same kind that wait for nobody (a member by itself) take
+// theirs too: they may hold a CU for as long as a solve.
+class Seats {
+public:
+    explicit Seats(shk_ctx ctx) : device_(ctx->device), most_(ctx->num_cus / kNumXcd) {}
+    ~Seats() { give(); }
+    Seats(const Seats &) = delete;
+    Seats &operator=(const Seats &) = delete;
+    void take(int groups);
+    void give();
+
+private:
+    int device_, most_, held_ = 0;
+};
 constexpr size_t kResLds = 158 * 1024;  // LDS of a resident work-group's window
 
 }  // namespace shk

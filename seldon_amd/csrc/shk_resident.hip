@@ -1,7 +1,6 @@
 // shk_resident.hip -- one Cg solve on chip (shk_resident.hpp): the kernel and
 // its launch.
 #include <algorithm>
-#include <mutex>
 
 #include "shk_resident.hpp"
 #include "shk_solver_state.hpp"
@@ -134,10 +133,10 @@ bool cg_resident_fits(shk_csr A)
            share + halo < 0xffff;
 }
 
-std::mutex &resident_mutex(int device)
+int cg_resident_groups(shk_csr A)
 {
-    static std::mutex mu[64];
-    return mu[device & 63];
+    const int share = res_rows_per_thread(A->m, A->dia_steps, std::min(A->ctx->num_cus, kResMaxTeam)) * kResThreads;
+    return (A->m + share - 1) / share;
 }
 
 template <typename T, int RPT, int KS>
@@ -158,7 +157,7 @@ int cg_resident(shk_ctx ctx, shk_csr A, const T *diag, T *x, T *r, void *zw, voi
     a.right = A->dia_right;
     a.steps = A->dia_steps;
     a.share = rpt * kResThreads;
-    a.k = (A->m + a.share - 1) / a.share;
+    a.k = cg_resident_groups(A);
     a.step = (const DiaStep *)A->dia_step;
     a.val = (const T *)A->dia_val;
     a.diag = diag;

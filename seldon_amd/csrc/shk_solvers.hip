@@ -2477,6 +2477,7 @@ constexpr int kChunk = 16;
 // one solve on chip (shk_resident.hip): whether the matrix fits, and the
 // launches after the first Finished(r); zw holds 2 n values, slot the partials
 bool cg_resident_fits(shk_csr A);
+int cg_resident_groups(shk_csr A);
 template <typename T>
 int cg_resident(shk_ctx ctx, shk_csr A, const T *diag, T *x, T *r, void *zw, void *slot, KState<T> *st);
 
@@ -2512,7 +2513,8 @@ int cg_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration *i
     SHK_HIP(hipGetLastError());
     const T *dg = (const T *)A->diag;
     if (resident && ctx->opt[SHK_OPT_ON_CHIP] && cg_resident_fits(A)) {
-        std::lock_guard<std::mutex> lk(resident_mutex(ctx->device));
+        Seats seats(ctx);
+        seats.take(cg_resident_groups(A));
         SHK_TRY(cg_resident<T>(ctx, A, jac ? dg : nullptr, x, r, p, S.partials, S.dst));
         SHK_TRY(S.read_state());
         if (!S.hst->res_stall) {
@@ -2624,6 +2626,8 @@ int bicgstab_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iterat
 // the orthogonalisation of a step in one kernel (shk_gmres.hip)
 template <typename T>
 bool gm_ortho_fits(shk_ctx ctx, int64_t ldv, int m);
+template <typename T>
+int gm_ortho_groups(shk_ctx ctx, int64_t ldv);
 size_t gm_ortho_words();
 template <typename T>
 int gm_ortho_start(shk_ctx ctx, void *slot);
@@ -2666,10 +2670,9 @@ int gmres_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration
     hipStream_t st = ctx->stream;
     dim3 g(S.nb), blk(kBlock);
     auto Vk = [&](int k) { return V + (size_t)k * ldv; };
-    std::unique_lock<std::mutex> lk(resident_mutex(ctx->device), std::defer_lock);
+    Seats seats(ctx);  // held over a chunk of steps, until the state is read back
     unsigned epoch = 0;
     if (resident) {
-        lk.lock();
         SHK_TRY(gm_ortho_start<T>(ctx, slot));
         if (ldv > n)
             hipLaunchKernelGGL(k_fill<T>, dim3(1), blk, 0, st, ldv - n, (T)0, w + n, (const int *)nullptr);
@@ -2694,6 +2697,7 @@ int gmres_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration
         SHK_CHECK(++guard <= (int64_t)it->max_iter + 2, SHK_ERR_STATE, "gmres: no progress");
         // Arnoldi steps of one cycle, enqueued in chunks
         for (int i0 = 0; i0 < m; i0 += step_chunk) {
+            if (resident) seats.take(gm_ortho_groups<T>(ctx, ldv));
             for (int i = i0; i < std::min(m, i0 + step_chunk); i++) {
                 SpmvArgs<T> a{};
                 a.x = Vk(i); a.y_out = w; a.alpha = (T)1; a.mlt = 1; a.diag = dg; a.skip = &S.dst->skip;
@@ -2731,10 +2735,10 @@ int gmres_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration
             }
             SHK_HIP(hipGetLastError());
             SHK_TRY(S.read_state());
+            seats.give();
             if (S.hst->res_stall) {
                 // a work-group waited too long for the others (a shared GPU):
                 // start over with a kernel per pass
-                lk.unlock();
                 ctx->count[SHK_COUNT_STARTED_OVER]++;
                 if (keep_x) SHK_HIP(hipMemcpyAsync(x, x0, sizeof(T) * n, hipMemcpyDeviceToDevice, st));
                 return gmres_impl<T>(ctx, A, x, b, prec, it, code, false);

@@ -163,3 +163,54 @@ def test_options_refuse_what_they_cannot_be(ctx):
             ctx.set_option(name, bad)
     lib = L.load()
     assert lib.shk_ctx_set_option(ctx.h, 99, 0) == -1 and lib.shk_ctx_counter(ctx.h, 99, None) == -1
+
+
+@pytest.mark.parametrize("method", ["cg", "gmres"])
+def test_contexts_of_two_threads_run_side_by_side(ctx, method):
+    """A long Cg solve of 64 work-groups in one thread does not keep short
+    solves of another from running and ending meanwhile."""
+    import threading
+    import time
+
+    from seldon_amd import krylov as K
+    A, S = wl.laplace2d(256, 256), wl.laplace2d(64, 64)
+    ctxs = [K.Context(0) for _ in range(2)]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    for c, s in zip(ctxs, streams):
+        c.bind_stream(s)
+    Ag, Sg = K.Matrix(A, ctx=ctxs[0]), K.Matrix(S, ctx=ctxs[1])
+    ab = torch.full((A.m,), float("nan"), dtype=torch.float64, device="cuda")  # never converges
+    sb = torch.tensor(wl.uniform(S.m, 2), device="cuda")
+    ax, sx = torch.zeros_like(ab), torch.zeros_like(sb)
+
+    def solve(Mg, x, b, tol, max_iter):
+        it = K.Iteration(max_iter, tol)
+        it.HideMessages()
+        it.SetRestart(20)
+        it.SetInitGuess(True)
+        f = K.Gmres if method == "gmres" and Mg is Sg else K.Cg
+        return f(Mg, x, b, K.Preconditioner_Base(), it)
+
+    solve(Sg, sx, sb, 1e-6, 2000)
+    torch.cuda.synchronize()
+    spans = []
+
+    def run():
+        t = time.perf_counter()
+        solve(Ag, ax, ab, 1e-10, 300000)  # about a second
+        spans.append((t, time.perf_counter()))
+
+    th = threading.Thread(target=run)
+    th.start()
+    time.sleep(0.1)
+    for _ in range(3):
+        solve(Sg, sx, sb, 1e-6, 2000)
+    ended = time.perf_counter()
+    th.join()
+    torch.cuda.synchronize()
+    print("long solve", spans[0][1] - spans[0][0], "short ones ended before it by", spans[0][1] - ended, flush=True)
+    assert spans[0][1] - spans[0][0] > 0.4
+    assert ended < spans[0][1] - 0.1
+    for c in ctxs:
+        c.synchronize()
+        c.bind_stream()

@@ -98,7 +98,8 @@ int shk_ctx_device_info(shk_ctx ctx, int *num_cus, int *num_xcds, char *arch, in
  * orthogonalisation of a Gmres step, SOR sweeps, batched systems on teams).
  * A wait that runs out (a GPU shared with other work) ends the kernel and the
  * call takes another way: Cg and Gmres start over with kernels that do not
- * wait, SOR lets one wavefront do the sweep, a batched solve reports
+ * wait, and the context's solves keep to those for a minute or until an option
+ * is set; SOR lets one wavefront do the sweep, a batched solve reports
  * SHK_ERR_STATE. */
 typedef enum {
     SHK_OPT_ON_CHIP = 0,     /* 1 (default): kernels that wait, where they fit; 0: Cg and Gmres without them */

@@ -70,6 +70,19 @@ int wait_ticks(shk_ctx ctx, long long seconds, long long *ticks)
     return SHK_OK;
 }
 
+constexpr std::chrono::seconds kNoWaitsFor(60);  // 2 s of waiting in a minute, at most
+
+bool may_wait(shk_ctx ctx)
+{
+    return ctx->opt[SHK_OPT_ON_CHIP] && std::chrono::steady_clock::now() >= ctx->no_waits_until;
+}
+
+void wait_ran_out(shk_ctx ctx)
+{
+    ctx->count[SHK_COUNT_STARTED_OVER]++;
+    ctx->no_waits_until = std::chrono::steady_clock::now() + kNoWaitsFor;
+}
+
 namespace {
 struct SeatQueue {
     std::mutex mu;
@@ -224,6 +237,7 @@ int shk_ctx_set_option(shk_ctx c, int option, int64_t value)
     else if (option == SHK_OPT_BUFFER_BYTES) ok = value >= 0 && value <= INT32_MAX;
     SHK_CHECK(ok, SHK_ERR_ARG, "shk_ctx_set_option: unknown option or value out of range");
     c->opt[option] = value;
+    c->no_waits_until = {};
     return SHK_OK;
 }
 

@@ -7,6 +7,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <chrono>
 #include <cstdint>
 #include <cstdio>
 #include <string>
@@ -87,6 +88,9 @@ struct shk_ctx_s {
     // device: red.ticket[kRescuedSlot])
     int64_t opt[3] = {1, -1, INT32_MAX};
     int64_t count[4] = {0, 0, 0, 0};
+    // after a wait that ran out, Cg and Gmres take the kernels without waits
+    // until then (a shared GPU is paid for once, not on every solve)
+    std::chrono::steady_clock::time_point no_waits_until{};
 };
 
 struct shk_csr_s {
@@ -328,6 +332,9 @@ int check_device_ptr(const void *p, const char *what);
 // seconds, or what SHK_OPT_WAIT_US says
 int wait_ticks(shk_ctx ctx, long long seconds, long long *ticks);
 constexpr int kRescuedSlot = 48;  // of red.ticket
+// whether a Cg or Gmres solve may use kernels that wait; one has run out of time
+bool may_wait(shk_ctx ctx);
+void wait_ran_out(shk_ctx ctx);
 // Kernels whose work-groups wait for each other need all of them on the GPU at
 // once: launches from several threads could each hold a part of it and none
 // enough.  Whoever launches one takes seats for its work-groups until it has

@@ -2512,7 +2512,7 @@ int cg_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration *i
     }
     SHK_HIP(hipGetLastError());
     const T *dg = (const T *)A->diag;
-    if (resident && ctx->opt[SHK_OPT_ON_CHIP] && cg_resident_fits(A)) {
+    if (resident && may_wait(ctx) && cg_resident_fits(A)) {
         Seats seats(ctx);
         seats.take(cg_resident_groups(A));
         SHK_TRY(cg_resident<T>(ctx, A, jac ? dg : nullptr, x, r, p, S.partials, S.dst));
@@ -2523,7 +2523,7 @@ int cg_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration *i
         }
     }
     if (S.hst->res_stall) {  // a member waited too long for the others (a shared GPU): x is as it was, start over
-        ctx->count[SHK_COUNT_STARTED_OVER]++;
+        wait_ran_out(ctx);
         return cg_impl<T>(ctx, A, x, b, prec, it, code, ext, ext_cap, false);
     }
     const int64_t limit = (int64_t)std::max(it->max_iter, 0) + 2;
@@ -2646,7 +2646,7 @@ int gmres_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration
     // columns of V at a stride of whole 256-byte lines (16-byte accesses for
     // every n)
     const int64_t ldv = ((int64_t)A->m + 31) & ~(int64_t)31;
-    resident = resident && ctx->opt[SHK_OPT_ON_CHIP] && gm_ortho_fits<T>(ctx, ldv, m);
+    resident = resident && may_wait(ctx) && gm_ortho_fits<T>(ctx, ldv, m);
     const bool keep_x = resident && !it->init_guess_null;  // to start over from
     SHK_TRY(S.setup(ctx, A, (size_t)m + 4 + (keep_x ? 1 : 0), small + 8 * gm_ortho_words() + 256 * (size_t)(m + 2), it));
     const int64_t n = S.n;
@@ -2739,7 +2739,7 @@ int gmres_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration
             if (S.hst->res_stall) {
                 // a work-group waited too long for the others (a shared GPU):
                 // start over with a kernel per pass
-                ctx->count[SHK_COUNT_STARTED_OVER]++;
+                wait_ran_out(ctx);
                 if (keep_x) SHK_HIP(hipMemcpyAsync(x, x0, sizeof(T) * n, hipMemcpyDeviceToDevice, st));
                 return gmres_impl<T>(ctx, A, x, b, prec, it, code, false);
             }

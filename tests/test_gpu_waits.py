@@ -165,6 +165,31 @@ def test_options_refuse_what_they_cannot_be(ctx):
     assert lib.shk_ctx_set_option(ctx.h, 99, 0) == -1 and lib.shk_ctx_counter(ctx.h, 99, None) == -1
 
 
+def test_a_wait_that_ran_out_is_remembered(ctx):
+    """One solve pays for a GPU that others use; those after it, the inner
+    solves of a refinement too, do not try again at once.  Setting an option
+    ends that."""
+    from seldon_amd import krylov as K
+    A = wl.laplace2d(181, 233)
+    b = wl.apply(A, wl.uniform(A.m, 11))
+    n0 = _counts(ctx, "cg_on_chip", "gmres_on_chip", "started_over")
+    ctx.set_option("wait_us", 0)
+    first, second = _cg(A, b, None, "jacobi"), _cg(A, b, None, "jacobi")
+    C = _convtri(100003)
+    _gmres(C, wl.apply(C, wl.uniform(C.m, 3)), None, 5)
+    assert _counts(ctx, "cg_on_chip", "gmres_on_chip", "started_over") == [n0[0], n0[1], n0[2] + 1]
+    for a, c in zip(first, second):
+        assert np.array_equal(a, c)
+    ctx.set_option("wait_us", 0)
+    A64, A32 = K.Matrix(C), K.Matrix(C, dtype=torch.float32)
+    bg = torch.tensor(wl.apply(C, wl.uniform(C.m, 3)), device="cuda")
+    assert K.solve_ir(A64, A32, torch.zeros_like(bg), bg, K.JacobiPreconditioner(), tol=1e-10)["code"] == 0
+    assert _counts(ctx, "cg_on_chip", "gmres_on_chip", "started_over") == [n0[0], n0[1], n0[2] + 2]
+    ctx.set_option("wait_us", -1)
+    _cg(A, b, None, "jacobi")
+    assert _counts(ctx, "cg_on_chip", "started_over") == [n0[0] + 1, n0[2] + 2]
+
+
 @pytest.mark.parametrize("method", ["cg", "gmres"])
 def test_contexts_of_two_threads_run_side_by_side(ctx, method):
     """A long Cg solve of 64 work-groups in one thread does not keep short

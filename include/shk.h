@@ -105,8 +105,9 @@ typedef enum {
     SHK_OPT_ON_CHIP = 0,     /* 1 (default): kernels that wait, where they fit; 0: Cg and Gmres without them */
     SHK_OPT_WAIT_US = 1,     /* how long a wait may take, in microseconds: -1 (default) for 2 s (SOR 4, batched
                                 20); 0 gives up after a look or two */
-    SHK_OPT_BUFFER_BYTES = 2 /* SOR: values exchanged through 32-bit offsets up to so many bytes (default
+    SHK_OPT_BUFFER_BYTES = 2, /* SOR: values exchanged through 32-bit offsets up to so many bytes (default
                                 2^31 - 1), through 64-bit addresses past them */
+    SHK_OPT_CG_ITERS = 3     /* iterations that one launch of a Cg held on chip does (default 32768) */
 } shk_option;
 int shk_ctx_set_option(shk_ctx ctx, int option, int64_t value);
 /* What the context's calls did since it was created (synchronises). */

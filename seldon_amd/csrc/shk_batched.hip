@@ -646,13 +646,13 @@ __global__ __launch_bounds__(kBrThreads, 2) void k_cg_batched_res(ResBatch a)
         res_post<double, 1, kBrThreads>(c, t, sh);
         if (!res_wait<double, 1, kBrThreads>(c, t, sh)) return;
         const double bn = sqrt(c[0]);
-        ResIter<double> it{0.0, a.tol, a.max_iter, 0, 0, c[0]};
+        ResIter<double> it{0.0, a.tol, a.max_iter, 0, 0, c[0], 0.0, nullptr};
         if (bn != 0.0) {
             it.facteur = 1.0 / bn;
             auto head = [&](int nb, double rr) { return it.facteur * sqrt(rr) < it.tol || nb >= it.max_iter; };
             unsigned zepoch = 0u;
             if (!head(0, c[0]) &&
-                !res_cg<double, kBrThreads, RPT, KS, false>(R, a.val, nullptr, x, r, zw, (double *)res_lds, it, t,
+                !res_cg<double, kBrThreads, RPT, KS, false, false>(R, a.val, nullptr, x, r, zw, (double *)res_lds, it, t,
                                                                 sh, zepoch, head))
                 return;
 #pragma unroll

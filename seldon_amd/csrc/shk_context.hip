@@ -235,6 +235,7 @@ int shk_ctx_set_option(shk_ctx c, int option, int64_t value)
     if (option == SHK_OPT_ON_CHIP) ok = value == 0 || value == 1;
     else if (option == SHK_OPT_WAIT_US) ok = value >= -1 && value <= 3600LL * 1000000;
     else if (option == SHK_OPT_BUFFER_BYTES) ok = value >= 0 && value <= INT32_MAX;
+    else if (option == SHK_OPT_CG_ITERS) ok = value >= 1 && value <= INT32_MAX;
     SHK_CHECK(ok, SHK_ERR_ARG, "shk_ctx_set_option: unknown option or value out of range");
     c->opt[option] = value;
     c->no_waits_until = {};

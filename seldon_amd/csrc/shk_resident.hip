@@ -9,19 +9,24 @@ namespace shk {
 
 constexpr int kResThreads = 512;
 constexpr long long kResWaitSeconds = 2;
+// A launch leaves a solve after SHK_OPT_CG_ITERS iterations (2^15: 0.13 s at
+// 4 us each) and the next one carries it on: contexts of other threads get
+// their turn on the GPU, however long a solve is.  Solves whose max_iter is
+// within that take kernels without the provision (LONG), which in the others
+// costs registers: 256^2 4.0 -> 4.2 us per iteration, with Jacobi 4.4 -> 5.0.
 
 template <typename T>
 struct ResSolve {
-    int m, left, right, steps, share, k;
+    int m, left, right, steps, share, k, iters;
     const DiaStep *step;
     const T *val, *diag, *x0;
-    T *r;                 // in: the residual; out: the solution (each member its own rows)
+    T *r;                 // in: the residual; out: the solution, or the residual (each member its own rows)
     ll_word *zw, *slot;
     long long limit;
     KState<T> *st;
 };
 
-template <typename T, int RPT, int KS, bool JAC>
+template <typename T, int RPT, int KS, bool JAC, bool LONG>
 __global__ __launch_bounds__(kResThreads, 2) void k_cg_resident(ResSolve<T> a)
 {
     extern __shared__ char res_lds[];
@@ -50,18 +55,24 @@ __global__ __launch_bounds__(kResThreads, 2) void k_cg_resident(ResSolve<T> a)
         x[u] = row < R.m1 ? a.x0[row] : (T)0;
         r[u] = row < R.m1 ? a.r[row] : (T)0;
     }
-    ResIter<T> it{st->facteur, st->tol, st->max_iter, st->nb_iter, 0, st->rho};
+    const int nb0 = st->nb_iter;
+    ResIter<T> it{st->facteur, st->tol, st->max_iter, nb0, 0, st->rho, (T)0, nullptr};
+    if (LONG) {  // the launch's share of iterations ends the loop too
+        it.max_iter = (int)min((int64_t)nb0 + a.iters, (int64_t)st->max_iter);
+        it.rho_1 = st->rho_1;
+        it.p = st->res_left;
+    }
     double *hist = st->hist;
     int *hist_it = st->hist_it;
     const int hist_cap = st->hist_cap;
     int hist_len = st->hist_len;
-    double last = 0.0;
+    double last = LONG ? st->last_res : 0.0;
     const bool lead = blockIdx.x == 0 && tid == 0;
     unsigned zepoch = 0u;
     __syncthreads();
     // Iteration::Finished (Iterative.cxx:272-319); every member decides alike,
     // the first records it
-    const bool ok = res_cg<T, kResThreads, RPT, KS, JAC>(
+    const bool ok = res_cg<T, kResThreads, RPT, KS, JAC, LONG>(
         R, a.val, a.diag, x, r, zw, (T *)res_lds, it, t, sh, zepoch, [&](int nb, T rr) {
             const double reste = it.facteur * (double)sqrt_t(rr);
             last = reste;
@@ -72,16 +83,29 @@ __global__ __launch_bounds__(kResThreads, 2) void k_cg_resident(ResSolve<T> a)
             hist_len++;
             return reste < it.tol || nb >= it.max_iter;
         });
+    const bool paused = LONG && ok && !it.code && !(last < it.tol) && it.nb < st->max_iter;
     if (!ok) return;
 #pragma unroll
     for (int u = 0; u < RPT; u++) {
         const int row = R.m0 + u * kResThreads + tid;
-        if (row < R.m1) a.r[row] = x[u];
+        if (row < R.m1) {
+            a.r[row] = LONG && paused ? r[u] : x[u];
+            if (LONG && paused) {
+                T *left = st->res_left;
+                left[row] = ((const T *)res_lds)[row - R.lo];
+                left[a.m + row] = x[u];
+            }
+        }
     }
     if (lead) {
         st->nb_iter = it.nb;
         st->hist_len = hist_len;
         if (it.nb > 0) st->last_res = last;
+        if (LONG && paused) {
+            st->rho_1 = it.rho_1;
+            st->res_paused = 1;
+            return;
+        }
         if (it.code) {
             st->fail = 1;
             st->error_code = it.code;
@@ -92,9 +116,15 @@ __global__ __launch_bounds__(kResThreads, 2) void k_cg_resident(ResSolve<T> a)
 }
 
 // sum words and z words to epoch 0
-__global__ __launch_bounds__(kBlock) void k_res_clear(int64_t nz, ll_word *zw, int ns, ll_word *slot, const int *skip)
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_res_clear(int64_t nz, ll_word *zw, int ns, ll_word *slot, KState<T> *st,
+                                                     T *left)
 {
-    if (*skip) return;
+    if (st->skip) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        st->res_paused = 0;
+        st->res_left = left;
+    }
     for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < nz; i += (int64_t)gridDim.x * kBlock) zw[i] = 0;
     if (blockIdx.x == 0)
         for (int i = threadIdx.x; i < ns; i += kBlock) slot[i] = 0;
@@ -140,14 +170,18 @@ int cg_resident_groups(shk_csr A)
 }
 
 template <typename T, int RPT, int KS>
-static void res_launch(const ResSolve<T> &a, dim3 grid, size_t lds, bool jac, hipStream_t s)
+static void res_launch(const ResSolve<T> &a, dim3 grid, size_t lds, bool jac, bool lng, hipStream_t s)
 {
-    if (jac) hipLaunchKernelGGL((k_cg_resident<T, RPT, KS, true>), grid, dim3(kResThreads), lds, s, a);
-    else hipLaunchKernelGGL((k_cg_resident<T, RPT, KS, false>), grid, dim3(kResThreads), lds, s, a);
+    const dim3 blk(kResThreads);
+    if (jac && lng) hipLaunchKernelGGL((k_cg_resident<T, RPT, KS, true, true>), grid, blk, lds, s, a);
+    else if (jac) hipLaunchKernelGGL((k_cg_resident<T, RPT, KS, true, false>), grid, blk, lds, s, a);
+    else if (lng) hipLaunchKernelGGL((k_cg_resident<T, RPT, KS, false, true>), grid, blk, lds, s, a);
+    else hipLaunchKernelGGL((k_cg_resident<T, RPT, KS, false, false>), grid, blk, lds, s, a);
 }
 
 template <typename T>
-int cg_resident(shk_ctx ctx, shk_csr A, const T *diag, T *x, T *r, void *zw, void *slot, KState<T> *st)
+int cg_resident(shk_ctx ctx, shk_csr A, const T *diag, T *x, T *r, void *zw, void *slot, KState<T> *st, T *pause,
+                bool carry)
 {
     const int rpt = res_rows_per_thread(A->m, A->dia_steps, std::min(ctx->num_cus, kResMaxTeam));
     hipStream_t s = ctx->stream;
@@ -161,25 +195,26 @@ int cg_resident(shk_ctx ctx, shk_csr A, const T *diag, T *x, T *r, void *zw, voi
     a.step = (const DiaStep *)A->dia_step;
     a.val = (const T *)A->dia_val;
     a.diag = diag;
-    a.x0 = x;
+    a.x0 = carry ? pause + A->m : x;
     a.r = r;
     a.zw = (ll_word *)zw;
     a.slot = (ll_word *)slot;
     a.st = st;
     SHK_TRY(wait_ticks(ctx, kResWaitSeconds, &a.limit));
+    a.iters = (int)ctx->opt[SHK_OPT_CG_ITERS];
     const int64_t nz = (int64_t)A->m * ll_words<T>();
-    hipLaunchKernelGGL(k_res_clear, dim3(red_blocks(nz)), dim3(kBlock), 0, s, nz, a.zw,
-                       2 * a.k * res_slot_words<T>(), a.slot, (const int *)&st->skip);
+    hipLaunchKernelGGL(k_res_clear<T>, dim3(red_blocks(nz)), dim3(kBlock), 0, s, nz, a.zw,
+                       2 * a.k * res_slot_words<T>(), a.slot, st, pause);
     const dim3 grid(a.k);
     const size_t lds = (size_t)(a.share + a.left + a.right + 1) * sizeof(T);
-    const bool jac = diag != nullptr;
+    const bool jac = diag != nullptr, lng = pause != nullptr;
     if (a.steps <= 5) {
-        if (rpt == 2) res_launch<T, 2, 5>(a, grid, lds, jac, s);
-        else if (rpt == 4) res_launch<T, 4, 5>(a, grid, lds, jac, s);
-        else res_launch<T, 8, 5>(a, grid, lds, jac, s);
+        if (rpt == 2) res_launch<T, 2, 5>(a, grid, lds, jac, lng, s);
+        else if (rpt == 4) res_launch<T, 4, 5>(a, grid, lds, jac, lng, s);
+        else res_launch<T, 8, 5>(a, grid, lds, jac, lng, s);
     } else {
-        if (rpt == 2) res_launch<T, 2, 7>(a, grid, lds, jac, s);
-        else res_launch<T, 4, 7>(a, grid, lds, jac, s);
+        if (rpt == 2) res_launch<T, 2, 7>(a, grid, lds, jac, lng, s);
+        else res_launch<T, 4, 7>(a, grid, lds, jac, lng, s);
     }
     hipLaunchKernelGGL(k_res_out<T>, dim3(red_blocks(A->m)), dim3(kBlock), 0, s, (int64_t)A->m, (const T *)r, x,
                        (const KState<T> *)st);
@@ -187,7 +222,8 @@ int cg_resident(shk_ctx ctx, shk_csr A, const T *diag, T *x, T *r, void *zw, voi
     return SHK_OK;
 }
 template int cg_resident<double>(shk_ctx, shk_csr, const double *, double *, double *, void *, void *,
-                                 KState<double> *);
-template int cg_resident<float>(shk_ctx, shk_csr, const float *, float *, float *, void *, void *, KState<float> *);
+                                 KState<double> *, double *, bool);
+template int cg_resident<float>(shk_ctx, shk_csr, const float *, float *, float *, void *, void *, KState<float> *, float *,
+                                bool);
 
 }  // namespace shk

@@ -323,6 +323,8 @@ struct ResIter {
     int nb;               // iterations done
     int code;             // breakdown (0: none)
     T rho;                // (r, z) at the start
+    T rho_1;              // (r, z) of the iteration that head ended the loop after
+    const T *p;           // p to carry on from, by row
 };
 
 // halo elements per thread fetched while the sum before them is on its way
@@ -335,7 +337,9 @@ constexpr int kResBatch = 4;  // of those, in flight together
 // (which did not end it).  x[u], r[u] hold row m0 + (u NW + wave) 64 + lane.
 // Returns false when a wait ran out.  `head(nb, |r|^2)` runs after every
 // iteration on each thread alike and says whether Finished(r) ends the solve.
-template <typename T, int NT, int RPT, int KS, bool JAC, class Head>
+// LONG: with it.nb > 0 the loop goes on where another launch's head ended it,
+// from that x, r, p and it.
+template <typename T, int NT, int RPT, int KS, bool JAC, bool LONG, class Head>
 __device__ __forceinline__ bool res_cg(const ResRows &R, const T *val, const T *diag, T (&x)[RPT], T (&r)[RPT],
                                        const LlBuf &zw, T *win, ResIter<T> &it, ResTeam &t, ResShared<T> &sh,
                                        unsigned &zepoch, Head head)
@@ -381,6 +385,10 @@ __device__ __forceinline__ bool res_cg(const ResRows &R, const T *val, const T *
         if (t.k > 1 && (row >= R.m1 - R.left || row < R.m0 + R.right)) ll_put(zw, row * ll_words<T>(), z, zepoch);
     };
     T rho = it.rho, rho_1 = (T)1, beta = (T)0, z[RPT];
+    const bool carried = LONG && it.nb > 0;
+    if (LONG && carried) {
+        for (int i = tid; i < R.hi - R.lo; i += NT) win[i] = it.p[R.lo + i];
+    }
     zepoch++;
 #pragma unroll
     for (int u = 0; u < RPT; u++) {
@@ -432,7 +440,7 @@ __device__ __forceinline__ bool res_cg(const ResRows &R, const T *val, const T *
     T za[kResAhead];
 #pragma unroll
     for (int q = 0; q < kResAhead; q++) za[q] = (T)0;
-    if (JAC) {  // rho = (r, z)
+    if (JAC || (LONG && carried)) {  // rho = (r, z), summed as below
         T c[1] = {(T)0};
 #pragma unroll
         for (int u = 0; u < RPT; u++) c[0] += r[u] * z[u];
@@ -444,6 +452,7 @@ __device__ __forceinline__ bool res_cg(const ResRows &R, const T *val, const T *
             it.code = 1;
             return ok;
         }
+        if (LONG && carried) beta = rho / it.rho_1;
     } else {
         fetch(za, 0);
     }
@@ -523,7 +532,10 @@ __device__ __forceinline__ bool res_cg(const ResRows &R, const T *val, const T *
         if (!ok) return false;
         rho_1 = rho;
         it.nb++;
-        if (head(it.nb, tot[0])) return true;
+        if (head(it.nb, tot[0])) {
+            if (LONG) it.rho_1 = rho_1;
+            return true;
+        }
         rho = tot[NV - 1];
         if (rho == (T)0) {
             it.code = 1;

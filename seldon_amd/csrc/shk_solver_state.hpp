@@ -21,8 +21,10 @@ struct KState {
     int skip;          // done, or (GMRES) the current cycle is over
     int stop_slot;     // TfQmr: half step that ended the solve
     int bi_nb, bi_stop;  // BiCgStab: iterations at Finished(s), which ended the solve
-    // resident Cg: a member's wait ran out / the solve ran to its end
-    unsigned res_stall, res_ran;
+    // resident Cg: a member's wait ran out / the solve ran to its end / was left
+    // to be carried on
+    unsigned res_stall, res_ran, res_paused;
+    T *res_left;       // p and x of a solve left so
     double *hist;
     int *hist_it;
     // Cg / BiCgStab scalars, typed like Seldon's `Complexe` (= value type)

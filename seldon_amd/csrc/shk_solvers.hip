@@ -2475,11 +2475,14 @@ struct Solve {
 constexpr int kChunk = 16;
 
 // one solve on chip (shk_resident.hip): whether the matrix fits, and the
-// launches after the first Finished(r); zw holds 2 n values, slot the partials
+// launches after the first Finished(r), or (carry) after the launches that left
+// it paused with p and x in `pause` (2 n values; null: no launch leaves it); zw
+// holds 2 n values, slot the partials
 bool cg_resident_fits(shk_csr A);
 int cg_resident_groups(shk_csr A);
 template <typename T>
-int cg_resident(shk_ctx ctx, shk_csr A, const T *diag, T *x, T *r, void *zw, void *slot, KState<T> *st);
+int cg_resident(shk_ctx ctx, shk_csr A, const T *diag, T *x, T *r, void *zw, void *slot, KState<T> *st, T *pause,
+                bool carry);
 
 template <typename T>
 int cg_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration *it, int *code,
@@ -2489,9 +2492,11 @@ int cg_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration *i
     S.ext = ext;
     S.ext_cap = ext_cap;
     const bool jac = prec == SHK_PREC_JACOBI;
-    SHK_TRY(S.setup(ctx, A, jac ? 4 : 3, 0, it));
+    resident = resident && may_wait(ctx) && cg_resident_fits(A);
+    const bool leave = resident && !ext && it->max_iter > ctx->opt[SHK_OPT_CG_ITERS];
+    SHK_TRY(S.setup(ctx, A, (jac ? 4 : 3) + (leave ? 2 : 0), 0, it));
     const int64_t n = S.n;
-    T *p = S.take(n), *q = S.take(n), *r = S.take(n), *z = jac ? S.take(n) : r;
+    T *p = S.take(n), *q = S.take(n), *r = S.take(n), *z = jac ? S.take(n) : r, *pause = leave ? S.take(2 * n) : nullptr;
     hipStream_t st = ctx->stream;
     dim3 g(S.nb), blk(kBlock);
     // Init(b) (Cg.cxx:58)
@@ -2512,11 +2517,14 @@ int cg_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration *i
     }
     SHK_HIP(hipGetLastError());
     const T *dg = (const T *)A->diag;
-    if (resident && may_wait(ctx) && cg_resident_fits(A)) {
+    if (resident) {
         Seats seats(ctx);
-        seats.take(cg_resident_groups(A));
-        SHK_TRY(cg_resident<T>(ctx, A, jac ? dg : nullptr, x, r, p, S.partials, S.dst));
-        SHK_TRY(S.read_state());
+        for (bool carry = false; !carry || S.hst->res_paused; carry = true) {
+            seats.take(cg_resident_groups(A));
+            SHK_TRY(cg_resident<T>(ctx, A, jac ? dg : nullptr, x, r, p, S.partials, S.dst, pause, carry));
+            SHK_TRY(S.read_state());
+        }
+        seats.give();
         if (!S.hst->res_stall) {
             if (S.hst->res_ran) ctx->count[SHK_COUNT_CG_ON_CHIP]++;
             return S.finish(it, code);

@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 @pytest.fixture
 def ctx(gpu):
     yield gpu
-    for name, value in (("on_chip", 1), ("wait_us", -1), ("buffer_bytes", 2**31 - 1)):
+    for name, value in (("on_chip", 1), ("wait_us", -1), ("buffer_bytes", 2**31 - 1), ("cg_iters", 1 << 15)):
         gpu.set_option(name, value)
 
 
@@ -158,11 +158,82 @@ def test_batched_stall_is_an_error(ctx):
 
 def test_options_refuse_what_they_cannot_be(ctx):
     from seldon_amd import _lib as L
-    for name, bad in (("on_chip", 2), ("wait_us", -2), ("buffer_bytes", 2**31)):
+    for name, bad in (("on_chip", 2), ("wait_us", -2), ("buffer_bytes", 2**31), ("cg_iters", 0)):
         with pytest.raises(L.ShkError):
             ctx.set_option(name, bad)
     lib = L.load()
     assert lib.shk_ctx_set_option(ctx.h, 99, 0) == -1 and lib.shk_ctx_counter(ctx.h, 99, None) == -1
+
+
+@pytest.mark.parametrize("name", ["one_member_odd", "band_wider_than_share", "four_rows_per_thread",
+                                  "eight_rows_per_thread", "seven_steps", "seven_steps_four_rows"])
+@pytest.mark.parametrize("prec", ["identity", "jacobi"])
+def test_cg_left_and_carried_on(ctx, name, prec):
+    """Launches of 1, 7 and 64 iterations give the bits of one launch."""
+    from tests.test_gpu_resident import MATRICES, _solve
+    A = MATRICES[name]()
+    b = wl.apply(A, wl.uniform(A.m, 11))
+    for dtype, x0 in ((torch.float64, None), (torch.float32, wl.uniform(A.m, 12))):
+        runs = []
+        for iters in (1 << 15, 1, 7, 64):
+            ctx.set_option("cg_iters", iters)
+            n0 = ctx.counter("cg_on_chip")
+            code, it, x = _solve(A, b, "row", dtype, prec, x0, max_iter=130)
+            assert ctx.counter("cg_on_chip") == n0 + 1
+            runs.append((code, it.nb_iter, it.history.copy(), x))
+        for run in runs[1:]:
+            for a, c in zip(run, runs[0]):
+                assert np.array_equal(a, c), (dtype, iters)
+
+
+def test_long_cg_gives_way(ctx):
+    """A solve that fills the GPU for a long time is left now and then: a
+    short one of another thread, which needs its place, ends long before it."""
+    import threading
+    import time
+
+    from seldon_amd import krylov as K
+    A, S = wl.laplace2d(1000, 490), wl.laplace2d(128, 128)  # 240 and 16 work-groups
+    ctxs = [K.Context(0) for _ in range(2)]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    for c, s in zip(ctxs, streams):
+        c.bind_stream(s)
+    ctxs[0].set_option("cg_iters", 2048)
+    Ag, Sg = K.Matrix(A, ctx=ctxs[0]), K.Matrix(S, ctx=ctxs[1])
+    ab = torch.full((A.m,), float("nan"), dtype=torch.float64, device="cuda")
+    sb = torch.tensor(wl.uniform(S.m, 2), device="cuda")
+    ax, sx = torch.zeros_like(ab), torch.zeros_like(sb)
+
+    def solve(Mg, x, b, max_iter):
+        it = K.Iteration(max_iter, 1e-6)
+        it.HideMessages()
+        it.SetInitGuess(True)
+        return K.Cg(Mg, x, b, K.Preconditioner_Base(), it)
+
+    solve(Sg, sx, sb, 2000)
+    torch.cuda.synchronize()
+    spans = []
+
+    def run():
+        t = time.perf_counter()
+        solve(Ag, ax, ab, 200000)  # about a second
+        spans.append((t, time.perf_counter()))
+
+    th = threading.Thread(target=run)
+    th.start()
+    time.sleep(0.1)
+    for _ in range(3):
+        solve(Sg, sx, sb, 2000)
+    ended = time.perf_counter()
+    th.join()
+    torch.cuda.synchronize()
+    print("long solve", spans[0][1] - spans[0][0], "short ones ended before it by", spans[0][1] - ended, flush=True)
+    assert spans[0][1] - spans[0][0] > 0.5
+    assert ended < spans[0][1] - 0.2
+    assert ctxs[0].counter("started_over") == ctxs[1].counter("started_over") == 0
+    for c in ctxs:
+        c.synchronize()
+        c.bind_stream()
 
 
 def test_a_wait_that_ran_out_is_remembered(ctx):

@@ -107,7 +107,11 @@ typedef enum {
                                 20); 0 gives up after a look or two */
     SHK_OPT_BUFFER_BYTES = 2, /* SOR: values exchanged through 32-bit offsets up to so many bytes (default
                                 2^31 - 1), through 64-bit addresses past them */
-    SHK_OPT_CG_ITERS = 3     /* iterations that one launch of a Cg held on chip does (default 32768) */
+    SHK_OPT_CG_ITERS = 3,    /* iterations that one launch of a Cg held on chip does (default 32768) */
+    SHK_OPT_SPARE_BYTES = 4  /* most device memory for one copy or workspace that a call can do without (default
+                                no limit): the SpMV copy of a stencil, what the kernels above need beyond the
+                                others, the buckets of an assembly.  Past it, and where the device has no more,
+                                the call takes the way that does without */
 } shk_option;
 int shk_ctx_set_option(shk_ctx ctx, int option, int64_t value);
 /* What the context's calls did since it was created (synchronises). */

@@ -474,10 +474,7 @@ static int coo_buckets(shk_ctx ctx, int64_t nnz, const int *row, const int *col,
     // the count's table is read before the keys are written over it
     const size_t table_bytes = sizeof(int) * (size_t)groups * nb;
     const size_t big = std::max(kb * (twice ? 2 : 1) + vb, al(table_bytes));
-    if (ensure_ws2(ctx, big + 3 * bb + 3 * pb) != SHK_OK) {
-        (void)hipGetLastError();
-        return SHK_OK;
-    }
+    if (!spare_ws2(ctx, big + 3 * bb + 3 * pb)) return SHK_OK;
     char *w = (char *)ctx->ws2;
     uint64_t *key = (uint64_t *)w, *key0 = (uint64_t *)(w + kb + vb);
     T *v = (T *)(w + kb);

@@ -736,7 +736,7 @@ static int launch_batch(shk_ctx ctx, hipStream_t st, int use_graph, Enqueue enqu
 }
 
 // The batch on chip; *solved = false when a system does not fit (irregular,
-// too wide a band, too many rows): nothing has been written then.
+// too wide a band, too many rows, no memory): nothing has been written then.
 static int batched_resident(shk_ctx ctx, shk_csr A, int count, const int *row_off_host, const std::vector<int> &sizes,
                             double *x, const double *b, double tol, int max_iter, int use_graph, int *its, int *codes,
                             bool *solved)
@@ -783,7 +783,7 @@ static int batched_resident(shk_ctx ctx, shk_csr A, int count, const int *row_of
         d_val = (double *)take(sizeof(double) * kBrSteps * kWave * (size_t)nslice);
     };
     lay();
-    SHK_TRY(ensure_ws2(ctx, used));
+    if (!spare_ws2(ctx, used)) return SHK_OK;
     base = (char *)ctx->ws2;
     lay();
     const size_t head_bytes = (size_t)((char *)d_band - (char *)d_flag) + sizeof(int2) * (size_t)count;

@@ -38,8 +38,10 @@ int ensure_ws(shk_ctx ctx, size_t bytes)
         ctx->ws_cap = 0;
     }
     hipError_t e = hipMalloc(&ctx->ws, bytes);
-    if (e != hipSuccess)
+    if (e != hipSuccess) {
+        (void)hipGetLastError();  // not left for a caller that does with less
         return fail(SHK_ERR_NOMEM, std::string("solver workspace: ") + hipGetErrorString(e));
+    }
     ctx->ws_cap = bytes;
     return SHK_OK;
 }
@@ -54,10 +56,28 @@ int ensure_ws2(shk_ctx ctx, size_t bytes)
         ctx->ws2_cap = 0;
     }
     hipError_t e = hipMalloc(&ctx->ws2, bytes);
-    if (e != hipSuccess)
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
         return fail(SHK_ERR_NOMEM, std::string("refinement workspace: ") + hipGetErrorString(e));
+    }
     ctx->ws2_cap = bytes;
     return SHK_OK;
+}
+
+hipError_t spare_malloc(shk_ctx ctx, void **p, size_t bytes)
+{
+    const hipError_t e = may_spare(ctx, bytes) ? hipMalloc(p, bytes) : hipErrorOutOfMemory;
+    if (e != hipSuccess) {
+        *p = nullptr;
+        (void)hipGetLastError();
+    }
+    return e;
+}
+
+bool spare_ws2(shk_ctx ctx, size_t bytes)
+{
+    if (!may_spare(ctx, bytes)) return false;
+    return ensure_ws2(ctx, bytes) == SHK_OK;
 }
 
 int wait_ticks(shk_ctx ctx, long long seconds, long long *ticks)
@@ -235,6 +255,7 @@ int shk_ctx_set_option(shk_ctx c, int option, int64_t value)
     if (option == SHK_OPT_ON_CHIP) ok = value == 0 || value == 1;
     else if (option == SHK_OPT_WAIT_US) ok = value >= -1 && value <= 3600LL * 1000000;
     else if (option == SHK_OPT_BUFFER_BYTES) ok = value >= 0 && value <= INT32_MAX;
+    else if (option == SHK_OPT_SPARE_BYTES) ok = value >= 0;
     else if (option == SHK_OPT_CG_ITERS) ok = value >= 1 && value <= INT32_MAX;
     SHK_CHECK(ok, SHK_ERR_ARG, "shk_ctx_set_option: unknown option or value out of range");
     c->opt[option] = value;

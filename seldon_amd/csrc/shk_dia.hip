@@ -103,8 +103,10 @@ int dia_build(shk_csr A, const int *ptr, const int *mid, const uint32_t *ind, co
     const int slices = (A->m + kWave - 1) / kWave;
     const dim3 grid((slices + kDiaWaves - 1) / kDiaWaves), blk(kBlock);
     int *flag = nullptr, h[4] = {0, 0, 0, 0};
-    SHK_HIP(hipMalloc(&flag, sizeof(h)));
-    hipError_t e = hipMemcpyAsync(flag, h, sizeof(h), hipMemcpyHostToDevice, s);
+    hipError_t e = spare_malloc(A->ctx, (void **)&flag, sizeof(h));
+    if (e == hipErrorOutOfMemory) return SHK_OK;
+    SHK_HIP(e);
+    e = hipMemcpyAsync(flag, h, sizeof(h), hipMemcpyHostToDevice, s);
     if (e == hipSuccess) {
         hipLaunchKernelGGL(k_dia_build, grid, blk, 0, s, A->m, ptr, mid, ind, 0, (DiaStep *)nullptr, (int *)nullptr,
                            flag, false);
@@ -120,9 +122,14 @@ int dia_build(shk_csr A, const int *ptr, const int *mid, const uint32_t *ind, co
     A->dia_right = h[3];
     A->dia_block = slices <= 4096 ? kBlock : 1024;
     A->dia_groups = (int)(((int64_t)slices * kWave + A->dia_block - 1) / A->dia_block);
-    SHK_HIP(hipMalloc(&A->dia_step, sizeof(DiaStep) * (size_t)slices * h[0]));
-    SHK_HIP(hipMalloc((void **)&A->dia_src, sizeof(int) * (size_t)slots));
-    SHK_HIP(hipMalloc(&A->dia_val, dsize(A->dtype) * (size_t)slots));
+    e = spare_malloc(A->ctx, &A->dia_step, sizeof(DiaStep) * (size_t)slices * h[0]);
+    if (e == hipSuccess) e = spare_malloc(A->ctx, (void **)&A->dia_src, sizeof(int) * (size_t)slots);
+    if (e == hipSuccess) e = spare_malloc(A->ctx, &A->dia_val, dsize(A->dtype) * (size_t)slots);
+    if (e == hipErrorOutOfMemory) {  // the layout already there serves
+        dia_free(A);
+        return SHK_OK;
+    }
+    SHK_HIP(e);
     hipLaunchKernelGGL(k_dia_build, grid, blk, 0, s, A->m, ptr, mid, ind, h[0], (DiaStep *)A->dia_step, A->dia_src,
                        (int *)nullptr, true);
     if (src_of)

@@ -86,7 +86,7 @@ struct shk_ctx_s {
     size_t ws2_cap = 0;
     // shk_ctx_set_option, shk_ctx_counter (SHK_COUNT_SOR_RESCUED is on the
     // device: red.ticket[kRescuedSlot])
-    int64_t opt[4] = {1, -1, INT32_MAX, 1 << 15};
+    int64_t opt[5] = {1, -1, INT32_MAX, 1 << 15, INT64_MAX};
     int64_t count[4] = {0, 0, 0, 0};
     // after a wait that ran out, Cg and Gmres take the kernels without waits
     // until then (a shared GPU is paid for once, not on every solve)
@@ -303,6 +303,11 @@ int ensure_ws(shk_ctx ctx, size_t bytes);
 template <typename T>
 int stored_arrays(shk_csr A, std::vector<int> &ptr, std::vector<int> &ind, std::vector<T> &val);
 int ensure_ws2(shk_ctx ctx, size_t bytes);
+// Memory that a call can do without: false (hipErrorOutOfMemory) where there
+// is none, or SHK_OPT_SPARE_BYTES says so, and no error is left behind.
+hipError_t spare_malloc(shk_ctx ctx, void **p, size_t bytes);
+inline bool may_spare(shk_ctx ctx, size_t bytes) { return (int64_t)bytes <= ctx->opt[SHK_OPT_SPARE_BYTES]; }
+bool spare_ws2(shk_ctx ctx, size_t bytes);
 // device address of shk_cg_noalloc's fixed scratch array, looked up once per
 // device with that device current (shk_solvers.hip)
 int noalloc_scratch_init(int device);

@@ -2493,8 +2493,15 @@ int cg_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration *i
     S.ext_cap = ext_cap;
     const bool jac = prec == SHK_PREC_JACOBI;
     resident = resident && may_wait(ctx) && cg_resident_fits(A);
-    const bool leave = resident && !ext && it->max_iter > ctx->opt[SHK_OPT_CG_ITERS];
-    SHK_TRY(S.setup(ctx, A, (jac ? 4 : 3) + (leave ? 2 : 0), 0, it));
+    bool leave = resident && !ext && it->max_iter > ctx->opt[SHK_OPT_CG_ITERS];
+    int st0 = SHK_ERR_NOMEM;
+    if (!leave || may_spare(ctx, 2 * sizeof(T) * (size_t)A->m))
+        st0 = S.setup(ctx, A, (jac ? 4 : 3) + (leave ? 2 : 0), 0, it);
+    if (st0 == SHK_ERR_NOMEM && leave) {  // the launched kernels do with less
+        resident = leave = false;
+        st0 = S.setup(ctx, A, jac ? 4 : 3, 0, it);
+    }
+    SHK_TRY(st0);
     const int64_t n = S.n;
     T *p = S.take(n), *q = S.take(n), *r = S.take(n), *z = jac ? S.take(n) : r, *pause = leave ? S.take(2 * n) : nullptr;
     hipStream_t st = ctx->stream;
@@ -2653,15 +2660,26 @@ int gmres_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration
     const size_t small = sizeof(double) * ((size_t)(m + 1) * (m + 1) + 3 * (size_t)(m + 1)) + 1024;
     // columns of V at a stride of whole 256-byte lines (16-byte accesses for
     // every n)
-    const int64_t ldv = ((int64_t)A->m + 31) & ~(int64_t)31;
+    int64_t ldv = ((int64_t)A->m + 31) & ~(int64_t)31;
     resident = resident && may_wait(ctx) && gm_ortho_fits<T>(ctx, ldv, m);
-    const bool keep_x = resident && !it->init_guess_null;  // to start over from
-    SHK_TRY(S.setup(ctx, A, (size_t)m + 4 + (keep_x ? 1 : 0), small + 8 * gm_ortho_words() + 256 * (size_t)(m + 2), it));
+    bool keep_x = resident && !it->init_guess_null;  // to start over from
+    // what the kernel that waits takes beyond the others: its words, the
+    // columns' padding and the kept x
+    const size_t words = 8 * gm_ortho_words();
+    const size_t more = words + 256 * (size_t)(m + 2) + (keep_x ? sizeof(T) * (size_t)ldv : 0);
+    int st0 = SHK_ERR_NOMEM;
+    if (resident && may_spare(ctx, more)) st0 = S.setup(ctx, A, (size_t)m + 3, small + more, it);
+    if (st0 == SHK_ERR_NOMEM) {
+        resident = keep_x = false;
+        ldv = A->m;
+        st0 = S.setup(ctx, A, (size_t)m + 3, small, it);
+    }
+    SHK_TRY(st0);
     const int64_t n = S.n;
     T *V = S.take(ldv * (int64_t)(m + 1));
     T *w = S.take(ldv), *r = S.take(n);
     double *H = (double *)S.take((int64_t)((small + sizeof(T) - 1) / sizeof(T)));
-    T *slot = S.take((int64_t)(8 * gm_ortho_words() / sizeof(T)));
+    T *slot = resident ? S.take((int64_t)(words / sizeof(T))) : nullptr;
     T *x0 = keep_x ? S.take(n) : nullptr;
     double *gs = H + (size_t)(m + 1) * (m + 1), *gc = gs + (m + 1), *gsn = gc + (m + 1);
     SHK_HIP(hipMemsetAsync(H, 0, small, ctx->stream));

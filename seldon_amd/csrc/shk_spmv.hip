@@ -486,7 +486,8 @@ static bool dia_plausible(int m, const HostPlan &P)
            (double)(steps * kWave) <= 2 * kDiaFill * (double)entries + (double)kDiaSlack;
 }
 
-// The diagonal-slice copy of a matrix just uploaded, where it applies:
+// The diagonal-slice copy of a matrix just uploaded, where it applies and
+// there is memory for it:
 // columns, expanded positions and the caller's values go up once more for
 // the build, what the layout above already holds is read in place.
 template <typename T>
@@ -499,7 +500,7 @@ static int dia_upload(shk_csr A, const HostPlan &P, const T *val_host)
     T *val = nullptr;
     hipError_t e = hipSuccess;
     auto put = [&](auto **dst, const auto *src, size_t n) {
-        if (e == hipSuccess) e = hipMalloc((void **)dst, sizeof(*src) * std::max<size_t>(n, 1));
+        if (e == hipSuccess) e = spare_malloc(A->ctx, (void **)dst, sizeof(*src) * std::max<size_t>(n, 1));
         if (e == hipSuccess) e = hipMemcpyAsync(*dst, src, sizeof(*src) * n, hipMemcpyHostToDevice, s);
     };
     if (own_ind) put(&ind, P.ind.data(), P.ind.size());
@@ -516,6 +517,10 @@ static int dia_upload(shk_csr A, const HostPlan &P, const T *val_host)
     hipFree(ind);
     hipFree(src_of);
     hipFree(val);
+    if (st == SHK_OK && e == hipErrorOutOfMemory) {
+        dia_free(A);
+        return SHK_OK;
+    }
     if (st == SHK_OK) SHK_HIP(e);
     return st;
 }

@@ -54,7 +54,7 @@ class Context:
         L.check(L.load().shk_ctx_device_info(self.h, ctypes.byref(cus), ctypes.byref(xcds), arch, 64))
         return dict(cus=cus.value, xcds=xcds.value, arch=arch.value.decode())
 
-    OPTIONS = {"on_chip": 0, "wait_us": 1, "buffer_bytes": 2, "cg_iters": 3}
+    OPTIONS = {"on_chip": 0, "wait_us": 1, "buffer_bytes": 2, "cg_iters": 3, "spare_bytes": 4}
     COUNTERS = {"cg_on_chip": 0, "gmres_on_chip": 1, "batch_on_chip": 2, "started_over": 3, "sor_rescued": 4}
 
     def set_option(self, name: str, value: int):

@@ -25,7 +25,7 @@ def _counts(ctx, *names):
 
 def _cg(A, b, x0, prec, max_iter=60):
     from seldon_amd import krylov as K
-    Ag, bg = K.Matrix(A), torch.tensor(b, device="cuda")
+    Ag, bg = A if isinstance(A, K.Matrix) else K.Matrix(A), torch.tensor(b, device="cuda")
     x = torch.full_like(bg, 7.0) if x0 is None else torch.tensor(x0, device="cuda")
     it = K.Iteration(max_iter, 1e-10)
     it.HideMessages()
@@ -59,7 +59,7 @@ def test_cg_starts_over(ctx, prec, guess):
 
 def _gmres(A, b, x0, restart, max_iter=14):
     from seldon_amd import krylov as K
-    Ag, bg = K.Matrix(A), torch.tensor(b, device="cuda")
+    Ag, bg = A if isinstance(A, K.Matrix) else K.Matrix(A), torch.tensor(b, device="cuda")
     x = torch.full_like(bg, 7.0) if x0 is None else torch.tensor(x0, device="cuda")
     it = K.Iteration(max_iter, 1e-8)
     it.SetRestart(restart)

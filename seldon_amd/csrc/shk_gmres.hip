@@ -138,21 +138,15 @@ __global__ __launch_bounds__(kGoThreads, 2) void k_gm_ortho(GmOrtho<T> a)
     if (!res_wait<T, 1, kGoThreads>(c, t, sh)) return;
     double hi = (double)sqrt_t(c[0]);
     const T scale = hi != 0.0 ? (T)(1.0 / hi) : (T)1;
-    const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(a.vnext, (short)0, bytes, 0x00020000);
-    // scaled in place first: a store's data registers are not written again
-    // while it may still be reading them (the compiler places no wait between
-    // a 16-byte buffer store with a register offset and the next write of its
-    // data, and V_{i+1} came out wrong now and then where it reused them)
+    // ordinary stores under a bounds test: what may follow a 16-byte store is
+    // the compiler's to arrange (buffer stores whose offset was in a register
+    // got no wait before the next write to their data, and V_{i+1} came out
+    // wrong now and then where the registers were used again)
 #pragma unroll
-    for (int q = 0; q < NV; q++)
-#pragma unroll
-        for (int e = 0; e < N; e++) w[q][e] = w[q][e] * scale;
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int q = 0; q < NV; q++)
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(ll_u4, w[q]), out, at, q * kGoThreads * 16, 0);
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+    for (int q = 0; q < NV; q++) {
+        const int o = at + q * kGoThreads * 16;
+        if (o < bytes) *(Vec *)((char *)a.vnext + o) = w[q] * scale;
+    }
     if (!lead) return;
     // FinGmStep's end of step on the LDS column (Gmres.cxx:135-162)
     if (tid == 0) {

@@ -726,7 +726,11 @@ namespace shk {
 
 // ------------------------------------------------------------ launch ----
 // work-groups an SpMV of A may launch (partials per fused dot)
-inline int spmv_partials(shk_csr A) { return A->dia_val ? dia_grid(A) : A->nblk_launch; }
+inline int spmv_partials(shk_csr A)
+{
+    if (A->dia_val) return dia_grid(A);
+    return A->layout == SHK_LAYOUT_SLICED ? A->sl_launch : A->nblk_launch;
+}
 
 template <typename T, typename Fin>
 inline int launch_spmv(shk_csr A, SpmvArgs<T> &a, Fin fin)

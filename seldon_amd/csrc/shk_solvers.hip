@@ -2333,6 +2333,7 @@ struct Solve {
     double *dhist = nullptr;
     int *dhist_it = nullptr;
     T *partials;
+    size_t maxb;            // work-groups a partial buffer of two values has room for
     T *part[3];             // partial buffers: two alternating pairs (Gmres's folded finishes) and one of
                             // six values (QCgs's smoothing step)
     char *ws;
@@ -2349,7 +2350,9 @@ struct Solve {
         return p;
     }
 
-    int setup(shk_ctx c, shk_csr a, size_t vec_count, size_t extra_bytes, const shk_iteration *it)
+    // at: another matrix (A^T) whose products leave partials here
+    int setup(shk_ctx c, shk_csr a, size_t vec_count, size_t extra_bytes, const shk_iteration *it,
+              shk_csr at = nullptr)
     {
         ctx = c;
         A = a;
@@ -2362,7 +2365,7 @@ struct Solve {
         size_t vb = (((size_t)n * sizeof(T) + 255) & ~(size_t)255);
         size_t hist_cap = it->hist && it->hist_cap > 0 ? (size_t)it->hist_cap : 0;
         size_t need = vec_count * vb + extra_bytes + 256 + hist_cap * (sizeof(double) + sizeof(int)) + 512;
-        const size_t maxb = (size_t)std::max(nb, spmv_partials(a));
+        maxb = (size_t)std::max({nb, spmv_partials(a), at ? spmv_partials(at) : 0});
         const size_t red = sizeof(T) * 10 * maxb;  // two buffers of [2][maxb], one of [6][maxb]
         if (ext) {
             need = (need + 255) & ~(size_t)255;
@@ -2443,7 +2446,16 @@ struct Solve {
     template <typename Fin>
     int spmv(SpmvArgs<T> &a, Fin fin)
     {
-        return launch_spmv<T, Fin>(A, a, fin);
+        return spmv_of(A, a, fin);
+    }
+
+    // the product of another matrix (A^T) with this solve's partial buffers
+    template <typename Fin>
+    int spmv_of(shk_csr M, SpmvArgs<T> &a, Fin fin)
+    {
+        SHK_CHECK(!a.partials || (size_t)spmv_partials(M) <= maxb, SHK_ERR_STATE,
+                  "solver: partial buffer smaller than the product's grid");
+        return launch_spmv<T, Fin>(M, a, fin);
     }
 
     // The iteration loop: body(stream, count) enqueues one chunk of count
@@ -2879,7 +2891,7 @@ int bicg_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration 
             SHK_TRY(S.spmv(a, FinDefer{}));  // delta: finished inside k_bicg_xr
             SpmvArgs<T> a2{};
             a2.x = pt; a2.y_out = qt; a2.alpha = (T)1; a2.mlt = 1; a2.skip = &S.dst->skip;
-            SHK_TRY((launch_spmv<T, FinNone>(At, a2, FinNone{})));
+            SHK_TRY(S.spmv_of(At, a2, FinNone{}));
             hipLaunchKernelGGL(k_bicg_xr<T>, g, blk, 0, cs, n, p, q, qt, x, r, rt, dg, z, zt, S.dst,
                                (const T *)S.part[0], a.grid_used, S.partials);
             S.fin(FinLanczosTop<T>{S.dst, 1});
@@ -2999,7 +3011,7 @@ int qmr_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration *
             hipLaunchKernelGGL(k_qmr_vy<T>, g, blk, 0, cs, n, pt, dg, v, y, S.dst);
             SpmvArgs<T> a2{};
             a2.x = q; a2.y_out = z; a2.alpha = (T)1; a2.mlt = 1; a2.skip = &S.dst->skip;
-            SHK_TRY((launch_spmv<T, FinNone>(At, a2, FinNone{})));
+            SHK_TRY(S.spmv_of(At, a2, FinNone{}));
             hipLaunchKernelGGL(k_qmr_w<T>, g, blk, 0, cs, n, (const T *)z, (const T *)y, w, S.dst, S.partials);
             S.fin(FinQmrTheta<T>{S.dst});
             hipLaunchKernelGGL(k_qmr_dsxr<T>, g, blk, 0, cs, n, p, pt, d, s, x, r, S.dst, S.partials);
@@ -3022,7 +3034,7 @@ int cgne_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration 
     SHK_TRY(transpose_of(A, &At));
     Solve<T> S;
     const bool jac = prec == SHK_PREC_JACOBI;
-    SHK_TRY(S.setup(ctx, A, 4, 0, it));
+    SHK_TRY(S.setup(ctx, A, 4, 0, it, At));
     const int64_t n = S.n;
     T *p = S.take(n), *q = S.take(n), *r = S.take(n), *z = S.take(n);
     const T *dg = jac ? (const T *)A->diag : nullptr;
@@ -3031,7 +3043,7 @@ int cgne_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration 
     dim3 g(S.nb), blk(kBlock);
     SpmvArgs<T> a0{};
     a0.x = b; a0.y_out = q; a0.alpha = (T)1; a0.mlt = 1; a0.skip = &S.dst->skip;
-    SHK_TRY((launch_spmv<T, FinNone>(At, a0, FinNone{})));
+    SHK_TRY(S.spmv_of(At, a0, FinNone{}));
     hipLaunchKernelGGL(k_sumsq<T>, g, blk, 0, st, n, (const T *)q, S.dst, S.partials);
     S.fin(FinCgneInit<T>{S.dst});
     if (!it->init_guess_null) {
@@ -3040,7 +3052,7 @@ int cgne_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration 
         SHK_TRY(S.spmv(a, FinNone{}));
         SpmvArgs<T> a2{};
         a2.x = p; a2.y_out = r; a2.alpha = (T)1; a2.mlt = 1; a2.skip = &S.dst->skip;
-        SHK_TRY((launch_spmv<T, FinNone>(At, a2, FinNone{})));
+        SHK_TRY(S.spmv_of(At, a2, FinNone{}));
     }
     hipLaunchKernelGGL(k_cgne_r0<T>, g, blk, 0, st, n, (const T *)q, r, x, it->init_guess_null ? 1 : 0, S.dst);
     SHK_HIP(hipGetLastError());
@@ -3057,7 +3069,7 @@ int cgne_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration 
             a2.x = q; a2.y_out = z; a2.alpha = (T)1; a2.mlt = 1;
             a2.dot0 = kDotVec; a2.u0 = p; a2.skip = &S.dst->skip;
             a2.partials = S.part[1];
-            SHK_TRY((launch_spmv<T, FinDefer>(At, a2, FinDefer{})));
+            SHK_TRY(S.spmv_of(At, a2, FinDefer{}));
             grid_finish<T>(cs, (const T *)S.part[1], a2.grid_used, (const int *)&S.dst->skip,
                            FinCgneDelta<T>{S.dst});
             hipLaunchKernelGGL(k_cgne_xr<T>, g, blk, 0, cs, n, (const T *)p, (const T *)z, x, r, S.dst,
@@ -3082,7 +3094,7 @@ int lsqr_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, shk_iteration *it, int *
     shk_csr At = nullptr;
     SHK_TRY(transpose_of(A, &At));
     Solve<T> S;
-    SHK_TRY(S.setup(ctx, A, 5, 0, it));
+    SHK_TRY(S.setup(ctx, A, 5, 0, it, At));
     const int64_t n = S.n;
     T *u = S.take(n), *u1 = S.take(n), *v = S.take(n), *v1 = S.take(n), *w = S.take(n);
     hipStream_t st = ctx->stream;
@@ -3105,7 +3117,7 @@ int lsqr_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, shk_iteration *it, int *
         SpmvArgs<T> a{};
         a.x = u; a.y_out = v; a.alpha = (T)1; a.mlt = 1; a.dot0 = kDotSelf; a.skip = &S.dst->skip;
         a.partials = S.part[1];
-        SHK_TRY((launch_spmv<T, FinDefer>(At, a, FinDefer{})));
+        SHK_TRY(S.spmv_of(At, a, FinDefer{}));
         grid_finish<T>(st, (const T *)S.part[1], a.grid_used, (const int *)&S.dst->skip, FinLsqrStart<T>{S.dst});
     }
     hipLaunchKernelGGL(k_lsqr_v0<T>, g, blk, 0, st, n, v, w, S.dst);
@@ -3114,7 +3126,8 @@ int lsqr_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, shk_iteration *it, int *
     SHK_TRY(S.run_chunks(limit, kChunk, [&](hipStream_t cs, int count) -> int {
         for (int k = 0; k < count; k++) {
             // Swap(u1, u); Swap(v1, v) after every loop: even slots use the
-            // first assignment, odd ones the other (a chunk has an even count)
+            // first assignment, odd ones the other (only the last chunk may have
+            // an odd count)
             T *uc = (k & 1) ? u1 : u, *un = (k & 1) ? u : u1;
             T *vc = (k & 1) ? v1 : v, *vn = (k & 1) ? v : v1;
             SpmvArgs<T> a{};
@@ -3125,7 +3138,7 @@ int lsqr_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, shk_iteration *it, int *
             hipLaunchKernelGGL(k_lsqr_scale<T>, g, blk, 0, cs, n, un, S.dst);
             SpmvArgs<T> a2{};
             a2.x = un; a2.y_out = vn; a2.alpha = (T)1; a2.mlt = 1; a2.skip = &S.dst->skip;
-            SHK_TRY((launch_spmv<T, FinNone>(At, a2, FinNone{})));
+            SHK_TRY(S.spmv_of(At, a2, FinNone{}));
             hipLaunchKernelGGL(k_lsqr_sub<T>, g, blk, 0, cs, n, (const T *)vc, vn, 1, S.dst, S.partials);
             S.fin(FinLsqrAlpha<T>{S.dst, k});
             hipLaunchKernelGGL(k_lsqr_xw<T>, g, blk, 0, cs, n, vn, w, x, S.dst, k);

@@ -110,3 +110,25 @@ def test_dia_leaves_other_matrices_alone(gpu, kind):
     yg = torch.empty(A.m, dtype=torch.float64, device="cuda")
     K.Mlt(K.Matrix(M), torch.tensor(x, device="cuda"), yg)
     assert _same(yg.cpu().numpy(), orc.mlt(M, x))
+
+
+@pytest.mark.parametrize("method", ["cgne", "lsqr"])
+@pytest.mark.parametrize("side", [512, 301])
+def test_transpose_with_a_larger_grid(gpu, method, side):
+    """A in the panel layout (128 work-groups at 512^2), A^T in diagonal
+    slices (1024): the solver's partial sums have room for either, and the
+    bits are those of a matrix that has the slices too."""
+    from seldon_amd import krylov as K
+    A = wl.laplace2d(side, side)
+    b = wl.apply(A, wl.uniform(A.m, 3))
+    bg = torch.tensor(b, device="cuda")
+    runs = []
+    for layout in ("panels", "auto"):
+        Ag = K.Matrix(A, layout=layout)
+        x = torch.zeros_like(bg)
+        it = K.Iteration(30, 1e-12)
+        it.HideMessages()
+        code = (K.Cgne if method == "cgne" else K.Lsqr)(Ag, x, bg, K.Preconditioner_Base(), it)
+        runs.append((code, it.nb_iter, it.history.copy(), x.cpu().numpy()))
+    for a, c in zip(*runs):
+        assert np.array_equal(a, c)

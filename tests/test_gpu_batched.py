@@ -1,6 +1,8 @@
 """Batched persistent Cg: every system against the oracle's Cg (Seldon's
 recurrences), graph and stream launches identical, and the FP32+FP64
-refinement variant to the FP64 tolerance."""
+refinement variant to the FP64 tolerance.  Stencil batches are solved on chip
+(work-group size and rows per pass do not apply); batches of permuted, reversed
+or longer rows take the streaming kernel, for which they do."""
 import numpy as np
 import pytest
 import torch
@@ -10,10 +12,46 @@ from seldon_amd import workloads as wl
 pytestmark = pytest.mark.gpu
 
 
-def _small_batch(count=24):
+def _permuted(S, seed):
+    """P S P^T with sorted columns: short rows without common offsets."""
+    order = np.random.default_rng(seed).permutation(S.m)
+    inv = np.argsort(order)
+    lens = np.diff(S.ptr)[order]
+    ptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    src = np.repeat(S.ptr[:-1][order] - ptr[:-1], lens) + np.arange(S.nnz)
+    rows, cols = np.repeat(np.arange(S.m), lens), inv[S.ind[src]]
+    by = np.lexsort((cols, rows))
+    return wl.CSR(S.m, S.n, ptr, cols[by].astype(np.int32), S.val[src][by])
+
+
+def _reversed(S):
+    """S with every row's entries in decreasing column order."""
+    src = np.repeat(S.ptr[1:] + S.ptr[:-1] - 1, np.diff(S.ptr)) - np.arange(S.nnz)
+    return wl.CSR(S.m, S.n, S.ptr, S.ind[src], S.val[src])
+
+
+def _wide(S, seed):
+    """A random symmetric diagonally dominant matrix of S's size, about 20
+    entries a row."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(seed)
+    R = sp.coo_matrix((rng.uniform(-1, 1, 10 * S.m), rng.integers(0, S.m, (2, 10 * S.m))), (S.m, S.m)).tocsr()
+    R = R + R.T
+    d = np.asarray(abs(R).sum(axis=1)).ravel()
+    A = (R + sp.diags(1.02 * d + 0.01)).tocsr()
+    A.sort_indices()
+    return wl.CSR(S.m, S.m, A.indptr.astype(np.int32), A.indices.astype(np.int32), A.data)
+
+
+def _as(kind, S, seed):
+    return {"stencil": lambda: S, "permuted": lambda: _permuted(S, seed), "reversed": lambda: _reversed(S),
+            "wide": lambda: _wide(S, seed)}[kind]()
+
+
+def _small_batch(count=24, kind="stencil"):
     from seldon_amd.batched import stack
     sides, eps = wl.batched_systems(count, 5, 8, 40)
-    systems = [wl.aniso2d(int(n), int(n), float(e)) for n, e in zip(sides, eps)]
+    systems = [_as(kind, wl.aniso2d(int(n), int(n), float(e)), s) for s, (n, e) in enumerate(zip(sides, eps))]
     A, row_off = stack(systems)
     xt = wl.uniform(A.m, 9)
     b = wl.apply(A, xt)
@@ -21,17 +59,23 @@ def _small_batch(count=24):
     return A, row_off, b, systems
 
 
+KINDS = ["stencil", "permuted", "reversed", "wide"]
+
+
+@pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("group,rpp", [(64, 1), (256, 4), (512, 2), (1024, 8)])
-def test_batched_matches_oracle_per_system(gpu, group, rpp):
+def test_batched_matches_oracle_per_system(gpu, group, rpp, kind):
     from oracle import oracle as orc
     from seldon_amd import krylov as K
     from seldon_amd.batched import cg_batched
-    A, row_off, b, systems = _small_batch()
+    A, row_off, b, systems = _small_batch(kind=kind)
     Ag = K.Matrix(A, layout="rows")
     bg = torch.tensor(b, device="cuda")
     x = torch.full_like(bg, 7.0)
+    n0 = gpu.counter("batch_on_chip")
     its, codes = cg_batched(Ag, row_off, x, bg, tol=1e-8, max_iter=5000, group=group, use_graph=False,
                             rows_per_pass=rpp)
+    assert gpu.counter("batch_on_chip") - n0 == (kind == "stencil")
     xh = x.cpu().numpy()
     for s, S in enumerate(systems):
         sl = slice(row_off[s], row_off[s + 1])
@@ -44,10 +88,11 @@ def test_batched_matches_oracle_per_system(gpu, group, rpp):
             assert np.linalg.norm(xh[sl] - r.x) <= 1e-6 * np.linalg.norm(r.x)
 
 
-def test_batched_graph_equals_stream_and_max_iter(gpu):
+@pytest.mark.parametrize("kind", KINDS)
+def test_batched_graph_equals_stream_and_max_iter(gpu, kind):
     from seldon_amd import krylov as K
     from seldon_amd.batched import cg_batched
-    A, row_off, b, systems = _small_batch()
+    A, row_off, b, systems = _small_batch(kind=kind)
     Ag = K.Matrix(A, layout="rows")
     bg = torch.tensor(b, device="cuda")
     x1, x2 = torch.zeros_like(bg), torch.zeros_like(bg)
@@ -91,7 +136,7 @@ def test_batched_ir_reaches_fp64_tolerance(gpu, inner_tol):
 def test_autotune_picks_a_candidate(gpu):
     from seldon_amd import krylov as K
     from seldon_amd.batched import CANDIDATES, ROWS_PER_PASS, autotune
-    A, row_off, b, systems = _small_batch()
+    A, row_off, b, systems = _small_batch(kind="permuted")
     Ag = K.Matrix(A, layout="rows")
     bg = torch.tensor(b, device="cuda")
     (g, u), entry = autotune(Ag, row_off, bg, use_cache=False)
@@ -100,12 +145,13 @@ def test_autotune_picks_a_candidate(gpu):
     assert entry["seconds"][f"{g}x{u}"] == min(entry["seconds"].values())
 
 
-def test_batched_rows_per_pass_results_identical(gpu):
+@pytest.mark.parametrize("kind", KINDS)
+def test_batched_rows_per_pass_results_identical(gpu, kind):
     """Keeping more rows in flight per thread changes no arithmetic: the
     same iterations, codes and solutions, bit for bit, for every setting."""
     from seldon_amd import krylov as K
     from seldon_amd.batched import cg_batched, cg_batched_ir
-    A, row_off, b, systems = _small_batch()
+    A, row_off, b, systems = _small_batch(kind=kind)
     A64 = K.Matrix(A, layout="rows")
     A32 = K.Matrix(A, dtype=torch.float32, layout="rows")
     bg = torch.tensor(b, device="cuda")
@@ -141,16 +187,17 @@ def test_batched_rejects_a_column_in_another_system(gpu):
     assert torch.all(x == 3.0)
 
 
-def test_batched_one_large_system_on_a_team_of_sixteen(gpu):
+@pytest.mark.parametrize("kind", KINDS)
+def test_batched_one_large_system_on_a_team_of_sixteen(gpu, kind):
     """A batch of one 200 x 200 anisotropic Laplacian (40,000 rows): its share
-    of the work is all of it, so 16 work-groups solve it together (members
-    meeting in device memory, the dots added in member order) -- same
+    of the work is all of it, so 16 work-groups (on chip 40) solve it together
+    (members meeting in device memory, the dots added in member order) -- same
     iterations (within 1) and solution as the oracle's Cg, and the same
     result bit for bit on a second run (the team's sums have a fixed order)."""
     from oracle import oracle as orc
     from seldon_amd import krylov as K
     from seldon_amd.batched import cg_batched, cg_batched_ir, stack
-    S = wl.aniso2d(200, 200, 30.0)
+    S = _as(kind, wl.aniso2d(200, 200, 30.0), 7)
     A, row_off = stack([S])
     xt = wl.uniform(A.m, 17)
     b = wl.apply(A, xt)

@@ -145,6 +145,21 @@ def test_autotune_picks_a_candidate(gpu):
     assert entry["seconds"][f"{g}x{u}"] == min(entry["seconds"].values())
 
 
+def test_autotune_leaves_on_chip_batches_alone(gpu):
+    """One solve says that work-group size and rows per pass do not apply: the
+    defaults, nothing timed and nothing cached for a batch of the same sizes
+    that would be streamed."""
+    from seldon_amd import batched as B
+    from seldon_amd import krylov as K
+    A, row_off, b, systems = _small_batch()
+    Ag = K.Matrix(A, layout="rows")
+    n0 = gpu.counter("batch_on_chip")
+    choice, entry = B.autotune(Ag, row_off, torch.tensor(b, device="cuda"))
+    assert choice == (B.DEFAULT_GROUP, B.DEFAULT_ROWS) and entry["on_chip"] and not entry["seconds"]
+    assert gpu.counter("batch_on_chip") == n0 + 1
+    assert not B.os.path.exists(B.CACHE) or B._signature("fp64", Ag, row_off) not in open(B.CACHE).read()
+
+
 @pytest.mark.parametrize("kind", KINDS)
 def test_batched_rows_per_pass_results_identical(gpu, kind):
     """Keeping more rows in flight per thread changes no arithmetic: the

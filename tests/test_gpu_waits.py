@@ -136,24 +136,26 @@ def test_sor_rescue_and_wide_words(ctx, st, c, wide, rescue):
         assert ctx.counter("sor_rescued") - n0 == (sweeps if rescue and wait == 0 else 0)
 
 
-def test_batched_stall_is_an_error(ctx):
+@pytest.mark.parametrize("kind", ["stencil", "permuted"])
+def test_batched_stall_is_an_error(ctx, kind):
     """A team whose members wait too long: the call says so, and the next one
     solves; a batch of one-member teams waits for nobody."""
     from seldon_amd import _lib as L
     from seldon_amd import krylov as K
     from seldon_amd.batched import cg_batched, stack
-    A, row_off = stack([wl.aniso2d(100, 100, 3.0), wl.aniso2d(9, 9, 1.0)])
+    from tests.test_gpu_batched import _as
+    A, row_off = stack([_as(kind, wl.aniso2d(200, 200, 3.0), 1)])
     S, s_off = stack([wl.aniso2d(9, 9, 1.0), wl.aniso2d(12, 7, 1.0)])
     Ag, Sg = K.Matrix(A, layout="rows"), K.Matrix(S, layout="rows")
     bg, sg = torch.ones(A.m, dtype=torch.float64, device="cuda"), torch.ones(S.m, dtype=torch.float64, device="cuda")
     n0 = ctx.counter("batch_on_chip")
     ctx.set_option("wait_us", 0)
     with pytest.raises(L.ShkError, match="waited too long"):
-        cg_batched(Ag, row_off, torch.zeros_like(bg), bg)
+        cg_batched(Ag, row_off, torch.zeros_like(bg), bg, max_iter=50)
     assert np.all(cg_batched(Sg, s_off, torch.zeros_like(sg), sg)[1] == 0)
     ctx.set_option("wait_us", -1)
     assert np.all(cg_batched(Ag, row_off, torch.zeros_like(bg), bg)[1] == 0)
-    assert ctx.counter("batch_on_chip") == n0 + 2
+    assert ctx.counter("batch_on_chip") == n0 + (2 if kind == "stencil" else 1)
 
 
 def test_options_refuse_what_they_cannot_be(ctx):

@@ -120,7 +120,8 @@ typedef enum {
     SHK_COUNT_GMRES_ON_CHIP = 1, /* Gmres solves with the orthogonalisation in one kernel per step */
     SHK_COUNT_BATCH_ON_CHIP = 2, /* batched calls held on chip */
     SHK_COUNT_STARTED_OVER = 3,  /* Cg and Gmres solves started over after a wait ran out */
-    SHK_COUNT_SOR_RESCUED = 4    /* SOR sweeps left to one wavefront */
+    SHK_COUNT_SOR_RESCUED = 4,   /* SOR sweeps left to one wavefront */
+    SHK_COUNT_COO_BUCKETS = 5    /* conversions from coordinates through buckets, not the general sort */
 } shk_counter;
 int shk_ctx_counter(shk_ctx ctx, int counter, int64_t *value);
 

@@ -511,6 +511,7 @@ static int coo_buckets(shk_ctx ctx, int64_t nnz, const int *row, const int *col,
         hipLaunchKernelGGL((k_coo_bucket<T, 8192>), dim3(nb), dim3(kCooThreads), blds, st, m, pk,
                            (const int *)base, (const uint64_t *)key, (const T *)v, ptr, ind, val_out);
     SHK_HIP(hipGetLastError());
+    ctx->count[SHK_COUNT_COO_BUCKETS]++;
     *done = true;
     return SHK_OK;
 }

@@ -266,7 +266,7 @@ int shk_ctx_set_option(shk_ctx c, int option, int64_t value)
 int shk_ctx_counter(shk_ctx c, int counter, int64_t *value)
 {
     SHK_CHECK(c && value, SHK_ERR_ARG, "shk_ctx_counter: null argument");
-    SHK_CHECK(counter >= 0 && counter <= SHK_COUNT_SOR_RESCUED, SHK_ERR_ARG, "shk_ctx_counter: unknown counter");
+    SHK_CHECK(counter >= 0 && counter <= SHK_COUNT_COO_BUCKETS, SHK_ERR_ARG, "shk_ctx_counter: unknown counter");
     SHK_HIP(hipStreamSynchronize(c->stream));
     if (counter != SHK_COUNT_SOR_RESCUED) {
         *value = c->count[counter];

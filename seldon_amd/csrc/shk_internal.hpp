@@ -87,7 +87,7 @@ struct shk_ctx_s {
     // shk_ctx_set_option, shk_ctx_counter (SHK_COUNT_SOR_RESCUED is on the
     // device: red.ticket[kRescuedSlot])
     int64_t opt[5] = {1, -1, INT32_MAX, 1 << 15, INT64_MAX};
-    int64_t count[4] = {0, 0, 0, 0};
+    int64_t count[6] = {0, 0, 0, 0, 0, 0};
     // after a wait that ran out, Cg and Gmres take the kernels without waits
     // until then (a shared GPU is paid for once, not on every solve)
     std::chrono::steady_clock::time_point no_waits_until{};

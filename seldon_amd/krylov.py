@@ -55,7 +55,8 @@ class Context:
         return dict(cus=cus.value, xcds=xcds.value, arch=arch.value.decode())
 
     OPTIONS = {"on_chip": 0, "wait_us": 1, "buffer_bytes": 2, "cg_iters": 3, "spare_bytes": 4}
-    COUNTERS = {"cg_on_chip": 0, "gmres_on_chip": 1, "batch_on_chip": 2, "started_over": 3, "sor_rescued": 4}
+    COUNTERS = {"cg_on_chip": 0, "gmres_on_chip": 1, "batch_on_chip": 2, "started_over": 3, "sor_rescued": 4,
+                "coo_buckets": 5}
 
     def set_option(self, name: str, value: int):
         L.check(L.load().shk_ctx_set_option(self.h, self.OPTIONS[name], int(value)))

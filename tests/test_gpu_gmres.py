@@ -37,6 +37,7 @@ def test_gmres_matches_oracle(gpu, m, restart):
     Ag, bg = K.Matrix(A), torch.tensor(b, device="cuda")
     ref = orc.solve("gmres", A, b, precond="jacobi", tol=1e-8, max_iter=14, restart=restart, x0=x0)
     runs = []
+    n0 = gpu.counter("gmres_on_chip")
     for _ in range(3):
         x = torch.full_like(bg, 7.0) if x0 is None else torch.tensor(x0, device="cuda")
         it = K.Iteration(14, 1e-8)
@@ -46,6 +47,7 @@ def test_gmres_matches_oracle(gpu, m, restart):
         code = K.Gmres(Ag, x, bg, K.JacobiPreconditioner(), it)
         runs.append((x.cpu().numpy(), it.history.copy()))
         assert (code, it.nb_iter, it.hist_len) == (ref.code, ref.nb_iter, len(ref.hist))
+    assert gpu.counter("gmres_on_chip") == n0 + 3
     for x, h in runs[1:]:
         assert np.array_equal(x, runs[0][0]) and np.array_equal(h, runs[0][1])
     # sums of up to 2M terms round by ~1e-13 of the vectors' norms; residuals
@@ -67,6 +69,7 @@ def test_gmres_f32(gpu, m):
     Ag = K.Matrix(A, dtype=torch.float32)
     bg = torch.tensor(b, device="cuda")
     out = []
+    n0 = gpu.counter("gmres_on_chip")
     for _ in range(2):
         x = torch.zeros_like(bg)
         it = K.Iteration(40, 1e-3)
@@ -75,6 +78,7 @@ def test_gmres_f32(gpu, m):
         assert K.Gmres(Ag, x, bg, K.JacobiPreconditioner(), it) == 0
         assert it.nb_iter <= 12
         out.append(x.cpu().numpy())
+    assert gpu.counter("gmres_on_chip") == n0 + 2
     assert np.array_equal(out[0], out[1])
     r = wl.apply(A, out[0].astype(np.float64)) - b
     assert np.linalg.norm(r) <= 3e-3 * np.linalg.norm(b)

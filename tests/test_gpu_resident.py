@@ -86,7 +86,9 @@ def test_resident_cg_matches_oracle(gpu, name, prec):
         x0 = wl.uniform(A.m, 12) if guess else None
         # 60 iterations, entry by entry: within ten times the oracle's own
         # spread under other orders of the dots' sums (never below 1e-12)
+        n0 = gpu.counter("cg_on_chip")
         code, it, x = _solve(M, b, storage, torch.float64, prec, x0, max_iter=60)
+        assert gpu.counter("cg_on_chip") == n0 + 1
         ref = orc.solve("cg", M, b, precond=PREC[prec], tol=1e-10, max_iter=60, x0=x0)
         assert (code, it.nb_iter, it.hist_len) == (ref.code, ref.nb_iter, len(ref.hist))
         full = orc.solve("cg", A, b, precond=PREC[prec], tol=1e-10, max_iter=60, x0=x0)
@@ -100,7 +102,9 @@ def test_resident_cg_f32(gpu, prec):
     from oracle import oracle as orc
     A = wl.laplace2d(75, 91)
     b = wl.apply(A, wl.uniform(A.m, 11))
+    n0 = gpu.counter("cg_on_chip")
     code, it, x = _solve(A, b, "row", torch.float32, prec, tol=1e-4)
+    assert gpu.counter("cg_on_chip") == n0 + 1
     ref = orc.solve("cg", A, b.astype(np.float32), precond=PREC[prec], tol=1e-4, max_iter=4000, dtype=np.float32)
     assert code == ref.code == 0 and abs(it.nb_iter - ref.nb_iter) <= 2
     assert np.linalg.norm(wl.apply(A, x.astype(np.float64)) - b) <= 1e-3 * np.linalg.norm(b)
@@ -150,10 +154,12 @@ def test_resident_batch_matches_oracle(gpu, kind):
     Ag = K.Matrix(A, layout="rows")
     bg = torch.tensor(b, device="cuda")
     runs = []
+    n0 = gpu.counter("batch_on_chip")
     for _ in range(2):
         x = torch.full_like(bg, 7.0)
         its, codes = cg_batched(Ag, row_off, x, bg, tol=1e-8, max_iter=5000)
         runs.append((its, codes, x.cpu().numpy()))
+    assert gpu.counter("batch_on_chip") == n0 + 2
     for a, c in zip(*runs):
         assert np.array_equal(a, c)
     its, codes, x = runs[0]

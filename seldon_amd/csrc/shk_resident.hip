@@ -141,10 +141,11 @@ __global__ __launch_bounds__(kBlock) void k_res_out(int64_t n, const T *__restri
 
 // Rows per thread (a member per CU, kResThreads threads each).  Few rows per
 // thread keep the sweep over them short, few members the sums: measured on
-// 2-D Laplacians, us per iteration with 2 / 4 / 8 rows: 64^2 3.5 / 4.0 / 3.5,
-// 256^2 4.4 / 4.7 / 5.5, 512^2 7.4 / 6.1 / 6.4; so two rows up to 128 members
-// of them, then four, and eight only where four no longer reach (1000^2: 11.0
-// against 34.7 for launched kernels).  Seven-step rows spill at eight.
+// 2-D Laplacians, us per iteration with 2 / 4 / 8 rows: 64^2 3.8 / 4.2 / 3.3,
+// 256^2 4.0 / 4.2 / 5.0, 512^2 6.8 / 5.4 / 5.5, 64^3 with Jacobi 13.9 / 13.2;
+// so two rows up to 128 members of them, then four, and eight only where four
+// no longer reach (1000^2: 10.0 against 32.0 for launched kernels).  Seven-step
+// rows spill at eight.
 static int res_rows_per_thread(int m, int steps, int cus)
 {
     for (int r : {2, 4})

@@ -13,7 +13,8 @@ constexpr long long kResWaitSeconds = 2;
 // 4 us each) and the next one carries it on: contexts of other threads get
 // their turn on the GPU, however long a solve is.  Solves whose max_iter is
 // within that take kernels without the provision (LONG), which in the others
-// costs registers: 256^2 4.0 -> 4.2 us per iteration, with Jacobi 4.4 -> 5.0.
+// costs registers: 256^2 4.07 -> 4.15 us per iteration, with Jacobi 4.53 -> 5.19,
+// 1000^2 10.0 -> 10.1 and 14.3 -> 14.3.
 
 template <typename T>
 struct ResSolve {
@@ -35,7 +36,8 @@ __global__ __launch_bounds__(kResThreads, 2) void k_cg_resident(ResSolve<T> a)
     if (st->skip) return;
     const int tid = threadIdx.x;
     if (tid == 0) sh.bad = 0;
-    ResTeam t{a.k, (int)blockIdx.x, LlBuf(a.slot, 2 * a.k * res_slot_words<T>()), 0u, &st->res_stall, a.limit, res_every(a.limit)};
+    ResTeam t{a.k, (int)blockIdx.x, LlBuf(a.slot, 2 * a.k * res_slot_words<T>()), 0u, &st->res_stall, a.limit,
+              res_every(a.limit)};
     const LlBuf zw(a.zw, (int64_t)a.m * ll_words<T>());
     ResRows R;
     R.r0 = 0;
@@ -224,7 +226,7 @@ int cg_resident(shk_ctx ctx, shk_csr A, const T *diag, T *x, T *r, void *zw, voi
 }
 template int cg_resident<double>(shk_ctx, shk_csr, const double *, double *, double *, void *, void *,
                                  KState<double> *, double *, bool);
-template int cg_resident<float>(shk_ctx, shk_csr, const float *, float *, float *, void *, void *, KState<float> *, float *,
-                                bool);
+template int cg_resident<float>(shk_ctx, shk_csr, const float *, float *, float *, void *, void *, KState<float> *,
+                                float *, bool);
 
 }  // namespace shk

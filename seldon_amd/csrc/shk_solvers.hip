@@ -2505,12 +2505,15 @@ int cg_impl(shk_ctx ctx, shk_csr A, T *x, const T *b, int prec, shk_iteration *i
     S.ext_cap = ext_cap;
     const bool jac = prec == SHK_PREC_JACOBI;
     resident = resident && may_wait(ctx) && cg_resident_fits(A);
-    bool leave = resident && !ext && it->max_iter > ctx->opt[SHK_OPT_CG_ITERS];
+    bool leave = resident && it->max_iter > ctx->opt[SHK_OPT_CG_ITERS];
     int st0 = SHK_ERR_NOMEM;
     if (!leave || may_spare(ctx, 2 * sizeof(T) * (size_t)A->m))
         st0 = S.setup(ctx, A, (jac ? 4 : 3) + (leave ? 2 : 0), 0, it);
-    if (st0 == SHK_ERR_NOMEM && leave) {  // the launched kernels do with less
-        resident = leave = false;
+    if (leave && (st0 == SHK_ERR_NOMEM || (ext && st0 == SHK_ERR_ARG))) {
+        // the launched kernels do with less; a fixed work memory that has no
+        // room for it keeps the solve in one launch
+        leave = false;
+        resident = resident && ext;
         st0 = S.setup(ctx, A, jac ? 4 : 3, 0, it);
     }
     SHK_TRY(st0);

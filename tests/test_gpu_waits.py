@@ -188,6 +188,22 @@ def test_cg_left_and_carried_on(ctx, name, prec):
                 assert np.array_equal(a, c), (dtype, iters)
 
 
+@pytest.mark.parametrize("side", [128, 1000])
+def test_cg_noalloc_left_and_carried_on(ctx, side):
+    """In the fixed work memory too, and in one launch where that has no room
+    for what a solve is left with (1M FP64 rows): the same bits."""
+    from seldon_amd import _lib as L
+    from tests.test_zz_no_alloc import _run
+    A, b, _ = wl.cg_laplace(side)
+    n0 = ctx.counter("cg_on_chip")
+    ref = _run(L.load().shk_cg, A, b, torch.float64, False, None)
+    ctx.set_option("cg_iters", 50)
+    got = _run(L.load().shk_cg_noalloc, A, b, torch.float64, False, None)
+    assert ctx.counter("cg_on_chip") == n0 + 2
+    for a, c in zip(got, ref):
+        assert np.array_equal(a, c)
+
+
 def test_long_cg_gives_way(ctx):
     """A solve that fills the GPU for a long time is left now and then: a
     short one of another thread, which needs its place, ends long before it."""
